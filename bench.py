@@ -11,8 +11,8 @@ roofline: the closest-hit extension kernel (by default k_trace_dyn: persistent
   waves that take new rays from a global queue once 64 (first bounce) or 48
   (later bounces) of their lanes are idle), algorithmic bytes per launch =
   32 B per ray read from memory (first-bounce eye rays are computed in the
-  kernel and read nothing) + 16 B hit out per ray + 128 B (FP32 layout) or
-  64 B (quantized layout) per 4-wide node visited + 48 B per triangle tested,
+  kernel and read nothing) + 16 B hit out per ray + 128 B per node visited
+  (8-wide, or 4-wide in the FP32 layout) + 48 B per triangle tested,
   over its HIP-event duration on the renderer stream.  Beside it, from
   rocprofv3 counter passes: the HBM bytes actually moved (FETCH_SIZE +
   WRITE_SIZE, calibrated on a copy), the VALUs' busy share and lane use
@@ -463,7 +463,7 @@ def main():
     ap.add_argument("--lds-stack", type=int, default=806, help="traversal variant: LDS stack entries (8/16/24; "
                     "806/807/808/1606 = 8 or 16 entries with >= 6, 7 or 8 waves per SIMD)")
     ap.add_argument("--lds-stack-shadow", type=int, default=806, help="the same for shadow rays (0: as --lds-stack)")
-    ap.add_argument("--node-format", type=int, default=1, help="BVH nodes: 0 = 128-byte FP32, 1 = 64-byte quantized")
+    ap.add_argument("--node-format", type=int, default=1, help="BVH nodes: 0 = FP32 4-wide, 1 = FP16-box 8-wide (128 bytes both)")
     ap.add_argument("--refill", type=int, default=64,
                     help="traversal lanes refill from a ray queue once this many of a wave's are idle (0: off)")
     ap.add_argument("--refill-secondary", type=int, default=48,
@@ -567,7 +567,7 @@ def main():
     rays = st["extension_rays"] + st["shadow_rays"]
     mrays = rays / wall / 1e6
     launches = max(st["extend_launches"], 1)
-    node_bytes = 64 if args.node_format else 128
+    node_bytes = 128                                  # both layouts
     # first-bounce eye rays are computed inside the extension kernel (no 32 B
     # ray read) when the refilling grid runs the first bounce over the
     # quantized nodes, as the renderer's schedule does above Refill Min Paths
@@ -622,7 +622,7 @@ def main():
                      "eye_rays_computed_in_kernel": bool(eye_in_kernel),
                      "stack_spills_per_ray": round(st["extend_spills"] / max(ext_rays, 1), 5),
                      "shadow_stack_spills_per_ray": round(st["shadow_spills"] / max(st["shadow_rays"], 1), 5),
-                     "box_tests_per_s": round(4 * st["extend_nodes"] / ext_s, 1) if ext_s > 0 else None,
+                     "box_tests_per_s": round((8 if args.node_format else 4) * st["extend_nodes"] / ext_s, 1) if ext_s > 0 else None,
                      "tri_tests_per_s": round(st["extend_tris"] / ext_s, 1) if ext_s > 0 else None,
                      "hbm_measured": None, "valu": None, "limiter": None},
         "time_to_equal_mse": None,

@@ -1,4 +1,4 @@
-// Binned-SAH BVH with NPBVHHelper semantics and its 4-wide re-layout.
+// Binned-SAH BVH with NPBVHHelper semantics and its 4-wide and 8-wide re-layouts.
 //
 // build_bvh_sah reproduces src/bvhhelper.cpp:55-311 bit for bit (same float
 // expressions, same bin boundaries, same strict-'<' cost minimum, same Hoare
@@ -447,73 +447,191 @@ void collapse_bvh4(const float* /*pos3*/, const u32* /*idx3*/, BvhHost& b, u32 l
 }
 
 
-// ---- 64-byte quantized nodes -------------------------------------------------
+// ---- 8-wide quantized nodes --------------------------------------------------
 
 namespace {
 
-inline float q_decode(float o, u32 q, float step) { return o + (float)q * step; }
+// FP16 bits of x in [0, 1] rounded down (up = false) or up.
+uint16_t h_round(double x, bool up) {
+  if (!(x > 0.0)) return 0;
+  if (x >= 1.0) return 0x3C00;
+  int e;
+  (void)std::frexp(x, &e);                     // x in [2^(e-1), 2^e)
+  const int q = std::max(e - 1, -14) - 10;     // exponent of the last place
+  const double m = std::ldexp(x, -q);
+  const uint32_t k = (uint32_t)(up ? std::ceil(m) : std::floor(m));
+  // k counts units of 2^q; subnormals and normals are one bit sequence, and a
+  // carry into the next binade is the next bit pattern
+  return (uint16_t)(((uint32_t)(q + 24) << 10) + k);
+}
+double h_value(uint16_t b) {
+  const int e = b >> 10, m = b & 0x3FF;
+  return e ? std::ldexp((double)(m + 1024), e - 25) : std::ldexp((double)m, -24);
+}
 
-// Smallest exponent e (step 2^(e-127)) with o + 255 * step >= hi.
-u32 q_exponent(float o, float hi) {
-  for (u32 e = 1; e < 255; e++) {
-    float step = ldexpf(1.f, (int)e - 127);
-    if (q_decode(o, 255u, step) >= hi) return e;
+constexpr int kW8 = 8;
+// Cost weights of the 8-wide collapse: one node visit (eight box tests, the
+// hit mask, its ordering, push and pop) against one triangle test.
+constexpr double kNode8Cost = 2.5, kTri8Cost = 1.0;
+
+// The boxes of up to eight children (box[s] null: unused slot) as fractions of
+// the node's extents.
+bool quantize_slots(Node8& q, const BinNode* const box[kW8], float& qmag) {
+  u32 exps = 0;
+  for (int a = 0; a < 3; a++) {
+    float o = INFINITY, top = -INFINITY;
+    for (int c = 0; c < kW8; c++) {
+      if (!box[c]) continue;
+      o = std::min(o, box[c]->mn[a]);
+      top = std::max(top, box[c]->mx[a]);
+    }
+    if (!(o <= top)) { o = 0.f; top = 0.f; }          // no child
+    // the smallest extent 2^(e-127) reaching top
+    int k = -126;
+    if ((double)top > (double)o) (void)std::frexp((double)top - (double)o, &k);
+    u32 e = (u32)std::min(254, std::max(1, k + 126));
+    while (e < 254 && (double)o + std::ldexp(1.0, (int)e - 127) < (double)top) e++;
+    const double ext = std::ldexp(1.0, (int)e - 127);
+    if (!((double)o + ext >= (double)top)) return false;
+    q.o[a] = o;
+    qmag = std::max(qmag, (float)std::max(std::fabs((double)o), std::fabs((double)o + ext) * 1.000001));
+    exps |= e << (8 * a);
+    for (int c = 0; c < kW8; c++) {
+      if (!box[c]) { q.h[a][0][c] = 0x3C00; q.h[a][1][c] = 0; continue; }
+      const double lo = box[c]->mn[a], hi = box[c]->mx[a];
+      const uint16_t hl = h_round((lo - o) / ext, false), hh = h_round((hi - o) / ext, true);
+      if ((double)o + h_value(hl) * ext > lo || (double)o + h_value(hh) * ext < hi) return false;
+      q.h[a][0][c] = hl;
+      q.h[a][1][c] = hh;
+    }
   }
-  return 0;
+  q.exps = exps;
+  return true;
 }
 
 }  // namespace
 
-bool quantize_bvh4(BvhHost& b) {
-  const std::vector<Node4>& in = b.nodes4;
-  std::vector<Node4Q>& out = b.nodes4q;
-  out.assign(in.size(), Node4Q());
-  float qmag = 1e-30f;
-  for (size_t i = 0; i < in.size(); i++) {
-    const Node4& n = in[i];
-    Node4Q& q = out[i];
-    std::memset(&q, 0, sizeof q);
-    const float* lo[3] = {n.lox, n.loy, n.loz};
-    const float* hi[3] = {n.hix, n.hiy, n.hiz};
-    uint8_t* qlo[3] = {q.lox, q.loy, q.loz};
-    uint8_t* qhi[3] = {q.hix, q.hiy, q.hiz};
-    u32 exps = 0;
-    for (int a = 0; a < 3; a++) {
-      float o = INFINITY, top = -INFINITY;
-      for (int c = 0; c < 4; c++) {
-        if (n.child[c] == kInvalid) continue;
-        o = std::min(o, lo[a][c]);
-        top = std::max(top, hi[a][c]);
-      }
-      if (!(o <= top)) { o = 0.f; top = 0.f; }          // no valid child
-      u32 e = q_exponent(o, top);
-      if (e == 0) return false;
-      const float step = ldexpf(1.f, (int)e - 127);
-      q.o[a] = o;
-      qmag = std::max(qmag, std::max(std::fabs(o), std::fabs(q_decode(o, 255u, step))));
-      exps |= e << (8 * a);
-      for (int c = 0; c < 4; c++) {
-        if (n.child[c] == kInvalid) { qlo[a][c] = 255; qhi[a][c] = 0; continue; }
-        double fl = std::floor(((double)lo[a][c] - (double)o) / (double)step);
-        u32 ql = (u32)std::max(0.0, std::min(255.0, fl));
-        while (ql > 0 && q_decode(o, ql, step) > lo[a][c]) ql--;
-        double fh = std::ceil(((double)hi[a][c] - (double)o) / (double)step);
-        u32 qh = (u32)std::max(0.0, std::min(255.0, fh));
-        while (qh < 255 && q_decode(o, qh, step) < hi[a][c]) qh++;
-        if (q_decode(o, ql, step) > lo[a][c] || q_decode(o, qh, step) < hi[a][c]) return false;
-        qlo[a][c] = (uint8_t)ql;
-        qhi[a][c] = (uint8_t)qh;
+// The dynamic program of collapse_bvh4 at eight entries: F[x][i] is the least
+// cost of hanging binary subtree x below an 8-wide node as at most i entries,
+// split[x][i] the entries its left child gets (kWhole: x is one entry).  Slots: a ray visits a node's children in the order
+// of slot ^ (its direction's octant, one bit per negative component), so slot s
+// takes a child that lies towards (s & 1 ? + : -, s & 2 ? + : -, s & 4 ? + : -)
+// of the node's centre; the pairs are picked greedily by that distance.
+bool collapse_bvh8(BvhHost& b, u32 leaf_max) {
+  const std::vector<BinNode>& bn = b.dnodes;
+  const u32 N = (u32)bn.size();
+  const u32 bound = std::min(leaf_max, kLeaf8);
+  b.nodes8.clear();
+  b.order8.clear();
+  b.depth8 = 0;
+  b.qmag = 1e-30f;
+  if (N == 0) return true;
+  constexpr uint8_t kWhole = 255;
+  std::vector<u32> cnt(N, 0), first(N, 0);
+  std::vector<std::array<double, kW8 + 1>> F(N);
+  std::vector<std::array<uint8_t, kW8 + 1>> split(N);
+  std::vector<uint8_t> as_leaf(N, 0);
+  const double inf = std::numeric_limits<double>::infinity();
+  for (u32 x = N; x-- > 0;) {
+    const BinNode& n = bn[x];
+    const bool leaf = n.n > 0;
+    const u32 l = x + 1, r = x + n.a;
+    if (leaf) { cnt[x] = n.n; first[x] = n.a; }
+    else { cnt[x] = cnt[l] + cnt[r]; first[x] = first[l]; }
+    const double dx = (double)n.mx[0] - n.mn[0], dy = (double)n.mx[1] - n.mn[1], dz = (double)n.mx[2] - n.mn[2];
+    const double A = std::max(0.0, dx * dy + dx * dz + dy * dz);
+    const double leafC = cnt[x] <= bound ? A * kTri8Cost * cnt[x] : inf;
+    std::array<double, kW8 + 1> G;
+    G.fill(inf);
+    split[x].fill(1);
+    if (!leaf)
+      for (int i = 2; i <= kW8; i++)
+        for (int k = 1; k < i; k++) {
+          const double c = F[l][k] + F[r][i - k];
+          if (c < G[i]) { G[i] = c; split[x][i] = (uint8_t)k; }
+        }
+    const double nodeC = leaf ? inf : A * kNode8Cost + G[kW8];
+    as_leaf[x] = cnt[x] <= bound && leafC <= nodeC;
+    const double one = std::min(leafC, nodeC);
+    F[x][0] = inf;
+    F[x][1] = one;
+    for (int i = 2; i <= kW8; i++) F[x][i] = std::min(one, G[i]);
+    // split[x][8] serves the node of its own; as entries of its parent, x stays
+    // whole where splitting it is no cheaper
+    split[x][1] = kWhole;
+    for (int i = 2; i < kW8; i++)
+      if (one <= G[i]) split[x][i] = kWhole;
+  }
+  std::vector<u32> ent;
+  // at most i entries for x below its parent (spread: x is the node itself)
+  auto take = [&](auto&& self, u32 x, int i, bool spread) -> void {
+    const int k = split[x][i];
+    if (!spread && (k == kWhole || bn[x].n > 0)) { ent.push_back(x); return; }
+    self(self, x + 1, k, false);
+    self(self, x + bn[x].a, i - k, false);
+  };
+  struct Item { u32 bin, slot, depth; };
+  std::queue<Item> q;
+  b.nodes8.push_back(Node8());
+  q.push({0, 0, 1});
+  b.order8.reserve(cnt[0]);
+  while (!q.empty()) {
+    const Item it = q.front();
+    q.pop();
+    b.depth8 = std::max(b.depth8, it.depth);
+    ent.clear();
+    if (it.bin == 0 && as_leaf[0]) ent.push_back(0);       // the whole scene in one leaf
+    else take(take, it.bin, kW8, true);
+    // slots
+    const BinNode& me = bn[it.bin];
+    u32 in[kW8];
+    const BinNode* box[kW8] = {};
+    const int n = (int)ent.size();
+    float pref[kW8][kW8];
+    for (int c = 0; c < n; c++) {
+      float m[3];
+      for (int a = 0; a < 3; a++)
+        m[a] = 0.5f * ((bn[ent[c]].mn[a] + bn[ent[c]].mx[a]) - (me.mn[a] + me.mx[a]));
+      for (int s = 0; s < kW8; s++)
+        pref[c][s] = (s & 1 ? m[0] : -m[0]) + (s & 2 ? m[1] : -m[1]) + (s & 4 ? m[2] : -m[2]);
+    }
+    bool placed[kW8] = {};
+    for (int k = 0; k < n; k++) {
+      int bc = -1, bs = -1;
+      for (int c = 0; c < n; c++)
+        for (int s = 0; s < kW8 && !placed[c]; s++)
+          if (!box[s] && (bc < 0 || pref[c][s] > pref[bc][bs])) { bc = c; bs = s; }
+      placed[bc] = true;
+      box[bs] = &bn[ent[bc]];
+      in[bs] = ent[bc];
+    }
+    Node8 nd;
+    std::memset(&nd, 0, sizeof nd);
+    if (!quantize_slots(nd, box, b.qmag)) return false;
+    nd.child = (u32)b.nodes8.size();
+    nd.tri = (u32)b.order8.size();
+    for (int s = 0; s < kW8; s++) {
+      if (!box[s]) continue;
+      const u32 x = in[s];
+      if (as_leaf[x]) {
+        for (u32 j = 0; j < cnt[x]; j++) {
+          nd.valid |= 1u << (4 * s + j);
+          b.order8.push_back(first[x] + j);
+        }
+      } else {
+        nd.exps |= 1u << (24 + s);
+        q.push({x, (u32)b.nodes8.size(), it.depth + 1});
+        b.nodes8.push_back(Node8());
       }
     }
-    q.exps = exps;
-    for (int c = 0; c < 4; c++) {
-      if (n.count[c] > 0xFFFFu) return false;
-      q.count[c] = (uint16_t)n.count[c];
-      q.child[c] = n.child[c];
+    b.nodes8[it.slot] = nd;
+    if (b.nodes8.size() > kMaxNodes8) {                    // traversed in the FP32 layout instead
+      b.nodes8.clear();
+      b.order8.clear();
+      return true;
     }
   }
-  b.qmag = qmag;
-  return true;
+  return b.depth8 <= kMaxDepth8;
 }
 
 }  // namespace cpt

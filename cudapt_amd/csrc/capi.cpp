@@ -79,14 +79,14 @@ struct cpt_scene {
   BvhHost bvh;
   bool has_bvh = false;
   bool uploaded = false;
-  // leaves of the 4-wide BVH hold at most leaf_max triangles: more leaf levels
-  // cost fewer triangle tests than they add node visits (2: 16 % more rays/s
-  // than 4 on the 262k-triangle sphere grid, 1 is level with 2)
+  // leaves hold at most leaf_max triangles (8-wide: at most kLeaf8 of them): on
+  // the 262k-triangle sphere grid the 64-frame still takes 21.0 / 19.7 / 19.7 /
+  // 19.7 ms at 1 / 2 / 3 / 4
   u32 mesh_version = 0, mat_version = 0, leaf_max = 2;
   hipStream_t stream = nullptr;
   DevArray<Node4> d_nodes4;
-  DevArray<Node4Q> d_nodes4q;
-  DevArray<float4> d_tris, d_tris_bin, d_vpos, d_vnrm, d_bnodes, d_tex, d_surf, d_env;
+  DevArray<Node8> d_nodes8;
+  DevArray<float4> d_tris, d_tris8, d_tris_bin, d_vpos, d_vnrm, d_bnodes, d_tex, d_surf, d_env;
   DevArray<uint4> d_tex_desc;
   DevArray<uint4> d_tri_verts;
   DevArray<uint2> d_boff;
@@ -98,7 +98,8 @@ struct cpt_scene {
   DevScene dev() const {
     DevScene s;
     s.nodes4 = d_nodes4.p;
-    s.nodes4q = d_nodes4q.p;
+    s.nodes8 = bvh.nodes8.empty() ? nullptr : d_nodes8.p;
+    s.tris8 = d_tris8.p;
     s.tris = d_tris.p;
     s.tri_verts = d_tri_verts.p;
     s.vpos = d_vpos.p;
@@ -360,7 +361,8 @@ int cpt_bvh_build_sah(cpt_scene* s, uint32_t max_depth) {
       !build_bvh_device(s->pos.data(), s->idx.data(), s->nt, s->bvh))
     return fail(CPT_E_STATE, "cpt_bvh_build_sah: build failed");
   collapse_bvh4(s->pos.data(), s->idx.data(), s->bvh, s->leaf_max);
-  if (!quantize_bvh4(s->bvh)) return fail(CPT_E_STATE, "cpt_bvh_build_sah: a node cannot be quantized to 64 bytes");
+  if (!collapse_bvh8(s->bvh, s->leaf_max))
+    return fail(CPT_E_STATE, "cpt_bvh_build_sah: a node cannot be quantized, or the 8-wide tree is deeper than %u", kMaxDepth8);
   if (s->bvh.depth4 > 31) return fail(CPT_E_LIMIT, "cpt_bvh_build_sah: 4-wide depth %u exceeds 31", s->bvh.depth4);
   s->has_bvh = true;
   s->uploaded = false;
@@ -388,7 +390,8 @@ int cpt_bvh4_set_leaf_size(cpt_scene* s, uint32_t max_tris) {
   s->leaf_max = max_tris;
   if (!s->has_bvh) return CPT_OK;
   collapse_bvh4(s->pos.data(), s->idx.data(), s->bvh, s->leaf_max);
-  if (!quantize_bvh4(s->bvh)) return fail(CPT_E_STATE, "cpt_bvh4_set_leaf_size: a node cannot be quantized to 64 bytes");
+  if (!collapse_bvh8(s->bvh, s->leaf_max))
+    return fail(CPT_E_STATE, "cpt_bvh4_set_leaf_size: a node cannot be quantized, or the 8-wide tree is deeper than %u", kMaxDepth8);
   if (s->bvh.depth4 > 31) return fail(CPT_E_LIMIT, "cpt_bvh4_set_leaf_size: 4-wide depth %u exceeds 31", s->bvh.depth4);
   s->uploaded = false;
   s->mesh_version++;
@@ -431,6 +434,14 @@ int cpt_scene_upload(cpt_scene* s) {
     return out;
   };
   std::vector<float4> tris = tri_data(s->bvh.dreorder), tris_bin = tri_data(s->bvh.reorder);
+  // the 8-wide tree's triangles: the same records in its own order, each with
+  // its index in the device leaf order
+  std::vector<float4> tris8(s->bvh.order8.size() * 3);
+  for (u32 i = 0; i < (u32)s->bvh.order8.size(); i++) {
+    const u32 leaf = s->bvh.order8[i];
+    for (int k = 0; k < 3; k++) tris8[(size_t)i * 3 + k] = tris[(size_t)leaf * 3 + k];
+    std::memcpy(&tris8[(size_t)i * 3 + 1].w, &leaf, 4);
+  }
   std::vector<uint4> tv(nt);
   for (u32 i = 0; i < nt; i++) {
     u32 o = s->bvh.dreorder[i];
@@ -450,7 +461,8 @@ int cpt_scene_upload(cpt_scene* s) {
     boff[i] = make_uint2(bn[i].a, bn[i].n);
   }
   HIP_TRY(s->d_nodes4.upload(s->bvh.nodes4.data(), s->bvh.nodes4.size(), s->stream));
-  HIP_TRY(s->d_nodes4q.upload(s->bvh.nodes4q.data(), s->bvh.nodes4q.size(), s->stream));
+  HIP_TRY(s->d_nodes8.upload(s->bvh.nodes8.data(), s->bvh.nodes8.size(), s->stream));
+  HIP_TRY(s->d_tris8.upload(tris8.data(), tris8.size(), s->stream));
   HIP_TRY(s->d_tris.upload(tris.data(), tris.size(), s->stream));
   HIP_TRY(s->d_tris_bin.upload(tris_bin.data(), tris_bin.size(), s->stream));
   HIP_TRY(s->d_tri_verts.upload(tv.data(), tv.size(), s->stream));
@@ -674,8 +686,8 @@ const char* const kInFlight = "Frames In Flight";
 // allocates from one error map and traces as one wavefront (1 = the
 // reference's one frame per allocation)
 const char* const kPassFrames = "Adaptive Pass Frames";
-// BVH node format of the traversal kernels: 0 = 128-byte FP32 4-wide nodes,
-// 1 = the same nodes quantized to 64 bytes
+// BVH node format of the traversal kernels: 0 = FP32 4-wide nodes, 1 = 8-wide
+// nodes with FP16 boxes (both 128 bytes)
 const char* const kNodeFormat = "Node Format";
 // traversal scheduling: 0 = one ray per thread; 1..64 = a persistent grid
 // whose lanes take the next ray from a global queue when theirs is finished,
@@ -916,6 +928,9 @@ LightJobs light_jobs(cpt_renderer* r, u32 f0, u32 nf) {
   return j;
 }
 
+// "Node Format" 1: the 8-wide quantized nodes (a scene too large for them has none).
+bool use_nodes8(const cpt_renderer* r, const DevScene& sc) { return r->attr(kNodeFormat) != 0 && sc.nodes8; }
+
 hipError_t timed_begin(cpt_renderer* r, int kind, hipEvent_t* a, hipStream_t st = nullptr) {
   if (!r->profiling) return hipSuccess;
   hipError_t e = r->take(a);
@@ -988,7 +1003,7 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
   }
   hipStream_t sst = ov ? r->side : r->stream;
   const bool eye0 =
-      gen_eye && big && r->attr(kRefill) >= 1.0 && r->attr(kNodeFormat) != 0 && fa.n_views == 0;
+      gen_eye && big && r->attr(kRefill) >= 1.0 && use_nodes8(r, sc) && fa.n_views == 0;
   if (gen_eye && !eye0) HIP_TRY(launch_gen_eye(fa, r->A.view(), r->stream));
   bool shadow_pending = false;
   // "Tail Bounce" t > 0: bounces t.. run as one k_tail launch (plain BDPT's
@@ -1014,13 +1029,13 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
           (uint32_t)(r->cus > 0 ? r->cus : 256) * (uint32_t)std::min(32.0, std::max(1.0, r->attr(kRefillGroups)));
       HIP_TRY(timed_begin(r, 10, &ev));
       HIP_TRY(launch_tail(sc, fa, cur->view(), r->fc.p, b, grid, r->lv.p, ac, (int)r->attr(kLdsStack),
-                          r->attr(kNodeFormat) != 0, r->stats.p, r->stream));
+                          use_nodes8(r, sc), r->stats.p, r->stream));
       HIP_TRY(timed_end(r, 10, ev));
       break;
     }
     r->extend_launches++;
     HIP_TRY(timed_begin(r, 0, &ev));
-    const int quant = r->attr(kNodeFormat) != 0;
+    const int quant = use_nodes8(r, sc);
     const uint32_t refill =
         big ? (uint32_t)std::min(64.0, std::max(0.0, r->attr(b == 0 ? kRefill : kRefillSecondary))) : 0u;
     const uint32_t dyn_grid =
@@ -1219,7 +1234,7 @@ int render_adaptive_frame(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa, co
   LightJobs jobs = light_jobs(r, fa.frame0, 1);
   if (jobs.n) {
     HIP_TRY(timed_begin(r, 3, &ev));
-    HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, r->stream));
+    HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, use_nodes8(r, sc), r->stream));
     HIP_TRY(timed_end(r, 3, ev));
   }
   Accum ac;
@@ -1331,13 +1346,13 @@ int render_bdpt_regen(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa0) {
     fa.frame0 = fa0.frame0 + k;
     if (fa.frame0 % 3 == 0) {
       HIP_TRY(timed_begin(r, 3, &ev));
-      HIP_TRY(launch_regen_light(sc, fa, r->lv.p, r->stream));
+      HIP_TRY(launch_regen_light(sc, fa, r->lv.p, use_nodes8(r, sc), r->stream));
       HIP_TRY(timed_end(r, 3, ev));
     }
     r->extend_launches++;
     HIP_TRY(timed_begin(r, 0, &ev));
     HIP_TRY(launch_regen_eye(sc, fa, r->lv.p, r->result.p, r->sample_n.p, (int)r->attr(kLdsStack),
-                             r->attr(kNodeFormat) != 0, r->stats.p, r->stream));
+                             use_nodes8(r, sc), r->stats.p, r->stream));
     HIP_TRY(timed_end(r, 0, ev));
   }
   return CPT_OK;
@@ -1369,7 +1384,7 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
       ls = r->side;
     }
     HIP_TRY(timed_begin(r, 3, &ev, ls));
-    HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, ls));
+    HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, use_nodes8(r, sc), ls));
     HIP_TRY(timed_end(r, 3, ev, ls));
     if (ls != r->stream) {
       HIP_TRY(hipEventRecord(r->ev_light, ls));
@@ -2088,7 +2103,7 @@ int batch_enqueue(cpt_batch* b, cpt_scene* s, u32 k) {
   std::memset(&jobs, 0, sizeof jobs);
   jobs.dev_groups = (k + 2) / 3 + 1;                 // groups k frames can span
   const u32 n = b->total * k;
-  HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, r->stream));
+  HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, use_nodes8(r, sc), r->stream));
   HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
   Accum ac;
   std::memset(&ac, 0, sizeof ac);

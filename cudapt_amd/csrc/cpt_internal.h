@@ -35,22 +35,26 @@ struct alignas(128) Node4 {
 };
 static_assert(sizeof(Node4) == 128, "Node4 must be one 128-byte line");
 
-// The same node in 64 bytes: child boxes quantized to 8 bits on a per-node
-// grid (origin o, power-of-two step 2^(e-127) per axis), decoded as
-// o + q * step in FP32.  The host picks every q so that the decoded box
-// contains the child's FP32 box (lo rounded down, hi up, checked with the
-// decode arithmetic), so culling stays conservative and hits unchanged.
-// Loaded as four 16-byte vectors: {o, exponents}, {lo/hi x, lo/hi y},
-// {lo/hi z, counts}, {children}.  Counts above 65535 cannot be stored (the
-// build reports it).
-struct alignas(64) Node4Q {
+// 8-wide node, 128 bytes = one line: child boxes as FP16 fractions h in [0, 1]
+// of a power-of-two extent 2^(e-127) per axis from the origin o.  The host picks
+// every h so that the box o + h * 2^(e-127) (in exact arithmetic) contains the
+// child's FP32 box, so culling stays conservative and hits unchanged; a
+// traversal multiplies them as they are (v_fma_mix_f32 takes FP16 operands).
+// Children sit in eight slots; interior children (imask) are consecutive nodes
+// from `child` on in slot order, and a leaf child's triangles (at most kLeaf8)
+// are consecutive from `tri` on, slot by slot: bit 4 s + j of `valid` is set for
+// triangle j of slot s.  Loaded as eight 16-byte vectors: {o, exponents +
+// imask}, {child, tri, valid, -}, then lo and hi of each axis.
+struct alignas(128) Node8 {
   float o[3];
-  u32 exps;            // ex | ey << 8 | ez << 16
-  uint8_t lox[4], hix[4], loy[4], hiy[4], loz[4], hiz[4];
-  uint16_t count[4];
-  u32 child[4];
+  u32 exps;            // ex | ey << 8 | ez << 16 | imask << 24
+  u32 child, tri, valid, pad;
+  uint16_t h[3][2][8]; // [axis][lo, hi][slot]; an unused slot has no imask or valid bit
 };
-static_assert(sizeof(Node4Q) == 64, "Node4Q must be 64 bytes");
+static_assert(sizeof(Node8) == 128, "Node8 must be one 128-byte line");
+constexpr u32 kLeaf8 = 4;          // most triangles of an 8-wide leaf child
+constexpr u32 kMaxNodes8 = 1u << 25;   // byte offsets of nodes fit 32 bits; a larger tree is not made
+constexpr u32 kMaxDepth8 = 64;     // levels of the 8-wide tree (a traversal keeps at most one stack entry a level)
 
 // Host result of the SAH build.
 struct BvhHost {
@@ -59,8 +63,10 @@ struct BvhHost {
   std::vector<BinNode> dnodes;     // the device tree's binary SAH build, same format
   std::vector<u32> dreorder;       // device leaf order -> original triangle id
   std::vector<Node4> nodes4;       // 4-wide re-layout (BFS order, root 0)
-  std::vector<Node4Q> nodes4q;     // the same nodes quantized to 64 bytes
-  float qmag = 1e-30f;             // max |o + q * step| over nodes4q's planes, at least 1e-30
+  std::vector<Node8> nodes8;       // 8-wide quantized re-layout (BFS order, root 0)
+  std::vector<u32> order8;         // its triangle order -> device leaf order
+  float qmag = 1e-30f;             // max |o + q * step| over nodes8's planes, at least 1e-30
+  u32 depth8 = 0;
   u32 depth4 = 0, leaves4 = 0;
 };
 
@@ -71,7 +77,10 @@ bool build_bvh_device(const float* pos3, const u32* idx3, u32 nt, BvhHost& out);
 // Collapse the device binary tree into 4-wide nodes (SAH-optimal); a leaf
 // range holds at most leaf_max triangles.
 void collapse_bvh4(const float* pos3, const u32* idx3, BvhHost& b, u32 leaf_max);
-// Quantize nodes4 into nodes4q; false when a node cannot be encoded.
-bool quantize_bvh4(BvhHost& b);
+// Collapse the device binary tree into 8-wide quantized nodes (SAH-optimal);
+// a leaf child holds at most min(leaf_max, kLeaf8) triangles.  No nodes when
+// they would exceed kMaxNodes8; false when a node cannot be encoded or the tree
+// is deeper than kMaxDepth8.
+bool collapse_bvh8(BvhHost& b, u32 leaf_max);
 
 }  // namespace cpt

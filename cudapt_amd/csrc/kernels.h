@@ -19,7 +19,8 @@ struct DevMaterial {
 // Device-resident scene.  Triangles are in BVH leaf order.
 struct DevScene {
   const Node4* nodes4;         // 128-byte 4-wide nodes
-  const Node4Q* nodes4q;       // the same nodes, 64-byte quantized
+  const Node8* nodes8;         // 8-wide quantized nodes; null: the scene is too large for them
+  const float4* tris8;         // their triangles, 3 per triangle as tris, e0.w = device leaf index bits
   const float4* tris;          // 3 per triangle: p0 (w = original id bits), e0 = p1-p0, e1 = p2-p0
   const uint4* tri_verts;      // v0, v1, v2, material
   const float4* vpos;          // vertex positions, w = texture u
@@ -44,7 +45,7 @@ struct DevScene {
   // env_w = 0: none
   const float4* env;
   uint32_t env_w, env_h;
-  float qmag;                  // bound on |o + q s| over every slab plane of nodes4q (>= 1e-30)
+  float qmag;                  // bound on |o + q s| over every slab plane of nodes8 (>= 1e-30)
 };
 
 // Per-path SoA state of the wavefront (one slot per live eye path).
@@ -146,7 +147,7 @@ hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, cons
                         float4* hits_out, int out_orig, int any_hit, uint32_t layout, DevStats* stats, hipStream_t st, int cost = 0);
 hipError_t launch_frame_begin(FrameCounters* fc, uint32_t n_paths, hipStream_t st);
 hipError_t launch_light_pass(const DevScene& sc, const FrameArgs& fa, const LightJobs& jobs, LightVert* lv,
-                             FrameCounters* fc, hipStream_t st);
+                             FrameCounters* fc, int quant, hipStream_t st);
 // nframes x W*H eye paths, slot = frame offset * W*H + pixel.
 // The BVH debug renderer's TraceDepth (spec = 0xFFFFFFFF) or
 // TraceDepthParent(spec) per ray over the reference tree: out = 3 u32 per ray.
@@ -157,7 +158,7 @@ hipError_t launch_gen_eye(const FrameArgs& fa, PathBuf pb, hipStream_t st);
 hipError_t launch_apply_frames(const FrameArgs& fa, const float4* rec_acc, float* result, uint32_t* sample_n,
                                int pt, hipStream_t st);
 // lds_stack: traversal variant, the stack entries kept in LDS (the rest in
-// private memory) and the minimum resident waves per SIMD the register
+// private memory; 8-wide nodes keep 6, 10 or 14 group entries for 8, 16 or 24) and the minimum resident waves per SIMD the register
 // allocator is held to: 8, 16, 24 (no minimum), 806, 807, 808 (8 entries, >= 6,
 // 7 or 8 waves), 1606 (16 entries, >= 6 waves).  Other values: invalid argument.
 inline bool traversal_variant_ok(int v) {
@@ -203,7 +204,7 @@ hipError_t launch_shade(const DevScene& sc, const FrameArgs& fa, PathBuf cur, Pa
 // pixel (eye_depth <= 8 levels) into the running mean.  lv holds
 // kRegenLightVerts vertices.
 constexpr uint32_t kRegenLightVerts = 640;
-hipError_t launch_regen_light(const DevScene& sc, const FrameArgs& fa, LightVert* lv, hipStream_t st);
+hipError_t launch_regen_light(const DevScene& sc, const FrameArgs& fa, LightVert* lv, int quant, hipStream_t st);
 hipError_t launch_regen_eye(const DevScene& sc, const FrameArgs& fa, const LightVert* lv, float* result,
                             uint32_t* sample_n, int lds_stack, int quant, DevStats* stats, hipStream_t st);
 // The bounces from bounce0 on, one thread per live slot of cur, as k_mega

@@ -1,9 +1,11 @@
 // gfx950 kernels of the streaming-BDPT hot path.
 //
-//  traverse4      closest/any hit over 128-byte 4-wide nodes, ordered
-//                 near-first, stack top 16 entries in LDS (column layout, no
-//                 bank conflicts), deeper entries in private memory.
-//                 Replaces TracePrimitive (src/cudaRTCommon.cu:66-127).
+//  trace8         closest/any hit of a wave's rays over 8-wide nodes with FP16
+//                 boxes: a node a lane per step, then the wave's leaf triangles
+//                 as one list, one (ray, triangle) pair per lane.  Replaces
+//                 TracePrimitive (src/cudaRTCommon.cu:66-127).
+//  traverse4      the same over 128-byte FP32 4-wide nodes, one ray a thread,
+//                 ordered near-first, stack top in LDS, deeper entries private.
 //  traverse_bin   the same query over the reference's binary CompactBVH
 //                 layout (src/cudaRTCommon.cu:527-541), kept as the baseline.
 //  k_light_pass   light-vertex cache: pt_genLightPathQueue_kernel +
@@ -25,6 +27,8 @@
 // (Ize 2013 slab widening + a slack covering IntersectTri's eps origin shift),
 // so the answer does not depend on the node layout or visiting order.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "devmath.h"
 #include "kernels.h"
@@ -105,8 +109,7 @@ __device__ __forceinline__ void cswap(uint64_t& a, uint64_t& b) {
   a = lo; b = hi;
 }
 
-// Child boxes and links of a 4-wide node in the 128-byte FP32 layout (the
-// 64-byte quantized layout is tested straight from its words, box4_q).
+// Child boxes and links of a 4-wide node (128 bytes, FP32).
 struct NodeView {
   float lx[4], hx[4], ly[4], hy[4], lz[4], hz[4];
   uint32_t ch[4], cn[4];
@@ -153,98 +156,38 @@ __device__ __forceinline__ LdsU64* lds_column(uint64_t* shared_base) {
 // The state of one ray's traversal, advanced one node at a time by ray_step, so
 // that a lane whose ray has finished can start another while the rest of its
 // wave is still traversing (k_trace_dyn) or simply loop (traverse4).
-// pn, pf: -o * idir moved out by the quantized box test's slack, per axis.
 struct RayState {
-  f3 o, d, idir, o2, pn, pf;
+  f3 o, d, idir, o2;
   float eps;
   TraceHit h;
   uint32_t node;
   int sp;
 };
-// qmag bounds the magnitude of every quantized slab plane of the scene.
-__device__ __forceinline__ void ray_begin(RayState& R, f3 o, f3 d, float maxd, float eps, float qmag) {
+__device__ __forceinline__ void ray_begin(RayState& R, f3 o, f3 d, float maxd, float eps) {
   R.o = o;
   R.d = d;
   R.idir = mk3(1.f / escape_zero(d.x), 1.f / escape_zero(d.y), 1.f / escape_zero(d.z));
-  // Slack of the quantized box test (box4_q): 2^-20 = 16 u per unit of
-  // |idir| (qmag + |o|), twice the rounding bound of that test's distances.
-  const float k = 0x1p-20f;
-  const float sx = (fabsf(R.idir.x) * (qmag + fabsf(o.x))) * k;
-  const float sy = (fabsf(R.idir.y) * (qmag + fabsf(o.y))) * k;
-  const float sz = (fabsf(R.idir.z) * (qmag + fabsf(o.z))) * k;
-  const f3 oi = mk3(-(o.x * R.idir.x), -(o.y * R.idir.y), -(o.z * R.idir.z));
-  R.pn = mk3(oi.x - sx, oi.y - sy, oi.z - sz);
-  R.pf = mk3(oi.x + sx, oi.y + sy, oi.z + sz);
   R.o2 = o + d * eps;
   R.eps = eps;
   R.h.t = maxd; R.h.u = R.h.v = 0.f; R.h.leaf = kInvalid; R.h.orig = kInvalid;
   R.node = 0;
   R.sp = 0;
 }
-// The four child boxes of a 64-byte quantized node against the ray: entry and
-// exit distances tn, tf (entry clamped at 0), children and leaf counts.  A
-// slab plane is o_a + q s_a with s_a a power of two, so its distance
-// (o_a + q s_a - ray.o_a) idir_a is fma(q, s_a idir_a, c_a) with
-// c_a = fma(o_a, idir_a, -ray.o_a idir_a) per node (s_a idir_a is exact); the
-// near plane of each axis (by the sign of idir_a) gives the entry and the far
-// plane the exit, so no per-axis min / max is needed.  With M = sc.qmag,
-// u = 2^-24 and slack = 16 u |idir_a| (M + |ray.o_a|), the distance differs
-// from the exact one to the host's plane by at most six roundings (idir
-// against 1 / d, the plane's own, -ray.o_a idir_a, the slack's addition and
-// the two fmas), each within u (|idir_a| (M + |ray.o_a|) + slack): under half
-// the slack, which is subtracted from entries (R.pn) and added to exits
-// (R.pf), so no box that the ray meets in exact arithmetic is culled.
-__device__ __forceinline__ void box4_q(const DevScene& sc, const RayState& R, float tn[4], float tf[4],
-                                       uint32_t ch[4], uint32_t cn[4]) {
-  const uint4* N = (const uint4*)(sc.nodes4q + R.node);
-  const uint4 A = N[0], B = N[1], C = N[2], D = N[3];
-  const float sx = __uint_as_float((A.w & 0xFFu) << 23) * R.idir.x;
-  const float sy = __uint_as_float(((A.w >> 8) & 0xFFu) << 23) * R.idir.y;
-  const float sz = __uint_as_float(((A.w >> 16) & 0xFFu) << 23) * R.idir.z;
-  const float ox = __uint_as_float(A.x), oy = __uint_as_float(A.y), oz = __uint_as_float(A.z);
-  const float nx = __builtin_fmaf(ox, R.idir.x, R.pn.x), fx = __builtin_fmaf(ox, R.idir.x, R.pf.x);
-  const float ny = __builtin_fmaf(oy, R.idir.y, R.pn.y), fy = __builtin_fmaf(oy, R.idir.y, R.pf.y);
-  const float nz = __builtin_fmaf(oz, R.idir.z, R.pn.z), fz = __builtin_fmaf(oz, R.idir.z, R.pf.z);
-  const bool px = R.idir.x >= 0.f, py = R.idir.y >= 0.f, pz = R.idir.z >= 0.f;
-  const uint32_t qnx = px ? B.x : B.y, qfx = px ? B.y : B.x;
-  const uint32_t qny = py ? B.z : B.w, qfy = py ? B.w : B.z;
-  const uint32_t qnz = pz ? C.x : C.y, qfz = pz ? C.y : C.x;
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    const int sh = 8 * c;
-    const float ex = __builtin_fmaf((float)((qnx >> sh) & 0xFFu), sx, nx);
-    const float ey = __builtin_fmaf((float)((qny >> sh) & 0xFFu), sy, ny);
-    const float ez = __builtin_fmaf((float)((qnz >> sh) & 0xFFu), sz, nz);
-    const float lx = __builtin_fmaf((float)((qfx >> sh) & 0xFFu), sx, fx);
-    const float ly = __builtin_fmaf((float)((qfy >> sh) & 0xFFu), sy, fy);
-    const float lz = __builtin_fmaf((float)((qfz >> sh) & 0xFFu), sz, fz);
-    tn[c] = fmaxf(fmaxf(ex, ey), fmaxf(ez, 0.f));
-    tf[c] = fminf(fminf(lx, ly), lz);
-  }
-  cn[0] = C.z & 0xFFFFu; cn[1] = C.z >> 16; cn[2] = C.w & 0xFFFFu; cn[3] = C.w >> 16;
-  ch[0] = D.x; ch[1] = D.y; ch[2] = D.z; ch[3] = D.w;
-}
-
-// The four child boxes of node R.node (either layout): entry / exit
-// distances, children and leaf counts.
-template <bool Q>
+// The four child boxes of node R.node: entry / exit distances (entry clamped
+// at 0), children and leaf counts.
 __device__ __forceinline__ void child_boxes(const DevScene& sc, const RayState& R, float tn[4], float tf[4],
                                             uint32_t ch[4], uint32_t cn[4]) {
-  if constexpr (Q) {
-    box4_q(sc, R, tn, tf, ch, cn);
-  } else {
-    NodeView nv;
-    load_node(sc, R.node, nv);
+  NodeView nv;
+  load_node(sc, R.node, nv);
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-      float t0x = (nv.lx[c] - R.o.x) * R.idir.x, t1x = (nv.hx[c] - R.o.x) * R.idir.x;
-      float t0y = (nv.ly[c] - R.o.y) * R.idir.y, t1y = (nv.hy[c] - R.o.y) * R.idir.y;
-      float t0z = (nv.lz[c] - R.o.z) * R.idir.z, t1z = (nv.hz[c] - R.o.z) * R.idir.z;
-      tn[c] = fmaxf(fmaxf(fminf(t0x, t1x), fminf(t0y, t1y)), fmaxf(fminf(t0z, t1z), 0.f));
-      tf[c] = fminf(fminf(fmaxf(t0x, t1x), fmaxf(t0y, t1y)), fmaxf(t0z, t1z)) * 1.0000004f;
-      ch[c] = nv.ch[c];
-      cn[c] = nv.cn[c];
-    }
+  for (int c = 0; c < 4; c++) {
+    float t0x = (nv.lx[c] - R.o.x) * R.idir.x, t1x = (nv.hx[c] - R.o.x) * R.idir.x;
+    float t0y = (nv.ly[c] - R.o.y) * R.idir.y, t1y = (nv.hy[c] - R.o.y) * R.idir.y;
+    float t0z = (nv.lz[c] - R.o.z) * R.idir.z, t1z = (nv.hz[c] - R.o.z) * R.idir.z;
+    tn[c] = fmaxf(fmaxf(fminf(t0x, t1x), fminf(t0y, t1y)), fmaxf(fminf(t0z, t1z), 0.f));
+    tf[c] = fminf(fminf(fmaxf(t0x, t1x), fmaxf(t0y, t1y)), fmaxf(t0z, t1z)) * 1.0000004f;
+    ch[c] = nv.ch[c];
+    cn[c] = nv.cn[c];
   }
 }
 
@@ -303,12 +246,12 @@ __device__ __forceinline__ bool pop_node(RayState& R, const LdsU64* lstk, const 
 // spill (an LDS word of the wave, or null) counts pushes that land below the
 // LDS top, in the private (scratch) stack: an LDS atomic on that rare event
 // instead of a counter register in the loop.
-template <bool ANY, int STK, bool Q>
+template <bool ANY, int STK>
 __device__ __forceinline__ bool ray_step(const DevScene& sc, RayState& R, bool cull, LdsU64* lstk, uint64_t* pstk,
                                          uint32_t& nn, uint32_t& nt, uint32_t* spill) {
   float tn[4], tf[4];
   uint32_t ch[4], cn[4];
-  child_boxes<Q>(sc, R, tn, tf, ch, cn);
+  child_boxes(sc, R, tn, tf, ch, cn);
   nn++;
   const float lim = R.h.t + cull_slack(R.h.t, R.eps);
   uint64_t key[4];
@@ -373,17 +316,344 @@ __device__ __forceinline__ bool ray_step(const DevScene& sc, RayState& R, bool c
 }
 
 // Closest (ANY: any) hit of one ray, the loop of ray_step.
-// Q: nodes in the 64-byte quantized layout.
-template <bool ANY, int STK = CPT_LDS_STACK, bool Q = false>
+template <bool ANY, int STK = CPT_LDS_STACK>
 __device__ bool traverse4(const DevScene& sc, f3 o, f3 d, float maxd, float eps, bool cull, LdsU64* lstk,
                           TraceHit& h, uint32_t& nn, uint32_t& nt) {
   RayState R;
-  ray_begin(R, o, d, maxd, eps, sc.qmag);
+  ray_begin(R, o, d, maxd, eps);
   uint64_t pstk[CPT_STACK_TOTAL - STK];
-  while (!ray_step<ANY, STK, Q>(sc, R, cull, lstk, pstk, nn, nt, nullptr)) {
+  while (!ray_step<ANY, STK>(sc, R, cull, lstk, pstk, nn, nt, nullptr)) {
   }
   h = R.h;
   return h.leaf != kInvalid;
+}
+
+// ---- 8-wide traversal -------------------------------------------------------
+// A wave traces its lanes' rays together.  Every step each lane visits one
+// 8-wide quantized node; then all the leaf triangles that the wave's lanes hit
+// in that step are tested as one list, one (ray, triangle) pair per lane
+// whoever's ray it is.  A lane that walks its own triangles makes the wave wait
+// for the longest run (three or four tests a step at a tenth of the lanes), and
+// makes each test's load wait for the one before; the list takes one test
+// and one round trip to memory for up to 64 pairs.  The ray a tester needs (o +
+// eps d, d) and the best hit it competes for live in LDS, one column per lane.
+//
+// What bounds it: VALU instructions where the launch is large (the vector units
+// issue all the time), the chain of node and triangle round trips of the
+// longest ray where it is small; eight children a node shorten both.  FP16
+// fractions cost no conversion (8-bit ones took one per plane: 205 against 150
+// VALU instructions a node).  Over 4-wide 64-byte nodes with each lane walking
+// its own triangles (sphere grid, 1280 x 720, 64 frames): 9.9 -> 6.3 nodes per
+// extension ray, 14.7 -> 8.9 per shadow ray, lane use 37 -> 56 % and more;
+// extension after the first bounce 8.65 -> 7.17 ms, first bounce 3.36 -> 3.24,
+// shadow 13.6 -> 10.4 ms; a frame of 480,000 paths 1.77 -> 1.46 ms.  A node
+// visited again for each child in plain octant order, without the nearest
+// child first and the second nearest's distance to cull the rest by, takes 14 %
+// more visits.
+//
+// The closest hit is the (t, original id) minimum: the order of the tests, the
+// visiting order and the conservative culling do not change it.
+template <int STK>
+struct Wave8 {
+  float ray[6][64];         // o + eps d, d
+  uint64_t best[64];        // t bits << 32 | original id + 1 of the closest hit; low word 0: none
+  uint32_t rec[4][64];      // that hit's t, u, v, device leaf index
+  uint64_t list[64];        // the round's tests: triangle | lane << 32
+  uint64_t stk[STK][64];    // top of the group stacks
+};
+// One ray's traversal: the node to visit next; sx, sy, sz: 16 where the
+// direction is negative (the byte offset of an axis's near plane in a node); pn,
+// pf: -o * idir moved out by the box test's slack, per axis.  A stack entry is a
+// group, the other interior children that the ray hit under one node: the first
+// child's node in the low word, above it the children still to visit (bit slot
+// ^ octant, so that lower bits come first along the ray), the node's interior
+// mask << 8, and the upper half of the bits of a lower bound on their entry
+// distances << 16.
+struct Ray8 {
+  f3 idir, pn, pf;
+  float eps, ht;
+  uint32_t node;
+  int sp;
+};
+
+// LDS accesses of one wave execute in issue order; this keeps the compiler
+// from moving them across the point.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+template <int STK>
+__device__ __forceinline__ void ray8_begin(Ray8& R, Wave8<STK>& W, int lane, f3 o, f3 d, float maxd, float eps,
+                                           float qmag) {
+  // within an ulp of 1 / d: the box test's slack covers it
+  R.idir = mk3(__builtin_amdgcn_rcpf(escape_zero(d.x)), __builtin_amdgcn_rcpf(escape_zero(d.y)),
+               __builtin_amdgcn_rcpf(escape_zero(d.z)));
+  // Slack of the quantized box test (box8): 2^-20 = 16 u per unit of
+  // |idir| (qmag + |o|), twice the rounding bound of that test's distances.
+  const float k = 0x1p-20f;
+  const float sx = (fabsf(R.idir.x) * (qmag + fabsf(o.x))) * k;
+  const float sy = (fabsf(R.idir.y) * (qmag + fabsf(o.y))) * k;
+  const float sz = (fabsf(R.idir.z) * (qmag + fabsf(o.z))) * k;
+  const f3 oi = mk3(-(o.x * R.idir.x), -(o.y * R.idir.y), -(o.z * R.idir.z));
+  R.pn = mk3(oi.x - sx, oi.y - sy, oi.z - sz);
+  R.pf = mk3(oi.x + sx, oi.y + sy, oi.z + sz);
+  R.eps = eps;
+  // no hit lies at t >= 0 below a maximum that is negative or NaN
+  R.ht = maxd > 0.f ? maxd : 0.f;
+  R.node = 0u;
+  R.sp = 0;
+  const f3 o2 = o + d * eps;
+  W.ray[0][lane] = o2.x; W.ray[1][lane] = o2.y; W.ray[2][lane] = o2.z;
+  W.ray[3][lane] = d.x; W.ray[4][lane] = d.y; W.ray[5][lane] = d.z;
+  W.best[lane] = (uint64_t)__float_as_uint(R.ht) << 32;
+}
+// The lane's result once its ray has finished.
+template <int STK>
+__device__ __forceinline__ bool ray8_hit(const Wave8<STK>& W, int lane, TraceHit& h) {
+  const uint32_t id = (uint32_t)W.best[lane];
+  if (id == 0u) {
+    h.t = kInfF; h.u = h.v = 0.f; h.leaf = h.orig = kInvalid;
+    return false;
+  }
+  h.t = __uint_as_float(W.rec[0][lane]);
+  h.u = __uint_as_float(W.rec[1][lane]);
+  h.v = __uint_as_float(W.rec[2][lane]);
+  h.leaf = W.rec[3][lane];
+  h.orig = id - 1u;
+  return true;
+}
+
+// The eight child boxes of a node against the ray: entry distances tn (clamped
+// at 0) and the mask of the boxes the ray meets at or before lim.  A slab plane
+// is o_a + h e_a with h the stored FP16 fraction and e_a a power of two, so its
+// distance (o_a + h e_a - ray.o_a) idir_a is fma(h, e_a idir_a, c_a) with
+// c_a = fma(o_a, idir_a, -ray.o_a idir_a) per node (e_a idir_a is exact); the
+// near plane of each axis (by the sign of idir_a) gives the entry and the far
+// plane the exit, so no per-axis min / max is needed.  With M = sc.qmag,
+// u = 2^-24 and slack = 16 u |idir_a| (M + |ray.o_a|), the distance differs
+// from the exact one to the host's plane by at most seven roundings (two for
+// idir, within an ulp of 1 / d, the plane's own, -ray.o_a idir_a, the slack's
+// addition and the two fmas), each within u (|idir_a| (M + |ray.o_a|) + slack):
+// under half the slack, which is subtracted from entries (R.pn) and added to exits
+// (R.pf), so no box that the ray meets in exact arithmetic is culled.
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ uint32_t box8(const char* __restrict__ nodes, uint32_t node, const Ray8& R, float lim,
+                                         float tn[8], uint4& A, uint4& B) {
+  const uint32_t at = node * 128u;
+  const uint32_t ox = R.idir.x >= 0.f ? 0u : 16u, oy = R.idir.y >= 0.f ? 0u : 16u, oz = R.idir.z >= 0.f ? 0u : 16u;
+  A = *(const uint4*)(nodes + at);
+  const h8 nx = *(const h8*)(nodes + (at | ox) + 32), fx = *(const h8*)(nodes + ((at | ox) ^ 16u) + 32);
+  const h8 ny = *(const h8*)(nodes + (at | oy) + 64), fy = *(const h8*)(nodes + ((at | oy) ^ 16u) + 64);
+  const h8 nz = *(const h8*)(nodes + (at | oz) + 96), fz = *(const h8*)(nodes + ((at | oz) ^ 16u) + 96);
+  B = *(const uint4*)(nodes + at + 16);
+  const float ex = __uint_as_float((A.w & 0xFFu) << 23) * R.idir.x;
+  const float ey = __uint_as_float(((A.w >> 8) & 0xFFu) << 23) * R.idir.y;
+  const float ez = __uint_as_float(((A.w >> 16) & 0xFFu) << 23) * R.idir.z;
+  const float qx = __uint_as_float(A.x), qy = __uint_as_float(A.y), qz = __uint_as_float(A.z);
+  const float cnx = __builtin_fmaf(qx, R.idir.x, R.pn.x), cfx = __builtin_fmaf(qx, R.idir.x, R.pf.x);
+  const float cny = __builtin_fmaf(qy, R.idir.y, R.pn.y), cfy = __builtin_fmaf(qy, R.idir.y, R.pf.y);
+  const float cnz = __builtin_fmaf(qz, R.idir.z, R.pn.z), cfz = __builtin_fmaf(qz, R.idir.z, R.pf.z);
+  uint32_t hits = 0;
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    const float ax = __builtin_fmaf((float)nx[c], ex, cnx), bx = __builtin_fmaf((float)fx[c], ex, cfx);
+    const float ay = __builtin_fmaf((float)ny[c], ey, cny), by = __builtin_fmaf((float)fy[c], ey, cfy);
+    const float az = __builtin_fmaf((float)nz[c], ez, cnz), bz = __builtin_fmaf((float)fz[c], ez, cfz);
+    tn[c] = fmaxf(fmaxf(ax, ay), fmaxf(az, 0.f));
+    const float tf = fminf(fminf(bx, by), fminf(bz, lim));
+    hits |= tn[c] <= tf ? 1u << c : 0u;
+  }
+  return hits;
+}
+
+// The wave's pending leaf triangles (tmask: bits of `valid`, the node's first
+// triangle tbase), tested against their lanes' rays, up to 64 a round.  Called
+// by the whole wave.
+template <int STK>
+__device__ __forceinline__ void test_pairs(const DevScene& sc, Wave8<STK>& W, int lane, uint32_t tmask,
+                                           uint32_t valid, uint32_t tbase, bool cull) {
+  uint32_t n = 0;                                   // pairs listed (uniform)
+  for (;;) {
+    const uint64_t more = __ballot(tmask != 0u);
+    const uint32_t m = (uint32_t)__popcll(more);
+    if (m != 0u && n + m <= 64u) {                  // every lane with triangles left lists its next one
+      if (tmask) {
+        const uint32_t pos =
+            n + __builtin_amdgcn_mbcnt_hi((uint32_t)(more >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)more, 0u));
+        const uint32_t low = tmask - 1u, below = low & ~tmask;
+        W.list[pos] = (uint64_t)(tbase + (uint32_t)__popc(valid & below)) | ((uint64_t)(uint32_t)lane << 32);
+        tmask &= low;
+      }
+      n += m;
+      continue;
+    }
+    wave_lds_order();
+    if ((uint32_t)lane < n) {
+      const uint64_t e = W.list[lane];
+      const uint32_t i = (uint32_t)e, own = (uint32_t)(e >> 32);
+      const float4* T = sc.tris8 + 3 * (size_t)i;
+      const float4 a = T[0], b = T[1], c = T[2];
+      const f3 o2 = mk3(W.ray[0][own], W.ray[1][own], W.ray[2][own]);
+      const f3 d = mk3(W.ray[3][own], W.ray[4][own], W.ray[5][own]);
+      // all of the triangle in one round trip, not its vertex in a second one
+      asm volatile("" : : "v"(a.x), "v"(a.y), "v"(a.z));
+      float u = 0.f, v = 0.f;
+      const float t = isect_tri(o2, d, ld3(a), ld3(b), ld3(c), cull, u, v);
+      if (t >= 0.f && t != kInfF) {                 // kInfF: missed
+        // t + 0: a hit at -0 orders as 0
+        const uint64_t key = ((uint64_t)__float_as_uint(t + 0.f) << 32) | (__float_as_uint(a.w) + 1u);
+        __hip_atomic_fetch_min(&W.best[own], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        wave_lds_order();
+        if (W.best[own] == key) {                   // each triangle is tested once per ray: one winner
+          W.rec[0][own] = __float_as_uint(t);
+          W.rec[1][own] = __float_as_uint(u);
+          W.rec[2][own] = __float_as_uint(v);
+          W.rec[3][own] = __float_as_uint(b.w);
+        }
+      }
+    }
+    wave_lds_order();
+    if (m == 0u) break;
+    n = 0;
+  }
+}
+
+// One step of the wave's active rays: a node visit each, the wave's triangle
+// tests, and each ray's next node: the nearest interior child hit, the others
+// pushed as one group (with the second nearest's distance), or else the first
+// child left of the top group that is still in front of the best hit.  Lanes
+// without a ray visit node R.node again for nothing (a branch round the visit
+// costs two dozen moves of its results) and take part in the triangle tests.
+// Clears `active` of the rays that finish.  spill (an LDS word of the wave, or
+// null) counts group pushes below the LDS top, into the private (scratch)
+// stack.
+template <bool ANY, int STK>
+__device__ __forceinline__ void ray8_step(const DevScene& sc, Ray8& R, bool& active, bool cull, Wave8<STK>& W,
+                                          LdsU64* stk, uint64_t* pstk, int lane, uint32_t& nn, uint32_t& nt,
+                                          uint32_t* spill) {
+  float tn[8];
+  uint4 A, B;
+  const uint32_t hits =
+      box8((const char*)sc.nodes8, R.node, R, R.ht + cull_slack(R.ht, R.eps), tn, A, B);
+  const uint32_t imask = A.w >> 24;
+  // the four triangle bits of each slot hit
+  uint32_t x = active ? hits : 0u;
+  x = (x | (x << 12)) & 0x000F000Fu;
+  x = (x | (x << 6)) & 0x03030303u;
+  x = (x | (x << 3)) & 0x11111111u;
+  const uint32_t tmask = ((x << 4) - x) & B.z;
+  nn += active ? 1u : 0u;
+  nt += (uint32_t)__popc(tmask);
+  if (__ballot(tmask != 0u)) {
+    test_pairs(sc, W, lane, tmask, B.z, B.y, cull);
+    const uint64_t best = W.best[lane];
+    if (ANY) {
+      if ((uint32_t)best != 0u) active = false;
+    } else if (active) {
+      R.ht = __uint_as_float((uint32_t)(best >> 32));
+    }
+  }
+  if (active) {
+    const uint32_t inner = hits & imask;
+    if (inner) {
+      // the two smallest entry distances, the child's slot in the low three bits
+      uint32_t k[8];
+#pragma unroll
+      for (int c = 0; c < 8; c++)
+        k[c] = ((__float_as_uint(tn[c]) & ~7u) | (uint32_t)c) |
+               (uint32_t)((int32_t)(~inner << (31 - c)) >> 31);
+      uint32_t m1 = min(k[0], k[1]), m2 = max(k[0], k[1]);
+#pragma unroll
+      for (int c = 2; c < 8; c += 2) {
+        const uint32_t lo = min(k[c], k[c + 1]), hi = max(k[c], k[c + 1]);
+        m2 = min(m2, max(min(m1, hi), lo));         // the median of m1, lo <= hi
+        m1 = min(m1, lo);
+      }
+      const uint32_t s = m1 & 7u;
+      R.node = B.x + (uint32_t)__popc(imask & ((1u << s) - 1u));
+      uint32_t rest = inner & ~(1u << s);
+      if (rest) {
+        if (!(R.idir.x >= 0.f)) rest = ((rest & 0x55u) << 1) | ((rest >> 1) & 0x55u);
+        if (!(R.idir.y >= 0.f)) rest = ((rest & 0x33u) << 2) | ((rest >> 2) & 0x33u);
+        if (!(R.idir.z >= 0.f)) rest = ((rest & 0x0Fu) << 4) | (rest >> 4);
+        const uint64_t e = (uint64_t)B.x | ((uint64_t)((m2 & 0xFFFF0000u) | (imask << 8) | rest) << 32);
+        if (R.sp < STK) {
+          stk[R.sp * 64] = e;
+        } else {
+          pstk[R.sp - STK] = e;
+          if (spill) atomicAdd(spill, 1u);
+        }
+        R.sp++;
+      }
+    } else {
+      const float lim = R.ht + cull_slack(R.ht, R.eps);
+      for (;;) {
+        if (R.sp == 0) { active = false; break; }
+        uint64_t e;
+        if (R.sp <= STK) e = stk[(R.sp - 1) * 64]; else e = pstk[R.sp - 1 - STK];
+        const uint32_t w = (uint32_t)(e >> 32);
+        if (__uint_as_float(w & 0xFFFF0000u) > lim) { R.sp--; continue; }
+        const uint32_t oct = (R.idir.x >= 0.f ? 0u : 1u) | (R.idir.y >= 0.f ? 0u : 2u) | (R.idir.z >= 0.f ? 0u : 4u);
+        const uint32_t s = (uint32_t)__builtin_ctz(w) ^ oct;
+        R.node = (uint32_t)e + (uint32_t)__popc((w >> 8) & 0xFFu & ((1u << s) - 1u));
+        const uint32_t left = w & (w - 1u);
+        if (left & 0xFFu) {
+          if (R.sp <= STK) stk[(R.sp - 1) * 64] = (uint64_t)(uint32_t)e | ((uint64_t)left << 32);
+          else pstk[R.sp - 1 - STK] = (uint64_t)(uint32_t)e | ((uint64_t)left << 32);
+        } else {
+          R.sp--;
+        }
+        break;
+      }
+    }
+  }
+}
+
+// Private stack entries below an STK-entry LDS top.
+template <int STK>
+constexpr int kPriv8 = (int)kMaxDepth8 - STK;
+
+// Closest (ANY: any) hit of the wave's rays, one per active lane.  Called by
+// the whole wave.
+template <bool ANY, int STK>
+__device__ bool trace8(const DevScene& sc, Wave8<STK>& W, bool active, f3 o, f3 d, float maxd, float eps, bool cull,
+                       TraceHit& h, uint32_t& nn, uint32_t& nt) {
+  const int lane = threadIdx.x & 63;
+  uint64_t pstk[kPriv8<STK>];
+  Ray8 R = {};                                      // lanes without a ray visit the root
+  const bool traced = active;
+  if (active) ray8_begin(R, W, lane, o, d, maxd, eps, sc.qmag);
+  while (__ballot(active))
+    ray8_step<ANY, STK>(sc, R, active, cull, W, (LdsU64*)&W.stk[0][lane], pstk, lane, nn, nt, nullptr);
+  return traced && ray8_hit(W, lane, h);
+}
+
+// LDS of a workgroup's traversals: 8-wide (Q) or 4-wide nodes.  STK is the
+// traversal variant's stack entries; a group entry stands for up to seven
+// nodes, so the 8-wide top takes fewer (six: six workgroups fit a compute
+// unit's LDS).
+template <int STK>
+constexpr int kStk8 = STK == 8 ? 6 : STK == 16 ? 10 : 14;
+template <int STK, bool Q>
+struct TravLds;
+template <int STK>
+struct TravLds<STK, true> {
+  Wave8<kStk8<STK>> w[kBlock / 64];
+};
+template <int STK>
+struct TravLds<STK, false> {
+  uint64_t stk[STK * kBlock];
+};
+// Closest (ANY: any) hit of every active thread's ray.  Called by whole waves.
+template <bool ANY, int STK, bool Q>
+__device__ __forceinline__ bool trace_rays(const DevScene& sc, TravLds<STK, Q>& L, bool active, f3 o, f3 d,
+                                           float maxd, float eps, bool cull, TraceHit& h, uint32_t& nn,
+                                           uint32_t& nt) {
+  if constexpr (Q)
+    return trace8<ANY>(sc, L.w[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)], active, o, d, maxd, eps, cull, h,
+                       nn, nt);
+  else
+    return active && traverse4<ANY, STK>(sc, o, d, maxd, eps, cull, lds_column(L.stk), h, nn, nt);
 }
 
 // Same query over the reference's binary layout (right child popped first).
@@ -509,6 +779,7 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
 static bool pathbuf_ok(const PathBuf& b) {
   return b.ray_o && b.ray_d && b.pix && b.sid && b.depth && b.mul && b.smp && b.acc && b.rng;
 }
+static bool nodes_ok(const DevScene& sc, int quant) { return quant ? sc.nodes8 && sc.tris8 : sc.nodes4 != nullptr; }
 static bool rec_ok(const SampleRec& r) { return r.acc && r.gpos && r.gnrm && r.gdif; }
 
 // ---------------------------------------------------------------- trace API
@@ -520,17 +791,23 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace(DevScene sc, const float
                                                   const float4* __restrict__ rd, uint32_t stride,
                                                   const uint32_t* __restrict__ countp, uint32_t n, uint32_t cull,
                                                   float4* __restrict__ out, DevStats* __restrict__ stats) {
-  __shared__ uint64_t lstk[STK * kBlock];
+  __shared__ TravLds<STK, LAYOUT == 2> lds;
   uint32_t count = countp ? *countp : n;
   uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   uint32_t nn = 0, nt = 0;
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
   if (i < count) {
-    float4 a = ro[(size_t)i * stride], b = rd[(size_t)i * stride];
-    TraceHit h;
-    bool hit = LAYOUT == 0   ? traverse4<ANY, STK>(sc, ld3(a), ld3(b), a.w, b.w, cull != 0, lds_column(lstk), h, nn, nt)
-               : LAYOUT == 2 ? traverse4<ANY, STK, true>(sc, ld3(a), ld3(b), a.w, b.w, cull != 0, lds_column(lstk), h,
-                                                         nn, nt)
-                             : traverse_bin<ANY>(sc, ld3(a), ld3(b), a.w, b.w, cull != 0, h, nn, nt);
+    a = ro[(size_t)i * stride];
+    b = rd[(size_t)i * stride];
+  }
+  TraceHit h;
+  bool hit = false;
+  if constexpr (LAYOUT == 1) {
+    if (i < count) hit = traverse_bin<ANY>(sc, ld3(a), ld3(b), a.w, b.w, cull != 0, h, nn, nt);
+  } else {
+    hit = trace_rays<ANY, STK, LAYOUT == 2>(sc, lds, i < count, ld3(a), ld3(b), a.w, b.w, cull != 0, h, nn, nt);
+  }
+  if (i < count) {
     if (OUT == 0) {
       float4 r;
       r.x = __uint_as_float(hit ? h.orig : kInvalid);
@@ -542,8 +819,8 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace(DevScene sc, const float
       float4 r;
       r.x = hit ? h.t : kInfF;
       r.y = __uint_as_float(hit ? h.leaf : kInvalid);
-      r.z = h.u;
-      r.w = h.v;
+      r.z = hit ? h.u : 0.f;
+      r.w = hit ? h.v : 0.f;
       out[i] = r;
     } else if (OUT == 2) {
       ((uint32_t*)out)[i] = hit ? 1u : 0u;
@@ -567,7 +844,8 @@ hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, cons
   dim3 grid((n + kBlock - 1) / kBlock), block(kBlock);
   const float4* ro = rays;
   const float4* rd = rays + 1;
-  if (layout > 2 || (layout == 2 && !sc.nodes4q) || (layout == 0 && !sc.nodes4)) return hipErrorInvalidValue;
+  if (layout == 2 && !sc.nodes8) layout = 0;       // a scene too large for 8-wide nodes
+  if (layout > 2 || (layout == 2 && !sc.tris8) || (layout == 0 && !sc.nodes4)) return hipErrorInvalidValue;
 #define CPT_TR(L, A, O) k_trace<L, A, O><<<grid, block, 0, st>>>(sc, ro, rd, 2, count, n, cull, hits_out, stats)
   if (cost) {
     if (layout == 0) CPT_TR(0, false, 3); else if (layout == 2) CPT_TR(2, false, 3); else CPT_TR(1, false, 3);
@@ -895,10 +1173,11 @@ __device__ __forceinline__ void store_lv(LightVert& V, f3 pos, f3 norm, f3 irrad
 }
 
 // Light-vertex caches, one workgroup per cache slot to build (light_paths <= kBlock).
+template <bool Q>
 __global__ __launch_bounds__(kBlock) void k_light_pass(DevScene sc, FrameArgs fa, LightJobs jobs,
                                                        LightVert* __restrict__ lv_all,
                                                        FrameCounters* __restrict__ fc) {
-  __shared__ uint64_t lstk[CPT_LDS_STACK * kBlock];
+  __shared__ TravLds<8, Q> lds;
   __shared__ uint32_t wcnt[kBlock / 64];
   const uint32_t x = threadIdx.x, L = fa.light_paths;
   uint32_t slot, job_frame;
@@ -957,11 +1236,12 @@ __global__ __launch_bounds__(kBlock) void k_light_pass(DevScene sc, FrameArgs fa
     for (int w = 0; w < kBlock / 64; w++) { if (w < wid) pre += wcnt[w]; total += wcnt[w]; }
     __syncthreads();
     if (total == 0) break;
+    TraceHit h;
+    uint32_t nn = 0, nt = 0;
+    const bool hit = trace_rays<false, 8, Q>(sc, lds, live, orig, dir, kInfF, (float)kBiasEps, false, h, nn, nt);
     if (live) {
       uint32_t slot = cur + pre + below;
-      TraceHit h;
-      uint32_t nn = 0, nt = 0;
-      if (!traverse4<false>(sc, orig, dir, kInfF, (float)kBiasEps, false, (LdsU64*)(lstk + x), h, nn, nt)) {
+      if (!hit) {
         lv[slot] = lv[x];
         live = false;
       } else {
@@ -992,15 +1272,17 @@ __global__ __launch_bounds__(kBlock) void k_light_pass(DevScene sc, FrameArgs fa
   if (x == 0) fc->light_n[slot] = cur;
 }
 hipError_t launch_light_pass(const DevScene& sc, const FrameArgs& fa, const LightJobs& jobs, LightVert* lv,
-                             FrameCounters* fc, hipStream_t st) {
+                             FrameCounters* fc, int quant, hipStream_t st) {
   if (jobs.n == 0 && jobs.dev_groups == 0) return hipSuccess;
-  if (!lv || !fc || fa.light_paths > (uint32_t)kBlock || (sc.n_light_tris && !sc.light_tris) ||
+  if (!lv || !sc.tris || !nodes_ok(sc, quant) || !fc || fa.light_paths > (uint32_t)kBlock || (sc.n_light_tris && !sc.light_tris) ||
       jobs.n > (uint32_t)kLightSlots || jobs.dev_groups > (uint32_t)kLightSlots ||
       (jobs.dev_groups && !fa.frame_dev))
     return hipErrorInvalidValue;
   for (uint32_t j = 0; j < jobs.n; j++)
     if (jobs.slot[j] >= (uint32_t)kLightSlots) return hipErrorInvalidValue;
-  k_light_pass<<<jobs.dev_groups ? jobs.dev_groups : jobs.n, kBlock, 0, st>>>(sc, fa, jobs, lv, fc);
+  const uint32_t grid = jobs.dev_groups ? jobs.dev_groups : jobs.n;
+  if (quant) k_light_pass<true><<<grid, kBlock, 0, st>>>(sc, fa, jobs, lv, fc);
+  else k_light_pass<false><<<grid, kBlock, 0, st>>>(sc, fa, jobs, lv, fc);
   return hipGetLastError();
 }
 
@@ -1208,7 +1490,7 @@ hipError_t launch_apply_frames(const FrameArgs& fa, const float4* rec_acc, float
 hipError_t launch_extend(const DevScene& sc, PathBuf pb, const FrameCounters* fc, int bounce, uint32_t max_n,
                          float4* hits, DevStats* stats, int lds_stack, int quant, hipStream_t st) {
   if (max_n == 0) return hipSuccess;
-  if (!pathbuf_ok(pb) || !fc || !hits || !sc.tris || !(quant ? (const void*)sc.nodes4q : (const void*)sc.nodes4))
+  if (!pathbuf_ok(pb) || !fc || !hits || !sc.tris || !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
   dim3 grid((max_n + kBlock - 1) / kBlock), block(kBlock);
   const uint32_t* cnt = &fc->active[bounce];
@@ -1234,7 +1516,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_extend_persist(DevScene sc, co
                                                                  uint32_t* __restrict__ queue,
                                                                  float4* __restrict__ out,
                                                                  DevStats* __restrict__ stats) {
-  __shared__ uint64_t lstk[STK * kBlock];
+  __shared__ TravLds<STK, Q> lds;
   __shared__ uint32_t base_s;
   const uint32_t count = *countp;
   uint32_t nn = 0, nt = 0;
@@ -1245,16 +1527,20 @@ __global__ __launch_bounds__(kBlock, MINW) void k_extend_persist(DevScene sc, co
     __syncthreads();
     if (base >= count) break;
     const uint32_t end = min(base + chunk, count);
-    for (uint32_t i = base + threadIdx.x; i < end; i += kBlock) {
-      float4 a = ro[i], b = rd[i];
+    for (uint32_t b0 = base; b0 < end; b0 += kBlock) {       // workgroup-uniform
+      const uint32_t i = b0 + threadIdx.x;
+      float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+      if (i < end) { a = ro[i]; b = rd[i]; }
       TraceHit h;
-      bool hit = traverse4<false, STK, Q>(sc, ld3(a), ld3(b), a.w, b.w, false, lds_column(lstk), h, nn, nt);
-      float4 r;
-      r.x = hit ? h.t : kInfF;
-      r.y = __uint_as_float(hit ? h.leaf : kInvalid);
-      r.z = h.u;
-      r.w = h.v;
-      out[i] = r;
+      const bool hit = trace_rays<false, STK, Q>(sc, lds, i < end, ld3(a), ld3(b), a.w, b.w, false, h, nn, nt);
+      if (i < end) {
+        float4 r;
+        r.x = hit ? h.t : kInfF;
+        r.y = __uint_as_float(hit ? h.leaf : kInvalid);
+        r.z = hit ? h.u : 0.f;
+        r.w = hit ? h.v : 0.f;
+        out[i] = r;
+      }
     }
   }
   if (stats) {
@@ -1269,7 +1555,7 @@ hipError_t launch_extend_persist(const DevScene& sc, PathBuf pb, const FrameCoun
                                  DevStats* stats, int lds_stack, int quant, uint32_t chunk, uint32_t grid,
                                  uint32_t* queue, hipStream_t st) {
   if (!pathbuf_ok(pb) || !fc || !hits || !sc.tris || !queue || chunk == 0 || grid == 0 ||
-      !(quant ? (const void*)sc.nodes4q : (const void*)sc.nodes4))
+      !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
   k_fill_u32<<<1, 1, 0, st>>>(queue, 0u);
   const uint32_t* cnt = &fc->active[bounce];
@@ -1312,11 +1598,12 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
                                                             DevStats* __restrict__ stats, uint32_t refill,
                                                             FrameArgs fa) {
   constexpr bool ANY = OUT == 3;
-  __shared__ uint64_t lstk_all[STK * kBlock];
-  LdsU64* lstk = lds_column(lstk_all);
-  uint64_t pstk[CPT_STACK_TOTAL - STK];
+  constexpr int S8 = kStk8<STK>;
+  __shared__ TravLds<STK, Q> lds;
+  uint64_t pstk[Q ? kPriv8<S8> : CPT_STACK_TOTAL - STK];
   const uint32_t count = *countp;
   const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint64_t below = (1ull << lane) - 1ull;
   const uint32_t waves = gridDim.x * (kBlock / 64);
   const uint32_t chunk = (uint64_t)count >= (uint64_t)kDynChunk * waves ? kDynChunk : 64u;
@@ -1333,23 +1620,30 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
   bool active = false;
   bool pending = false;                    // finished, result not yet written
   uint32_t ray = 0;
-  RayState R;
+  std::conditional_t<Q, Ray8, RayState> R = {};   // 8-wide: lanes without a ray visit the root
   uint32_t nn = 0, nt = 0;
   __shared__ uint32_t spill_all[kBlock / 64];
-  uint32_t* spill = spill_all + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t* spill = spill_all + wid;
   if (lane == 0) *spill = 0u;
   for (;;) {
     const uint64_t idle = __ballot(!active);
     const uint32_t n_idle = (uint32_t)__popcll(idle);
     if (n_idle >= refill && pending) {
       pending = false;
-      const bool hit = R.h.leaf != kInvalid;
+      TraceHit h;
+      bool hit;
+      if constexpr (Q) {
+        hit = ray8_hit(lds.w[wid], lane, h);
+      } else {
+        h = R.h;
+        hit = h.leaf != kInvalid;
+      }
       if (OUT == 1) {
         float4 r;
-        r.x = hit ? R.h.t : kInfF;
-        r.y = __uint_as_float(hit ? R.h.leaf : kInvalid);
-        r.z = R.h.u;
-        r.w = R.h.v;
+        r.x = hit ? h.t : kInfF;
+        r.y = __uint_as_float(hit ? h.leaf : kInvalid);
+        r.z = hit ? h.u : 0.f;
+        r.w = hit ? h.v : 0.f;
         out[ray] = r;
       } else if (!hit) {
         const float4 c = contrib[ray];
@@ -1378,14 +1672,18 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
         const uint32_t take = min(n_idle - given, cend - cnext);
         if (!active && rank >= given && rank < given + take) {
           ray = cnext + (rank - given);
+          float4 a, b4;
           if (EYE) {
             uint32_t dk;
             const PathState e = eye_slot(fa, ray, dk);
-            ray_begin(R, ld3(e.ro), ld3(e.rd), e.ro.w, e.rd.w, sc.qmag);
+            a = e.ro;
+            b4 = e.rd;
           } else {
-            const float4 a = ro[ray], b4 = rd[ray];
-            ray_begin(R, ld3(a), ld3(b4), a.w, b4.w, sc.qmag);
+            a = ro[ray];
+            b4 = rd[ray];
           }
+          if constexpr (Q) ray8_begin(R, lds.w[wid], lane, ld3(a), ld3(b4), a.w, b4.w, sc.qmag);
+          else ray_begin(R, ld3(a), ld3(b4), a.w, b4.w);
           active = true;
         }
         cnext += take;
@@ -1394,7 +1692,12 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
     }
     // every lane idle with nothing left to take: the results were written above
     if (__ballot(active) == 0ull) break;
-    if (active && ray_step<ANY, STK, Q>(sc, R, false, lstk, pstk, nn, nt, spill)) {
+    if constexpr (Q) {
+      const bool was = active;
+      ray8_step<ANY, S8>(sc, R, active, false, lds.w[wid], (LdsU64*)&lds.w[wid].stk[0][lane], pstk, lane, nn, nt,
+                         spill);
+      if (was && !active) pending = true;
+    } else if (active && ray_step<ANY, STK>(sc, R, false, lds_column(lds.stk), pstk, nn, nt, spill)) {
       active = false;
       pending = true;
     }
@@ -1414,7 +1717,7 @@ hipError_t launch_trace_dyn(const DevScene& sc, const float4* ro, const float4* 
                             int quant, int shadow, uint32_t grid, uint32_t refill, uint32_t* queue,
                             hipStream_t st, const FrameArgs* eye) {
   if (!ro || !rd || !count || !queue || grid == 0 || refill < 1 || refill > 64 || !sc.tris ||
-      !(quant ? (const void*)sc.nodes4q : (const void*)sc.nodes4))
+      !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
   if (shadow ? (!contrib || !pathbuf_ok(nxt) || eye) : !out) return hipErrorInvalidValue;
   const FrameArgs fa = eye ? *eye : FrameArgs{};
@@ -1954,14 +2257,20 @@ template <int STK, int MINW = 0, bool Q = false>
 __global__ __launch_bounds__(kBlock, MINW) void k_shadow(DevScene sc, ShadowBuf sb, PathBuf nxt,
                                                    const FrameCounters* __restrict__ fc, int bounce,
                                                    DevStats* __restrict__ stats) {
-  __shared__ uint64_t lstk[STK * kBlock];
+  __shared__ TravLds<STK, Q> lds;
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   const uint32_t count = fc->shadow[bounce];
   uint32_t nn = 0, nt = 0;
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
   if (i < count) {
-    float4 a = sb.ray_o[i], b = sb.ray_d[i], c = sb.contrib[i];
-    TraceHit h;
-    if (!traverse4<true, STK, Q>(sc, ld3(a), ld3(b), a.w, b.w, false, lds_column(lstk), h, nn, nt)) {
+    a = sb.ray_o[i];
+    b = sb.ray_d[i];
+  }
+  TraceHit h;
+  const bool hit = trace_rays<true, STK, Q>(sc, lds, i < count, ld3(a), ld3(b), a.w, b.w, false, h, nn, nt);
+  if (i < count) {
+    if (!hit) {
+      const float4 c = sb.contrib[i];
       const uint32_t bits = __float_as_uint(c.w), slot = bits & ~kShadowNoCount;
       float4 acc = nxt.acc[slot];
       acc.x = acc.x + c.x;
@@ -1983,7 +2292,7 @@ hipError_t launch_shadow(const DevScene& sc, ShadowBuf sb, PathBuf nxt, const Fr
                          uint32_t max_n, int lds_stack, int quant, DevStats* stats, hipStream_t st) {
   if (max_n == 0) return hipSuccess;
   if (!pathbuf_ok(nxt) || !sb.ray_o || !sb.ray_d || !sb.contrib || !fc || !sc.tris ||
-      !(quant ? (const void*)sc.nodes4q : (const void*)sc.nodes4))
+      !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
   dim3 grid((max_n + kBlock - 1) / kBlock), block(kBlock);
 #define CPT_SH(S, W, Q) k_shadow<S, W, Q><<<grid, block, 0, st>>>(sc, sb, nxt, fc, bounce, stats)
@@ -2118,10 +2427,10 @@ hipError_t launch_regen(const FrameArgs& fa, PathBuf pb, const Accum& ac, FrameC
 constexpr uint32_t kRegenLightN = kRegenLightVerts, kRegenLightDepth = 5, kRegenMaxLevels = 8;
 constexpr uint32_t kDomainRegenLight = 4u, kDomainRegenEye = 5u;
 
+template <bool Q>
 __global__ __launch_bounds__(kRegenLightN / kRegenLightDepth) void k_regen_light(DevScene sc, FrameArgs fa,
                                                                                   LightVert* __restrict__ lv) {
-  __shared__ uint64_t lstk_all[CPT_LDS_STACK * kBlock];   // column layout: the stride is kBlock
-  LdsU64* lstk = lds_column(lstk_all);
+  __shared__ TravLds<8, Q> lds;
   const uint32_t x = threadIdx.x;
   const uint64_t inc = ((uint64_t)x << 1) | 1u;
   uint64_t st;
@@ -2134,7 +2443,11 @@ __global__ __launch_bounds__(kRegenLightN / kRegenLightDepth) void k_regen_light
     bool nvalid = false;
     LightVert& V = lv[x * kRegenLightDepth + k];
     store_lv(V, o * 0.f, o * 0.f, o * 0.f, o * 0.f, none);
-    if (!valid || length(irr) < (float)kBiasEps) {
+    const bool start = !valid || length(irr) < (float)kBiasEps;
+    TraceHit h;
+    uint32_t nn = 0, nt = 0;
+    const bool hit = trace_rays<false, 8, Q>(sc, lds, !start, o, d, kInfF, (float)kBiasEps, false, h, nn, nt);
+    if (start) {
       if (sc.n_light_tris > 0) {                         // a new path on an emitter (:94-158)
         uint32_t id = (uint32_t)(uniform01(st, inc) * (float)sc.n_light_tris);
         if (id >= sc.n_light_tris) id = sc.n_light_tris - 1;
@@ -2155,9 +2468,7 @@ __global__ __launch_bounds__(kRegenLightN / kRegenLightDepth) void k_regen_light
         store_lv(V, s.pos, s.norm, s.emissive, mk3(0.f, 0.f, 0.f), s);
       }
     } else {
-      TraceHit h;
-      uint32_t nn = 0, nt = 0;
-      if (traverse4<false>(sc, o, d, kInfF, (float)kBiasEps, false, lstk, h, nn, nt)) {   // :159-299
+      if (hit) {                                         // :159-299
         const float w = (1.f - h.u) - h.v;
         const Surf s = fetch_surf(sc, h.leaf, w, h.u, h.v, true);
         const f3 nl = dot(s.norm, d) < 0.f ? s.norm : s.norm * -1.f;
@@ -2180,12 +2491,12 @@ template <int STK, bool Q>
 __global__ __launch_bounds__(kBlock) void k_regen_eye(DevScene sc, FrameArgs fa, const LightVert* __restrict__ lv,
                                                       float* __restrict__ result, uint32_t* __restrict__ sample_n,
                                                       DevStats* __restrict__ stats) {
-  __shared__ uint64_t lstk_all[STK * kBlock];
-  LdsU64* lstk = lds_column(lstk_all);
+  __shared__ TravLds<STK, Q> lds;
   const uint32_t W = fa.width, H = fa.height, pix = blockIdx.x * kBlock + threadIdx.x;
   const int lane = threadIdx.x & 63;
   uint32_t ext = 0, shr = 0, paths = 0, en = 0, et = 0, sn = 0, stc = 0;
-  if (pix < W * H) {
+  {                                                      // whole waves: lanes past the image carry no path
+    bool live = pix < W * H;
     const uint32_t levels = fa.eye_depth < kRegenMaxLevels ? fa.eye_depth : kRegenMaxLevels;
     const uint32_t y = pix / W, x = pix - y * W;
     const uint64_t inc = ((uint64_t)pix << 1) | 1u;
@@ -2208,22 +2519,33 @@ __global__ __launch_bounds__(kBlock) void k_regen_eye(DevScene sc, FrameArgs fa,
     uint32_t depth = 0, count = 0, D = levels;
     f3 mul[kRegenMaxLevels], em[kRegenMaxLevels], con[kRegenMaxLevels];   // per level: f, emission, connection
     uint32_t bank = 0;                                     // levels where a camera path starts
-    paths = 1;
+    paths = live;
     for (uint32_t L = 0; L < levels; L++) {
+      if (__ballot(live) == 0ull) break;                 // wave-uniform
       TraceHit h;
-      ext++;
-      if (!traverse4<false, STK, Q>(sc, o, d, kInfF, (float)kBiasEps, false, lstk, h, en, et)) {   // :620-623
+      ext += live;
+      const bool hit = trace_rays<false, STK, Q>(sc, lds, live, o, d, kInfF, (float)kBiasEps, false, h, en, et);
+      if (live && !hit) {                                // :620-623
         D = L;
-        break;
+        live = false;
       }
+      // the level's bounce; a connection waits for its occlusion test below
+      Surf s;
+      Bounce b;
+      f3 nl, P = o, toL = d, no = o, nd = d;
+      float dist = 0.f;
+      bool diffuse = false, lit = false;
+      uint32_t li = 0;
+      if (live) {
       const float w = (1.f - h.u) - h.v;
-      const Surf s = fetch_surf(sc, h.leaf, w, h.u, h.v, true);
-      const f3 nl = dot(s.norm, d) < 0.f ? s.norm : s.norm * -1.f;
-      const Bounce b = sample_bounce(st, inc, o, d, h.t, s, nl, RT_EYE, false, true);
+      s = fetch_surf(sc, h.leaf, w, h.u, h.v, true);
+      nl = dot(s.norm, d) < 0.f ? s.norm : s.norm * -1.f;
+      b = sample_bounce(st, inc, o, d, h.t, s, nl, RT_EYE, false, true);
       weight = weight * length(b.mul);
       if (length(s.emissive) > 0.f) weight = 0.f;
       if (depth == 0) bank |= 1u << L;
-      f3 c = mk3(0.f, 0.f, 0.f), no = b.orig, nd = b.dir;
+      no = b.orig;
+      nd = b.dir;
       if (!prob_rand(st, inc, weight)) {                 // a new camera path for the pixel (:562-571)
         weight = 1.f;
         depth = 0;
@@ -2234,33 +2556,46 @@ __global__ __launch_bounds__(kBlock) void k_regen_eye(DevScene sc, FrameArgs fa,
       } else {
         depth++;
         if (b.type == RT_DIFF) {                          // GetLightFromRandLightVertices (:400-431)
-          const f3 P = s.pos + nl * (float)kBiasEps;
-          uint32_t li = (uint32_t)(uniform01(st, inc) * (float)kRegenLightN);
+          diffuse = true;
+          P = s.pos + nl * (float)kBiasEps;
+          li = (uint32_t)(uniform01(st, inc) * (float)kRegenLightN);
           if (li >= kRegenLightN) li = kRegenLightN - 1;
           const LightVert& LV = lv[li];
           const f3 lpos = mk3(LV.pos[0], LV.pos[1], LV.pos[2]), lirr = mk3(LV.irrad[0], LV.irrad[1], LV.irrad[2]);
-          const f3 ldir = mk3(LV.irradDir[0], LV.irradDir[1], LV.irradDir[2]);
-          f3 irrad = mk3(0.f, 0.f, 0.f), irradDir = irrad;
-          const f3 toL = normalize(lpos - P);
-          const float dist = length(lpos - P);
-          if (length(lirr) > 0.f && dot(nl, toL) > 0.f) {
-            TraceHit hs;
-            shr++;
-            if (!traverse4<true, STK, Q>(sc, P, toL, (float)shadow_max((double)dist, fa.flags), (float)kBiasEps,
-                                         false, lstk, hs, sn, stc)) {
-              if (length(ldir) > (float)kFltEps)
-                irrad = shading(toL * -1.f, ldir, lirr, mk3(LV.norm[0], LV.norm[1], LV.norm[2]),
-                                mk3(LV.diff[0], LV.diff[1], LV.diff[2]), LV.metallic, LV.roughness, LV.specular,
-                                1.f, 1.f) +
-                        mk3(LV.emissive[0], LV.emissive[1], LV.emissive[2]);
-              else
-                irrad = lirr;
-              irradDir = toL;
-            }
-          }
-          c = vmax0(shading(d * -1.f, irradDir, irrad, nl, s.diff, s.metal, s.rough, s.spec, 1.f - s.trans, 1.f));
-          if (length(c) > 0.f) count += 4;
+          toL = normalize(lpos - P);
+          dist = length(lpos - P);
+          lit = length(lirr) > 0.f && dot(nl, toL) > 0.f;
         }
+      }
+      }
+      bool occluded = false;
+      if (__ballot(lit)) {
+        TraceHit hs;
+        shr += lit;
+        occluded = trace_rays<true, STK, Q>(sc, lds, lit, P, toL, (float)shadow_max((double)dist, fa.flags),
+                                            (float)kBiasEps, false, hs, sn, stc);
+      }
+      if (!live) continue;
+      f3 c = mk3(0.f, 0.f, 0.f);
+      if (diffuse) {
+        const LightVert& LV = lv[li];
+        f3 irrad = c, irradDir = c;
+        if (lit) {
+          const f3 lirr = mk3(LV.irrad[0], LV.irrad[1], LV.irrad[2]);
+          const f3 ldir = mk3(LV.irradDir[0], LV.irradDir[1], LV.irradDir[2]);
+          if (!occluded) {
+            if (length(ldir) > (float)kFltEps)
+              irrad = shading(toL * -1.f, ldir, lirr, mk3(LV.norm[0], LV.norm[1], LV.norm[2]),
+                              mk3(LV.diff[0], LV.diff[1], LV.diff[2]), LV.metallic, LV.roughness, LV.specular,
+                              1.f, 1.f) +
+                      mk3(LV.emissive[0], LV.emissive[1], LV.emissive[2]);
+            else
+              irrad = lirr;
+            irradDir = toL;
+          }
+        }
+        c = vmax0(shading(d * -1.f, irradDir, irrad, nl, s.diff, s.metal, s.rough, s.spec, 1.f - s.trans, 1.f));
+        if (length(c) > 0.f) count += 4;
       }
       mul[L] = b.mul;
       em[L] = s.emissive;
@@ -2277,6 +2612,7 @@ __global__ __launch_bounds__(kBlock) void k_regen_eye(DevScene sc, FrameArgs fa,
         r = mk3(0.f, 0.f, 0.f);
       }
     }
+    if (pix < W * H) {
     const uint32_t nold = fa.frame0 == 0 ? 0u : sample_n[pix], nn = nold + count;
     const float ri = 1.f / (float)nn, oi = (float)nold * ri;
     float* res = result + (size_t)pix * 3;
@@ -2284,6 +2620,7 @@ __global__ __launch_bounds__(kBlock) void k_regen_eye(DevScene sc, FrameArgs fa,
     res[1] = fmaxf(ri * accum.y + oi * res[1], 0.f);
     res[2] = fmaxf(ri * accum.z + oi * res[2], 0.f);
     sample_n[pix] = nn;
+    }
   }
   if (stats) {
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&stats->frames, 1ull);
@@ -2301,9 +2638,10 @@ __global__ __launch_bounds__(kBlock) void k_regen_eye(DevScene sc, FrameArgs fa,
   }
 }
 
-hipError_t launch_regen_light(const DevScene& sc, const FrameArgs& fa, LightVert* lv, hipStream_t st) {
-  if (!lv || !sc.tris || (sc.n_light_tris && !sc.light_tris)) return hipErrorInvalidValue;
-  k_regen_light<<<1, kRegenLightN / kRegenLightDepth, 0, st>>>(sc, fa, lv);
+hipError_t launch_regen_light(const DevScene& sc, const FrameArgs& fa, LightVert* lv, int quant, hipStream_t st) {
+  if (!lv || !sc.tris || !nodes_ok(sc, quant) || (sc.n_light_tris && !sc.light_tris)) return hipErrorInvalidValue;
+  if (quant) k_regen_light<true><<<1, kRegenLightN / kRegenLightDepth, 0, st>>>(sc, fa, lv);
+  else k_regen_light<false><<<1, kRegenLightN / kRegenLightDepth, 0, st>>>(sc, fa, lv);
   return hipGetLastError();
 }
 hipError_t launch_regen_eye(const DevScene& sc, const FrameArgs& fa, const LightVert* lv, float* result,
@@ -2311,7 +2649,7 @@ hipError_t launch_regen_eye(const DevScene& sc, const FrameArgs& fa, const Light
   const uint64_t n = (uint64_t)fa.width * fa.height;
   if (n == 0) return hipSuccess;
   if (!lv || !result || !sample_n || n > 0xFFFFFFFFull - kBlock || fa.eye_depth < 1 ||
-      fa.eye_depth > kRegenMaxLevels || !sc.tris || !(quant ? (const void*)sc.nodes4q : (const void*)sc.nodes4))
+      fa.eye_depth > kRegenMaxLevels || !sc.tris || !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
   const uint32_t grid = (uint32_t)((n + kBlock - 1) / kBlock);
 #define CPT_RG(S, W, Q) k_regen_eye<S, Q><<<grid, kBlock, 0, st>>>(sc, fa, lv, result, sample_n, stats)
@@ -2342,25 +2680,30 @@ hipError_t launch_regen_eye(const DevScene& sc, const FrameArgs& fa, const Light
 // One bounce of a path that one thread carries (k_mega, k_tail): the closest
 // hit, shade_path, and the occlusion ray of the connection it sets up, whose
 // contribution is added when nothing occludes it.
+// Called by whole waves; `live` lanes carry a path.
 template <int STK, bool Q>
 __device__ __forceinline__ void carry_bounce(const DevScene& sc, const FrameArgs& fa, FrameCounters* fc,
-                                             const LightVert* lv, const Accum& ac, PathState& p, LdsU64* lstk,
-                                             bool& survive, bool& emit, uint32_t& en, uint32_t& et, uint32_t& sn,
-                                             uint32_t& st) {
+                                             const LightVert* lv, const Accum& ac, PathState& p,
+                                             TravLds<STK, Q>& lds, bool live, bool& survive, bool& emit, uint32_t& en,
+                                             uint32_t& et, uint32_t& sn, uint32_t& st) {
   TraceHit h;
-  const bool hit = traverse4<false, STK, Q>(sc, ld3(p.ro), ld3(p.rd), p.ro.w, p.rd.w, false, lstk, h, en, et);
-  const float4 hv = make_float4(hit ? h.t : kInfF, __uint_as_float(hit ? h.leaf : kInvalid), h.u, h.v);
+  const bool hit = trace_rays<false, STK, Q>(sc, lds, live, ld3(p.ro), ld3(p.rd), p.ro.w, p.rd.w, false, h, en, et);
   ShadowRay sr;
   sr.o = sr.d = sr.c = make_float4(0.f, 0.f, 0.f, 0.f);
-  shade_path(sc, fa, fc, lv, ac, p, hv, survive, emit, sr);
-  if (emit) {
-    TraceHit hs;
-    if (!traverse4<true, STK, Q>(sc, ld3(sr.o), ld3(sr.d), sr.o.w, sr.d.w, false, lstk, hs, sn, st)) {
-      p.acc.x = p.acc.x + sr.c.x;
-      p.acc.y = p.acc.y + sr.c.y;
-      p.acc.z = p.acc.z + sr.c.z;
-      p.acc.w = __uint_as_float(__float_as_uint(p.acc.w) + 4u);
-    }
+  if (live) {
+    const float4 hv = make_float4(hit ? h.t : kInfF, __uint_as_float(hit ? h.leaf : kInvalid), hit ? h.u : 0.f,
+                                  hit ? h.v : 0.f);
+    shade_path(sc, fa, fc, lv, ac, p, hv, survive, emit, sr);
+  }
+  if (__ballot(emit) == 0ull) return;                       // wave-uniform
+  TraceHit hs;
+  const bool occluded =
+      trace_rays<true, STK, Q>(sc, lds, emit, ld3(sr.o), ld3(sr.d), sr.o.w, sr.d.w, false, hs, sn, st);
+  if (emit && !occluded) {
+    p.acc.x = p.acc.x + sr.c.x;
+    p.acc.y = p.acc.y + sr.c.y;
+    p.acc.z = p.acc.z + sr.c.z;
+    p.acc.w = __uint_as_float(__float_as_uint(p.acc.w) + 4u);
   }
 }
 
@@ -2402,9 +2745,8 @@ template <int STK, bool Q>
 __global__ __launch_bounds__(kBlock) void k_mega(DevScene sc, FrameArgs fa, FrameCounters* __restrict__ fc,
                                                  const LightVert* __restrict__ lv, Accum ac,
                                                  DevStats* __restrict__ stats) {
-  __shared__ uint64_t lstk_all[STK * kBlock];
+  __shared__ TravLds<STK, Q> lds;
   __shared__ uint32_t n_live[16], n_shadow[16];
-  LdsU64* lstk = lds_column(lstk_all);
   if (threadIdx.x < 16) { n_live[threadIdx.x] = 0u; n_shadow[threadIdx.x] = 0u; }
   __syncthreads();
   const uint32_t wh = fa.width * fa.height;
@@ -2422,10 +2764,8 @@ __global__ __launch_bounds__(kBlock) void k_mega(DevScene sc, FrameArgs fa, Fram
   for (uint32_t b = 0; b < depth; b++) {
     if (__ballot(live) == 0ull) break;                    // wave-uniform
     bool survive = false, emit = false;
-    if (live) {
-      carry_bounce<STK, Q>(sc, fa, fc, lv, ac, p, lstk, survive, emit, en, et, sn, st);
-      live = survive;
-    }
+    carry_bounce<STK, Q>(sc, fa, fc, lv, ac, p, lds, live, survive, emit, en, et, sn, st);
+    live = survive;
     const uint32_t cs = (uint32_t)__popcll(__ballot(survive)), ce = (uint32_t)__popcll(__ballot(emit));
     if (lane == 0) {
       if (cs) atomicAdd(&n_live[b], cs);
@@ -2447,9 +2787,8 @@ __global__ __launch_bounds__(kBlock) void k_tail(DevScene sc, FrameArgs fa, Path
                                                  FrameCounters* __restrict__ fc, uint32_t bounce0,
                                                  const LightVert* __restrict__ lv, Accum ac,
                                                  DevStats* __restrict__ stats) {
-  __shared__ uint64_t lstk_all[STK * kBlock];
+  __shared__ TravLds<STK, Q> lds;
   __shared__ uint32_t n_live[16], n_shadow[16];
-  LdsU64* lstk = lds_column(lstk_all);
   if (threadIdx.x < 16) { n_live[threadIdx.x] = 0u; n_shadow[threadIdx.x] = 0u; }
   __syncthreads();
   const uint32_t count = fc->active[bounce0];
@@ -2481,11 +2820,9 @@ __global__ __launch_bounds__(kBlock) void k_tail(DevScene sc, FrameArgs fa, Path
     for (uint32_t b = bounce0; b < depth; b++) {
       if (__ballot(live) == 0ull) break;                  // wave-uniform
       bool survive = false, emit = false;
-      if (live) {
-        carry_bounce<STK, Q>(sc, fa, fc, lv, ac, p, lstk, survive, emit, en, et, sn, st);
-        live = survive;
-        nr++;
-      }
+      nr += live;
+      carry_bounce<STK, Q>(sc, fa, fc, lv, ac, p, lds, live, survive, emit, en, et, sn, st);
+      live = survive;
       const uint32_t cs = (uint32_t)__popcll(__ballot(survive)), ce = (uint32_t)__popcll(__ballot(emit));
       if (lane == 0) {
         if (cs) atomicAdd(&n_live[b], cs);
@@ -2503,7 +2840,7 @@ hipError_t launch_tail(const DevScene& sc, const FrameArgs& fa, PathBuf cur, Fra
   // variant (written at depth 0 only) is allowed
   if (!fc || !lv || !ac.rec.acc || ac.apply != 2 || fa.eye_depth > 16 ||
       bounce0 == 0 || bounce0 >= fa.eye_depth || grid == 0 || !pathbuf_ok(cur) || !sc.tris ||
-      !(quant ? (const void*)sc.nodes4q : (const void*)sc.nodes4))
+      !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
 #define CPT_TL(S, W, Q) k_tail<S, Q><<<grid, kBlock, 0, st>>>(sc, fa, cur, fc, bounce0, lv, ac, stats)
 #define CPT_TL_Q(S, W) CPT_TL(S, W, true)
@@ -2524,7 +2861,7 @@ hipError_t launch_mega(const DevScene& sc, const FrameArgs& fa, FrameCounters* f
   if (n == 0) return hipSuccess;
   if (n > 0xFFFFFFFFull - kBlock || !fc || !lv || !ac.rec.acc || ac.apply != 2 || (ac.variant & kVariantGbuf) ||
       fa.eye_depth > 16 || !sc.tris ||
-      !(quant ? (const void*)sc.nodes4q : (const void*)sc.nodes4))
+      !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
   dim3 grid((uint32_t)((n + kBlock - 1) / kBlock)), block(kBlock);
 #define CPT_MG(S, W, Q) k_mega<S, Q><<<grid, block, 0, st>>>(sc, fa, fc, lv, ac, stats)

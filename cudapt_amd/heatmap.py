@@ -7,8 +7,8 @@ as written over the reference's binary tree).
 One primary ray per pixel through the pixel centre (the debug renderer's
 pinhole, src/cudaRTBVHDebug.cu:113-117: no jitter), traced closest-hit; the
 map holds each ray's node visits and triangle tests in the chosen layout
-(0: 128-byte 4-wide nodes, 1: the reference's binary tree, 2: 64-byte
-quantized 4-wide nodes).  `to_rgb` renders it as the reference displays cost:
+(0: FP32 4-wide nodes, 1: the reference's binary tree, 2: 8-wide nodes with
+quantized boxes).  `to_rgb` renders it as the reference displays cost:
 red for rays that reach no leaf, green for rays that do, value / 10.
 """
 from __future__ import annotations

@@ -123,8 +123,9 @@ int cpt_bvh_build_sah(cpt_scene* s, uint32_t max_depth);
 int cpt_bvh_export(cpt_scene* s, float* bounds6, uint32_t* off2, uint32_t* reorder, uint32_t* node_n);
 
 /* No reference counterpart: the most triangles a leaf of the 4-wide device BVH
- * holds (1..64, default 2).  The SAH-optimal collapse of the binary tree picks
- * leaves of at most that many triangles.  Applies to the current BVH (rebuilt at once,
+ * holds (1..64, default 2; the 8-wide one holds at most 4 of them).  The
+ * SAH-optimal collapse of the binary tree picks leaves of at most that many
+ * triangles.  Applies to the current BVH (rebuilt at once,
  * uploaded by the next render) and to later builds; hits do not depend on it. */
 int cpt_bvh4_set_leaf_size(cpt_scene* s, uint32_t max_tris);
 
@@ -146,8 +147,8 @@ int cpt_trace_closest(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cu
 
 /* Same over device arrays already resident in HBM, launched on `stream`
  * (a hipStream_t, NULL = the scene's stream).  layout 0 = 4-wide nodes,
- * 1 = the reference's binary CompactBVH layout, 2 = 4-wide nodes quantized to
- * 64 bytes (the same hits: culling stays conservative). */
+ * 1 = the reference's binary CompactBVH layout, 2 = 8-wide nodes with quantized
+ * boxes (the same hits: culling stays conservative). */
 int cpt_trace_closest_device(cpt_scene* s, const cpt_ray* d_rays, uint32_t n, uint32_t cull, cpt_hit* d_hits,
                              void* stream, uint32_t layout);
 
@@ -288,7 +289,7 @@ typedef struct cpt_stats {
   double extend_ms, shadow_ms, shade_ms, light_ms, total_ms;
   double filter_ms, error_ms, gen_ms, accum_ms;   /* adaptive phases (PERFBREAKDOWN, AdapBilatAtomic.cu:1409-1536) */
   double mlp_ms;                                  /* learned error model: features + inference */
-  uint64_t shadow_nodes, shadow_tris;             /* 4-wide nodes visited / triangles tested by shadow rays */
+  uint64_t shadow_nodes, shadow_tris;             /* nodes visited / triangles tested by shadow rays */
   uint64_t extend_spills, shadow_spills;          /* traversal-stack pushes that went past the LDS entries into
                                                      the private (scratch) stack, refilling-wave kernels */
   uint64_t tail_rays, tail_nodes, tail_tris;      /* "Tail Bounce": extension rays traced by the tail kernel, and
@@ -328,7 +329,7 @@ typedef struct cpt_batch_config {
   uint32_t use_graph;         /* 1: capture one iteration as a hipGraph and replay it */
   uint32_t eye_depth, light_depth, light_paths;
   uint64_t seed;
-  uint32_t node_format;       /* 0: 128-byte FP32 4-wide nodes, 1: 64-byte quantized nodes */
+  uint32_t node_format;       /* 0: FP32 4-wide nodes, 1: 8-wide quantized nodes */
   uint32_t refill;            /* extension rays: 0 = as extend_chunk says; 1..64 = persistent waves whose
                                  lanes take new rays once this many are idle (overrides extend_chunk) */
 } cpt_batch_config;
