@@ -128,6 +128,23 @@ struct cpt_scene {
 
 namespace {
 
+// The sum of the device's kStatSlots copies.
+hipError_t read_stats(const DevStats* d, DevStats& out) {
+  std::vector<DevStats> h(kStatSlots);
+  hipError_t e = hipMemcpy(h.data(), d, sizeof(DevStats) * kStatSlots, hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return e;
+  out = h[0];
+  for (u32 i = 1; i < kStatSlots; i++) {
+    const DevStats& x = h[i];
+    out.ext_rays += x.ext_rays; out.shadow_rays += x.shadow_rays; out.eye_paths += x.eye_paths; out.frames += x.frames;
+    out.ext_nodes += x.ext_nodes; out.ext_tris += x.ext_tris;
+    out.sh_nodes += x.sh_nodes; out.sh_tris += x.sh_tris;
+    out.ext_spill += x.ext_spill; out.sh_spill += x.sh_spill;
+    out.tail_rays += x.tail_rays; out.tail_nodes += x.tail_nodes; out.tail_tris += x.tail_tris;
+  }
+  return hipSuccess;
+}
+
 int ensure_stream(hipStream_t& st) {
   if (!st) HIP_TRY(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
   return CPT_OK;
@@ -476,8 +493,8 @@ int cpt_scene_upload(cpt_scene* s) {
   rc = upload_materials(s);
   if (rc) return rc;
   if (!s->d_stats.p) {
-    HIP_TRY(s->d_stats.alloc(1));
-    HIP_TRY(hipMemsetAsync(s->d_stats.p, 0, sizeof(DevStats), s->stream));
+    HIP_TRY(s->d_stats.alloc(kStatSlots));
+    HIP_TRY(hipMemsetAsync(s->d_stats.p, 0, sizeof(DevStats) * kStatSlots, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
   }
   s->uploaded = true;
@@ -614,11 +631,11 @@ int cpt_trace_counters(cpt_scene* s, uint64_t* nodes, uint64_t* tris, uint64_t* 
   if (!s->d_stats.p) return fail(CPT_E_STATE, "cpt_trace_counters: scene not uploaded");
   DevStats h;
   HIP_TRY(hipStreamSynchronize(s->stream));
-  HIP_TRY(hipMemcpy(&h, s->d_stats.p, sizeof h, hipMemcpyDeviceToHost));
+  HIP_TRY(read_stats(s->d_stats.p, h));
   if (nodes) *nodes = h.ext_nodes;
   if (tris) *tris = h.ext_tris;
   if (rays) *rays = h.ext_rays;
-  if (reset) HIP_TRY(hipMemset(s->d_stats.p, 0, sizeof(DevStats)));
+  if (reset) HIP_TRY(hipMemset(s->d_stats.p, 0, sizeof(DevStats) * kStatSlots));
   return CPT_OK;
 }
 
@@ -769,6 +786,7 @@ struct cpt_renderer {
   struct Ev { hipEvent_t a, b; int kind; };
   std::vector<Ev> events;          // recorded pairs awaiting readback
   std::vector<hipEvent_t> pool;    // reusable events
+  int parts = 0;                   // 1: the frame's counts are partly in FrameCounters::part (k_tail, k_mega)
   double ms[11] = {0};  // extend, shadow, shade, light, total, filter, error sum, generation, accumulation, model,
                         // tail
   // shadow rays of bounce b traced on `side` while bounce b + 1's extension
@@ -890,10 +908,10 @@ int renderer_alloc(cpt_renderer* r) {
   }
   HIP_TRY(r->queue.alloc(2));
   HIP_TRY(r->fc.alloc(1));
-  HIP_TRY(r->stats.alloc(1));
+  HIP_TRY(r->stats.alloc(kStatSlots));
   HIP_TRY(r->result.alloc(n * 3));
   HIP_TRY(r->sample_n.alloc(n));
-  HIP_TRY(hipMemsetAsync(r->stats.p, 0, sizeof(DevStats), r->stream));
+  HIP_TRY(hipMemsetAsync(r->stats.p, 0, sizeof(DevStats) * kStatSlots, r->stream));
   HIP_TRY(hipMemsetAsync(r->result.p, 0, sizeof(float) * n * 3, r->stream));
   HIP_TRY(hipMemsetAsync(r->sample_n.p, 0, sizeof(u32) * n, r->stream));
   HIP_TRY(hipMemsetAsync(r->fc.p, 0, sizeof(FrameCounters), r->stream));
@@ -984,6 +1002,7 @@ int update_gauss(cpt_renderer* r, float sigma, u32 radius) {
 int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 max_n, const Accum& ac,
                 bool gen_eye = false) {
   hipEvent_t ev = nullptr;
+  r->parts = 0;
   PathSet* cur = &r->A;
   PathSet* nxt = &r->B;
   ShadowBuf sb;
@@ -1028,6 +1047,7 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
       const uint32_t grid =
           (uint32_t)(r->cus > 0 ? r->cus : 256) * (uint32_t)std::min(32.0, std::max(1.0, r->attr(kRefillGroups)));
       HIP_TRY(timed_begin(r, 10, &ev));
+      r->parts = 1;
       HIP_TRY(launch_tail(sc, fa, cur->view(), r->fc.p, b, grid, r->lv.p, ac, (int)r->attr(kLdsStack),
                           use_nodes8(r, sc), r->stats.p, r->stream));
       HIP_TRY(timed_end(r, 10, ev));
@@ -1328,7 +1348,7 @@ int render_adaptive_frame(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa, co
                                   r->gnrm.p, r->gdif.p, r->sq.p, r->big_list.p, r->big_n.p, r->stream));
     HIP_TRY(timed_end(r, 8, ev));
   }
-  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, fa.nframes, fa.eye_depth, r->stream));
+  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, fa.nframes, fa.eye_depth, r->parts, r->stream));
   return CPT_OK;
 }
 
@@ -1405,6 +1425,7 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
     ac.tend = r->tend.p;
   }
   if (mega) {
+    r->parts = 1;
     r->extend_launches++;
     HIP_TRY(timed_begin(r, 0, &ev));
     HIP_TRY(launch_mega(sc, fa, r->fc.p, r->lv.p, ac, (int)r->attr(kLdsStack), r->attr(kNodeFormat) != 0,
@@ -1415,7 +1436,7 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
     if (rc) return rc;
   }
   if (regen) {                                     // the restarts, as a second wavefront
-    HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, fa.nframes, fa.eye_depth, r->stream));
+    HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, fa.nframes, fa.eye_depth, r->parts, r->stream));
     HIP_TRY(timed_begin(r, 7, &ev));
     HIP_TRY(launch_regen(fa, r->A.view(), ac, r->fc.p, r->stream));
     HIP_TRY(timed_end(r, 7, ev));
@@ -1427,7 +1448,7 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
   HIP_TRY(timed_begin(r, 8, &ev));
   HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, pt ? 1 : 0, r->stream));
   HIP_TRY(timed_end(r, 8, ev));
-  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, regen ? 0u : fa.nframes, fa.eye_depth, r->stream));
+  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, regen ? 0u : fa.nframes, fa.eye_depth, r->parts, r->stream));
   return CPT_OK;
 }
 
@@ -1729,7 +1750,7 @@ int cpt_renderer_stats(cpt_renderer* r, cpt_stats* out, int reset) {
   if (!r->allocated) return CPT_OK;
   HIP_TRY(hipStreamSynchronize(r->stream));
   DevStats h;
-  HIP_TRY(hipMemcpy(&h, r->stats.p, sizeof h, hipMemcpyDeviceToHost));
+  HIP_TRY(read_stats(r->stats.p, h));
   for (auto& e : r->events) {
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, e.a, e.b));
@@ -1764,7 +1785,7 @@ int cpt_renderer_stats(cpt_renderer* r, cpt_stats* out, int reset) {
   out->tail_tris = h.tail_tris;
   out->tail_ms = r->ms[10];
   if (reset) {
-    HIP_TRY(hipMemset(r->stats.p, 0, sizeof(DevStats)));
+    HIP_TRY(hipMemset(r->stats.p, 0, sizeof(DevStats) * kStatSlots));
     for (double& m : r->ms) m = 0;
     r->extend_launches = 0;
   }
@@ -2114,7 +2135,7 @@ int batch_enqueue(cpt_batch* b, cpt_scene* s, u32 k) {
   int rc = bounce_loop(r, sc, fa, n, ac, true);
   if (rc) return rc;
   HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, 0, r->stream));
-  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, k, fa.eye_depth, r->stream));
+  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, k, fa.eye_depth, r->parts, r->stream));
   HIP_TRY(launch_frame_advance(b->frame_dev.p, k, r->stream));
   return CPT_OK;
 }
@@ -2479,7 +2500,7 @@ int cpt_batch_autotune(cpt_batch* b, cpt_scene* s, uint32_t iterations, cpt_batc
   b->ms = 0.0;
   b->cfg = best_cfg;
   batch_apply_config(b);
-  HIP_TRY(hipMemset(b->r->stats.p, 0, sizeof(DevStats)));
+  HIP_TRY(hipMemset(b->r->stats.p, 0, sizeof(DevStats) * kStatSlots));
   if (best) *best = best_cfg;
   return CPT_OK;
 }

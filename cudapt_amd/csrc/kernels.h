@@ -122,15 +122,23 @@ struct LightJobs {
 };
 
 // Device counters of one frame (zeroed by frame_begin).
+constexpr uint32_t kPartSlots = 64;
 struct FrameCounters {
   uint32_t active[16];            // live paths entering bounce b
   uint32_t shadow[16];            // shadow rays emitted at bounce b
   uint32_t light_n[kLightSlots];  // light-vertex cache size per slot
-  uint32_t pad[16];
+  // counts of the kernels that carry whole paths (active, then shadow), spread
+  // over kPartSlots as the statistics are; frame_end adds them in and clears them
+  uint32_t part[kPartSlots][32];
 };
 
-// Cumulative device statistics.
-struct DevStats {
+// Cumulative device statistics, kStatSlots copies of them: each wave adds to the
+// copy of its workgroup (stat_slot) and the host sums them.  Atomics on one
+// address are served one after the other, about 12 ns each at a launch's end: with
+// one copy, the 15,626 waves of 1,000,003 occlusion rays took 471 us on the
+// heightfield, with these 255; a frame of 480,000 paths 1460 -> 1210 us.
+constexpr uint32_t kStatSlots = 256;
+struct alignas(128) DevStats {
   unsigned long long ext_rays, shadow_rays, eye_paths, frames;
   unsigned long long ext_nodes, ext_tris;
   unsigned long long sh_nodes, sh_tris;
@@ -290,7 +298,9 @@ hipError_t launch_scan_counts(const uint32_t* counts, uint32_t n, uint32_t* offs
                               uint32_t* total, hipStream_t st);
 hipError_t launch_shadow(const DevScene& sc, ShadowBuf sb, PathBuf nxt, const FrameCounters* fc, int bounce,
                          uint32_t max_n, int lds_stack, int quant, DevStats* stats, hipStream_t st);
-hipError_t launch_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, hipStream_t st);
+// parts: add FrameCounters::part in (a tail or a megakernel ran).
+hipError_t launch_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, int parts,
+                            hipStream_t st);
 // Closest hit (shadow = 0: hits into out) or connection visibility (shadow = 1:
 // contributions into nxt) of the `*count` rays by a persistent grid whose
 // lanes refill themselves with the next ray from the global counter `queue`.

@@ -769,6 +769,7 @@ hipError_t launch_bvh_depth(const DevScene& sc, const float4* rays, uint32_t n, 
   return hipGetLastError();
 }
 
+__device__ __forceinline__ DevStats* stat_slot(DevStats* stats) { return stats + blockIdx.x % kStatSlots; }
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -829,6 +830,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace(DevScene sc, const float
     }
   }
   if (stats) {
+    stats = stat_slot(stats);
     uint32_t sn = wave_sum(nn), st = wave_sum(nt);
     if ((threadIdx.x & 63) == 0 && (sn | st)) {
       atomicAdd(&stats->ext_nodes, (unsigned long long)sn);
@@ -1138,7 +1140,21 @@ hipError_t launch_frame_begin_dev(FrameCounters* fc, const uint32_t* total, uint
   return hipGetLastError();
 }
 
-__global__ void k_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth) {
+__global__ void k_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, int parts) {
+  if (parts) {                                      // 32 counters, two threads each
+    const uint32_t c = threadIdx.x & 31u, half = threadIdx.x >> 5;
+    uint32_t v = 0;
+#pragma unroll 8
+    for (uint32_t s = half; s < kPartSlots; s += 2) {
+      v += fc->part[s][c];
+      fc->part[s][c] = 0u;
+    }
+    v += __shfl_xor(v, 32, 64);
+    if (half == 0) {
+      if (c < 16) fc->active[c] += v; else fc->shadow[c - 16] += v;
+    }
+    __syncthreads();
+  }
   if (threadIdx.x == 0) {
     unsigned long long e = 0, s = 0;
     for (uint32_t b = 0; b < depth && b < 16; b++) { e += fc->active[b]; s += fc->shadow[b]; }
@@ -1148,8 +1164,9 @@ __global__ void k_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes
     stats->frames += nframes;
   }
 }
-hipError_t launch_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, hipStream_t st) {
-  k_frame_end<<<1, 64, 0, st>>>(fc, stats, nframes, depth);
+hipError_t launch_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, int parts,
+                            hipStream_t st) {
+  k_frame_end<<<1, 64, 0, st>>>(fc, stats, nframes, depth, parts);
   return hipGetLastError();
 }
 __global__ void k_frame_advance(uint32_t* frame_dev, uint32_t k) {
@@ -1544,6 +1561,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_extend_persist(DevScene sc, co
     }
   }
   if (stats) {
+    stats = stat_slot(stats);
     uint32_t sn = wave_sum(nn), st = wave_sum(nt);
     if ((threadIdx.x & 63) == 0 && (sn | st)) {
       atomicAdd(&stats->ext_nodes, (unsigned long long)sn);
@@ -1703,6 +1721,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
     }
   }
   if (stats) {
+    stats = stat_slot(stats);
     uint32_t sn = wave_sum(nn), st = wave_sum(nt);
     const uint32_t ss = *spill;         // the wave's own word, after its last atomic
     if (lane == 0 && (sn | st)) {
@@ -2281,6 +2300,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_shadow(DevScene sc, ShadowBuf 
     }
   }
   if (stats) {
+    stats = stat_slot(stats);
     uint32_t sn = wave_sum(nn), st = wave_sum(nt);
     if ((threadIdx.x & 63) == 0 && (sn | st)) {
       atomicAdd(&stats->sh_nodes, (unsigned long long)sn);
@@ -2623,6 +2643,7 @@ __global__ __launch_bounds__(kBlock) void k_regen_eye(DevScene sc, FrameArgs fa,
     }
   }
   if (stats) {
+    stats = stat_slot(stats);
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&stats->frames, 1ull);
     const uint32_t a0 = wave_sum(ext), a1 = wave_sum(shr), a2 = wave_sum(paths);
     const uint32_t b0 = wave_sum(en), b1 = wave_sum(et), b2 = wave_sum(sn), b3 = wave_sum(stc);
@@ -2716,9 +2737,11 @@ __device__ __forceinline__ void carry_flush(FrameCounters* fc, DevStats* stats, 
                                             uint32_t sn, uint32_t st, uint32_t nr = 0) {
   if (threadIdx.x < depth) {
     const uint32_t b = threadIdx.x;
-    if (b + 1 < 16 && n_live[b]) atomicAdd(&fc->active[b + 1], n_live[b]);
-    if (n_shadow[b]) atomicAdd(&fc->shadow[b], n_shadow[b]);
+    uint32_t* part = fc->part[blockIdx.x % kPartSlots];
+    if (b + 1 < 16 && n_live[b]) atomicAdd(&part[b + 1], n_live[b]);
+    if (n_shadow[b]) atomicAdd(&part[16 + b], n_shadow[b]);
   }
+  if (stats) stats = stat_slot(stats);
   if (stats && TAIL) {
     const uint32_t a0 = wave_sum(en + sn), a1 = wave_sum(et + st), a2 = wave_sum(nr);
     if ((threadIdx.x & 63) == 0 && (a0 | a1 | a2)) {
