@@ -67,6 +67,13 @@ struct DevArray {
 
 }  // namespace
 
+// Host rays up to which a query skips the two copies: its kernel reads the rays
+// and writes the hits over the bus, sooner than the copies are set up (Cornell
+// box, 1,021 / 8,192 / 32,768 rays: 27 / 37 / 84 us against 50 / 58 / 106;
+// heightfield 65 / 86 / 129 against 81 / 102 / 159).  The bound keeps the pinned
+// staging at 1.5 MB a scene.
+constexpr u32 kStageRays = 32768;
+
 struct cpt_scene {
   std::vector<float> pos, nrm, uv;
   std::vector<float4> tex;              // RTScene::m_pTextures' texels (RGBA), concatenated
@@ -93,8 +100,11 @@ struct cpt_scene {
   DevArray<DevMaterial> d_mats;
   DevArray<u32> d_light;
   DevArray<float4> d_rays, d_hits;
+  // staging of small host queries (cpt_trace_closest): kStageRays rays, then as
+  // many hits, in pinned memory that the kernel reads and writes in place
+  float4* stage = nullptr;
   DevArray<DevStats> d_stats;
-  u32 n_light = 0;
+  u32 n_light = 0, cus = 256;
   DevScene dev() const {
     DevScene s;
     s.nodes4 = d_nodes4.p;
@@ -122,6 +132,7 @@ struct cpt_scene {
     return s;
   }
   ~cpt_scene() {
+    if (stage) (void)hipHostFree(stage);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -492,6 +503,10 @@ int cpt_scene_upload(cpt_scene* s) {
   HIP_TRY(s->d_boff.upload(boff.data(), boff.size(), s->stream));
   rc = upload_materials(s);
   if (rc) return rc;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+    s->cus = (u32)cus;
   if (!s->d_stats.p) {
     HIP_TRY(s->d_stats.alloc(kStatSlots));
     HIP_TRY(hipMemsetAsync(s->d_stats.p, 0, sizeof(DevStats) * kStatSlots, s->stream));
@@ -515,8 +530,11 @@ int cpt_trace_closest_device(cpt_scene* s, const cpt_ray* d_rays, uint32_t n, ui
   if (!s->uploaded) return fail(CPT_E_STATE, "cpt_trace_closest_device: scene not uploaded");
   if (layout > 2) return fail(CPT_E_ARG, "cpt_trace_closest_device: layout %u not 0, 1 or 2", layout);
   hipStream_t st = stream ? (hipStream_t)stream : s->stream;
-  HIP_TRY(launch_trace(s->dev(), (const float4*)d_rays, n, nullptr, cull, (float4*)d_hits, 1, 0, layout,
-                       s->d_stats.p, st));
+  if (layout == 1)
+    HIP_TRY(launch_trace(s->dev(), (const float4*)d_rays, n, nullptr, cull, (float4*)d_hits, 1, 0, layout,
+                         s->d_stats.p, st));
+  else
+    HIP_TRY(launch_trace_rays(s->dev(), (const float4*)d_rays, n, cull, (float4*)d_hits, 0, s->d_stats.p, s->cus, st));
   if (!stream) HIP_TRY(hipStreamSynchronize(st));
   return CPT_OK;
 }
@@ -526,8 +544,8 @@ int cpt_trace_occluded_device(cpt_scene* s, const cpt_ray* d_rays, uint32_t n, u
   if (!s || (n && (!d_rays || !d_occluded))) return fail(CPT_E_ARG, "cpt_trace_occluded_device: null argument");
   if (!s->uploaded) return fail(CPT_E_STATE, "cpt_trace_occluded_device: scene not uploaded");
   hipStream_t st = stream ? (hipStream_t)stream : s->stream;
-  HIP_TRY(launch_trace(s->dev(), (const float4*)d_rays, n, nullptr, cull, (float4*)d_occluded, 0, 1, 0, s->d_stats.p,
-                       st));
+  HIP_TRY(launch_trace_rays(s->dev(), (const float4*)d_rays, n, cull, (float4*)d_occluded, 1, s->d_stats.p, s->cus,
+                            st));
   if (!stream) HIP_TRY(hipStreamSynchronize(st));
   return CPT_OK;
 }
@@ -536,10 +554,20 @@ int cpt_trace_closest(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cu
   if (!s || (n && (!rays || !hits))) return fail(CPT_E_ARG, "cpt_trace_closest: null argument");
   if (!s->uploaded) return fail(CPT_E_STATE, "cpt_trace_closest: scene not uploaded");
   if (n == 0) return CPT_OK;
+  if (n <= kStageRays) {
+    if (!s->stage)
+      HIP_TRY(hipHostMalloc((void**)&s->stage, (sizeof(cpt_ray) + sizeof(cpt_hit)) * kStageRays, hipHostMallocDefault));
+    float4* hit = s->stage + 2 * (size_t)kStageRays;
+    std::memcpy(s->stage, rays, sizeof(cpt_ray) * n);
+    HIP_TRY(launch_trace_rays(s->dev(), s->stage, n, cull, hit, 0, s->d_stats.p, s->cus, s->stream));
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    std::memcpy(hits, hit, sizeof(cpt_hit) * n);
+    return CPT_OK;
+  }
   HIP_TRY(s->d_rays.alloc((size_t)n * 2));
   HIP_TRY(s->d_hits.alloc(n));
   HIP_TRY(hipMemcpyAsync(s->d_rays.p, rays, sizeof(cpt_ray) * n, hipMemcpyHostToDevice, s->stream));
-  HIP_TRY(launch_trace(s->dev(), s->d_rays.p, n, nullptr, cull, s->d_hits.p, 1, 0, 0, s->d_stats.p, s->stream));
+  HIP_TRY(launch_trace_rays(s->dev(), s->d_rays.p, n, cull, s->d_hits.p, 0, s->d_stats.p, s->cus, s->stream));
   HIP_TRY(hipMemcpyAsync(hits, s->d_hits.p, sizeof(cpt_hit) * n, hipMemcpyDeviceToHost, s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   return CPT_OK;

@@ -153,6 +153,10 @@ constexpr int kBlock = 256;
 // ---- launches -------------------------------------------------------------
 hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, const uint32_t* count, uint32_t cull,
                         float4* hits_out, int out_orig, int any_hit, uint32_t layout, DevStats* stats, hipStream_t st, int cost = 0);
+// The trace entry points' rays (cpt_ray records, hits by original triangle id or
+// occlusion flags) over the 8-wide nodes.
+hipError_t launch_trace_rays(const DevScene& sc, const float4* rays, uint32_t n, uint32_t cull, float4* out, int any,
+                             DevStats* stats, uint32_t cus, hipStream_t st);
 hipError_t launch_frame_begin(FrameCounters* fc, uint32_t n_paths, hipStream_t st);
 hipError_t launch_light_pass(const DevScene& sc, const FrameArgs& fa, const LightJobs& jobs, LightVert* lv,
                              FrameCounters* fc, int quant, hipStream_t st);

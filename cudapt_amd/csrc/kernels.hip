@@ -1615,11 +1615,12 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
                                                             const float4* __restrict__ contrib, PathBuf nxt,
                                                             DevStats* __restrict__ stats, uint32_t refill,
                                                             FrameArgs fa) {
-  constexpr bool ANY = OUT == 3;
+  constexpr bool API = OUT == 0 || OUT == 2;        // fa.width rays as cpt_ray records, fa.flags: back-face test
+  constexpr bool ANY = OUT == 2 || OUT == 3;
   constexpr int S8 = kStk8<STK>;
   __shared__ TravLds<STK, Q> lds;
   uint64_t pstk[Q ? kPriv8<S8> : CPT_STACK_TOTAL - STK];
-  const uint32_t count = *countp;
+  const uint32_t count = API ? fa.width : *countp;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint64_t below = (1ull << lane) - 1ull;
@@ -1629,11 +1630,14 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
   // atomic is issued (every wave's atomic on the one counter would cost more
   // than a small launch's traversal); otherwise every chunk comes from the
   // counter, in the order waves ask.
-  const bool fixed = (uint64_t)count <= (uint64_t)waves * chunk;
+  // Queries of the trace entry points have no counter (calls on several streams
+  // would share it): wave w takes chunks w, w + waves, ...
+  const bool fixed = !API && (uint64_t)count <= (uint64_t)waves * chunk;
   const uint32_t wave = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  const uint64_t first = fixed ? (uint64_t)wave * chunk : (uint64_t)count;
+  const uint64_t first = fixed || API ? (uint64_t)wave * chunk : (uint64_t)count;
   uint32_t cnext = (uint32_t)min<uint64_t>(first, count);   // the wave's chunk (uniform across the wave)
   uint32_t cend = (uint32_t)min<uint64_t>(first + chunk, count);
+  uint32_t base = cnext;                   // where the chunk began (uniform)
   bool exhausted = false;                  // uniform
   bool active = false;
   bool pending = false;                    // finished, result not yet written
@@ -1663,6 +1667,10 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
         r.z = hit ? h.u : 0.f;
         r.w = hit ? h.v : 0.f;
         out[ray] = r;
+      } else if (OUT == 0) {
+        out[ray] = make_float4(__uint_as_float(h.orig), h.t, h.u, h.v);
+      } else if (OUT == 2) {
+        ((uint32_t*)out)[ray] = hit ? 1u : 0u;
       } else if (!hit) {
         const float4 c = contrib[ray];
         const uint32_t bits = __float_as_uint(c.w), slot = bits & ~kShadowNoCount;
@@ -1680,11 +1688,16 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
       while (given < n_idle) {
         if (cnext >= cend) {
           if (fixed) { exhausted = true; break; }
-          uint32_t q = 0;
-          if (lane == 0) q = atomicAdd(queue, chunk);
-          const uint64_t b = __shfl(q, 0, 64);
+          uint64_t b;
+          if (API) {
+            b = (uint64_t)base + (uint64_t)waves * chunk;
+          } else {
+            uint32_t q = 0;
+            if (lane == 0) q = atomicAdd(queue, chunk);
+            b = __shfl(q, 0, 64);
+          }
           if (b >= count) { exhausted = true; break; }
-          cnext = (uint32_t)b;
+          base = cnext = (uint32_t)b;
           cend = (uint32_t)min<uint64_t>(b + chunk, count);
         }
         const uint32_t take = min(n_idle - given, cend - cnext);
@@ -1696,6 +1709,9 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
             const PathState e = eye_slot(fa, ray, dk);
             a = e.ro;
             b4 = e.rd;
+          } else if (API) {
+            a = ro[2 * (size_t)ray];
+            b4 = ro[2 * (size_t)ray + 1];
           } else {
             a = ro[ray];
             b4 = rd[ray];
@@ -1712,7 +1728,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
     if (__ballot(active) == 0ull) break;
     if constexpr (Q) {
       const bool was = active;
-      ray8_step<ANY, S8>(sc, R, active, false, lds.w[wid], (LdsU64*)&lds.w[wid].stk[0][lane], pstk, lane, nn, nt,
+      ray8_step<ANY, S8>(sc, R, active, API && fa.flags, lds.w[wid], (LdsU64*)&lds.w[wid].stk[0][lane], pstk, lane, nn, nt,
                          spill);
       if (was && !active) pending = true;
     } else if (active && ray_step<ANY, STK>(sc, R, false, lds_column(lds.stk), pstk, nn, nt, spill)) {
@@ -1761,6 +1777,34 @@ hipError_t launch_trace_dyn(const DevScene& sc, const float4* ro, const float4* 
 #undef CPT_DYN_1F
 #undef CPT_DYN_1E
 #undef CPT_DYN
+  return hipGetLastError();
+}
+
+// Rays of the trace entry points: the persistent grid's workgroups (six a compute
+// unit are resident: more would start after the first have drained; 3, 4, 5, 6
+// and 8 take 415, 365, 339, 335 and 403 us for 2,097,143 closest-hit rays on the
+// heightfield), lanes refilled once 16 are idle (64, 48, 32, 16: 457, 347, 335,
+// 328 us there; 327, 278, 281, 266 on the sphere grid).  Up to one chunk of 64
+// rays a wave the grid is no larger than the rays and nothing is refilled.
+// One thread per ray over 128-byte 4-wide nodes took 920 us on the sphere grid,
+// and 1,000,003 occlusion rays on the heightfield 255.
+constexpr uint32_t kTraceGroups = 6, kTraceRefill = 16;
+hipError_t launch_trace_rays(const DevScene& sc, const float4* rays, uint32_t n, uint32_t cull, float4* out, int any,
+                             DevStats* stats, uint32_t cus, hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  if (!sc.nodes8) return launch_trace(sc, rays, n, nullptr, cull, out, any ? 0 : 1, any, 0, stats, st);
+  if (!rays || !out || !sc.tris8 || cus == 0) return hipErrorInvalidValue;
+  FrameArgs fa = {};
+  fa.width = n;
+  fa.flags = cull ? 1u : 0u;
+  const uint32_t blocks = (n + kBlock - 1) / kBlock;
+  const uint32_t grid = blocks < kTraceGroups * cus ? blocks : kTraceGroups * cus;
+  if (any)
+    k_trace_dyn<2, 8, 6, true><<<grid, kBlock, 0, st>>>(sc, rays, nullptr, nullptr, nullptr, out, nullptr, PathBuf{},
+                                                        stats, kTraceRefill, fa);
+  else
+    k_trace_dyn<0, 8, 6, true><<<grid, kBlock, 0, st>>>(sc, rays, nullptr, nullptr, nullptr, out, nullptr, PathBuf{},
+                                                        stats, kTraceRefill, fa);
   return hipGetLastError();
 }
 

@@ -146,9 +146,9 @@ int cpt_scene_destroy(cpt_scene* s);
 int cpt_trace_closest(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cull, cpt_hit* hits);
 
 /* Same over device arrays already resident in HBM, launched on `stream`
- * (a hipStream_t, NULL = the scene's stream).  layout 0 = 4-wide nodes,
- * 1 = the reference's binary CompactBVH layout, 2 = 8-wide nodes with quantized
- * boxes (the same hits: culling stays conservative). */
+ * (a hipStream_t, NULL = the scene's stream).  layout 0 and 2 = the device tree
+ * (8-wide nodes with quantized boxes, whose culling stays conservative),
+ * 1 = the reference's binary CompactBVH layout.  The hits are the same. */
 int cpt_trace_closest_device(cpt_scene* s, const cpt_ray* d_rays, uint32_t n, uint32_t cull, cpt_hit* d_hits,
                              void* stream, uint32_t layout);
 
@@ -190,8 +190,8 @@ int cpt_filter_cross_bilateral_device_noalloc(const float* d_color, const float*
 /* Traversal cost per ray, the counterpart of the reference's BVH debug
  * renderer (TraceCost / TraceDepth, src/cudaRTCommon.cu:129-273;
  * src/cudaRTBVHDebug.cu): cost2[2i] = nodes visited, cost2[2i+1] = triangles
- * tested by ray i's closest-hit traversal in `layout` (as for
- * cpt_trace_closest_device).  Host arrays. */
+ * tested by ray i's closest-hit traversal in `layout` (0: FP32 4-wide nodes, 1
+ * and 2 as for cpt_trace_closest_device).  Host arrays. */
 int cpt_trace_cost(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cull, uint32_t layout, uint32_t* cost2);
 
 /* The BVH debug renderer's depth queries (src/cudaRTBVHDebug.cu modes

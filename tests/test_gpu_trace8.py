@@ -62,3 +62,13 @@ def test_max_distance(cpt, scene):
                                                      np.float32(1e20)])
     ref, _ = O.trace(rays, "brute")
     assert hits_equal(_hits(cpt, S, rays), ref).all()
+
+
+@pytest.mark.parametrize("n", [1, 32768, 32769, 500000])
+def test_host_queries(cpt, n):
+    """Both sides of the pinned staging's bound, and more rays than the persistent grid's lanes."""
+    sc = scenes.cornell()
+    S, O = cpt.Scene(sc), oracle.Scene(sc)
+    rays = random_rays(n, [-0.99, 0.01, -0.99], [0.99, 1.99, 0.99], seed=n)
+    ref, _ = O.trace(rays, "brute")
+    assert hits_equal(S.trace(rays), ref).all()
