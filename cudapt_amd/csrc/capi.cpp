@@ -865,7 +865,7 @@ struct cpt_renderer {
   u32 gauss_radius = 0;
   u32 persist_chunk = 0, persist_grid = 0;   // persistent extend grid (0: one thread per ray)
   int cus = 0;                               // compute units of the device
-  DevArray<u32> queue;                       // its global work-queue counter
+  DevArray<u32> queue;                       // work counters of the refilling launches, then k_extend_persist's
   cpt_mlp* mlp = nullptr;              // learned error model (adaptive mode)
   DevArray<float> mlp_x, mlp_y, mlp_e, sq_f, sq_e;
   u32 cap = 0;
@@ -934,7 +934,7 @@ int renderer_alloc(cpt_renderer* r) {
     HIP_TRY(r->term_rng.alloc(cap));
     HIP_TRY(r->tend.alloc(kMaxInFlight));
   }
-  HIP_TRY(r->queue.alloc(2));
+  HIP_TRY(r->queue.alloc((size_t)kQueues * kDealers * kDealStride + 1));
   HIP_TRY(r->fc.alloc(1));
   HIP_TRY(r->stats.alloc(kStatSlots));
   HIP_TRY(r->result.alloc(n * 3));
@@ -1041,7 +1041,7 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
   // overlap bounce b + 1's extension rays (which read only ray origins and
   // directions; the shadow kernel writes only accumulators); shading of bounce
   // b + 1, which reads those accumulators and rewrites the shadow queue, waits
-  // for it.  The two refilling grids take their rays from separate counters.
+  // for it.  Every refilling launch has counters of its own.
   const bool ov = r->overlap_shadow;
   if (ov) {
     if (!r->side) HIP_TRY(hipStreamCreateWithFlags(&r->side, hipStreamNonBlocking));
@@ -1052,6 +1052,10 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
   const bool eye0 =
       gen_eye && big && r->attr(kRefill) >= 1.0 && use_nodes8(r, sc) && fa.n_views == 0;
   if (gen_eye && !eye0) HIP_TRY(launch_gen_eye(fa, r->A.view(), r->stream));
+  const auto queue = [r](u32 kind, u32 b) { return r->queue.p + (size_t)(kind * 16 + b) * kDealers * kDealStride; };
+  const uint32_t cus = r->cus > 0 ? (uint32_t)r->cus : 256u;
+  const uint32_t groups = (uint32_t)std::min(32.0, std::max(1.0, r->attr(kRefillGroups)));
+  if (big) HIP_TRY(launch_queues_clear(r->queue.p, r->stream));
   bool shadow_pending = false;
   // "Tail Bounce" t > 0: bounces t.. run as one k_tail launch (plain BDPT's
   // frames and the adaptive frames after the warm-up, whose accumulation goes
@@ -1072,11 +1076,9 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
         HIP_TRY(hipStreamWaitEvent(r->stream, r->ev_light, 0));
         r->light_pending = false;
       }
-      const uint32_t grid =
-          (uint32_t)(r->cus > 0 ? r->cus : 256) * (uint32_t)std::min(32.0, std::max(1.0, r->attr(kRefillGroups)));
       HIP_TRY(timed_begin(r, 10, &ev));
       r->parts = 1;
-      HIP_TRY(launch_tail(sc, fa, cur->view(), r->fc.p, b, grid, r->lv.p, ac, (int)r->attr(kLdsStack),
+      HIP_TRY(launch_tail(sc, fa, cur->view(), r->fc.p, b, groups * cus, r->lv.p, ac, (int)r->attr(kLdsStack),
                           use_nodes8(r, sc), r->stats.p, r->stream));
       HIP_TRY(timed_end(r, 10, ev));
       break;
@@ -1086,15 +1088,14 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
     const int quant = use_nodes8(r, sc);
     const uint32_t refill =
         big ? (uint32_t)std::min(64.0, std::max(0.0, r->attr(b == 0 ? kRefill : kRefillSecondary))) : 0u;
-    const uint32_t dyn_grid =
-        (uint32_t)(r->cus > 0 ? r->cus : 256) * (uint32_t)std::min(32.0, std::max(1.0, r->attr(kRefillGroups)));
     if (refill)
       HIP_TRY(launch_trace_dyn(sc, cur->view().ray_o, cur->view().ray_d, r->fc.p->active + b, r->hits.p, nullptr,
-                               PathBuf{}, r->stats.p, (int)r->attr(kLdsStack), quant, 0, dyn_grid, refill, r->queue.p,
+                               PathBuf{}, r->stats.p, (int)r->attr(kLdsStack), quant, 0, groups, cus, refill, queue(0, b),
                                r->stream, eye0 && b == 0 ? &fa : nullptr));
     else if (r->persist_chunk)
       HIP_TRY(launch_extend_persist(sc, cur->view(), r->fc.p, (int)b, r->hits.p, r->stats.p, (int)r->attr(kLdsStack),
-                                    quant, r->persist_chunk, r->persist_grid, r->queue.p, r->stream));
+                                    quant, r->persist_chunk, r->persist_grid,
+                                    queue(kQueues / 16, 0), r->stream));
     else
       HIP_TRY(launch_extend(sc, cur->view(), r->fc.p, (int)b, max_n, r->hits.p, r->stats.p, (int)r->attr(kLdsStack),
                             quant, r->stream));
@@ -1122,8 +1123,8 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
       HIP_TRY(timed_begin(r, 1, &ev, sst));
       if (refill_sh)
         HIP_TRY(launch_trace_dyn(sc, sb.ray_o, sb.ray_d, r->fc.p->shadow + b, nullptr, sb.contrib, nxt->view(),
-                                 r->stats.p, (int)r->attr(kLdsStackShadow), quant, 1, dyn_grid, refill_sh,
-                                 r->queue.p + (ov ? 1 : 0), sst));
+                                 r->stats.p, (int)r->attr(kLdsStackShadow), quant, 1, groups, cus, refill_sh,
+                                 queue(1, b), sst));
       else
         HIP_TRY(launch_shadow(sc, sb, nxt->view(), r->fc.p, (int)b, max_n, (int)r->attr(kLdsStackShadow), quant,
                               r->stats.p, sst));
@@ -2190,7 +2191,7 @@ int batch_prepare(cpt_batch* b, cpt_scene* s) {
   }
   int rc = lv_alloc(r);
   if (rc) return rc;
-  HIP_TRY(r->queue.alloc(2));
+  HIP_TRY(r->queue.alloc((size_t)kQueues * kDealers * kDealStride + 1));
   if (b->buf_key != (const void*)r->A.ray_o.p) {   // buffers moved: a captured graph points at the old ones
     b->drop_graph();
     b->buf_key = (const void*)r->A.ray_o.p;

@@ -147,6 +147,11 @@ struct alignas(128) DevStats {
 };
 
 constexpr int kMaxDepth = 15;
+// Work counters of the refilling launches: kDealers a launch, a cache line each,
+// for the extension and the shadow rays of each of 16 bounces.
+constexpr uint32_t kDealers = 8, kDealStride = 32, kQueues = 32;
+// Rays a wave takes at once: at most, and where a launch has less than one ray a lane.
+constexpr uint32_t kDealMax = 1024, kDealLow = 16;
 constexpr int kMaxFilterRadius = 31;   // GAUSSIANCOST_N = 64 entries (include/cudaBilateralFilter.h:3)
 constexpr int kBlock = 256;
 
@@ -305,14 +310,17 @@ hipError_t launch_shadow(const DevScene& sc, ShadowBuf sb, PathBuf nxt, const Fr
 // parts: add FrameCounters::part in (a tail or a megakernel ran).
 hipError_t launch_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, int parts,
                             hipStream_t st);
+hipError_t launch_queues_clear(uint32_t* queue, hipStream_t st);   // all kQueues launches' counters
 // Closest hit (shadow = 0: hits into out) or connection visibility (shadow = 1:
 // contributions into nxt) of the `*count` rays by a persistent grid whose
-// lanes refill themselves with the next ray from the global counter `queue`.
+// lanes refill themselves, their rays dealt through the launch's own kDealers
+// counters at `queue` (kDealStride words apart, zero before).  At most `groups`
+// workgroups on each of `cus` compute units.
 // eye (closest hit over quantized nodes only): ray i is the eye ray of path
 // slot i of the batch `*eye` describes, computed in place of reading ro / rd.
 hipError_t launch_trace_dyn(const DevScene& sc, const float4* ro, const float4* rd, const uint32_t* count,
                             float4* out, const float4* contrib, PathBuf nxt, DevStats* stats, int lds_stack,
-                            int quant, int shadow, uint32_t grid, uint32_t refill, uint32_t* queue,
+                            int quant, int shadow, uint32_t groups, uint32_t cus, uint32_t refill, uint32_t* queue,
                             hipStream_t st, const FrameArgs* eye = nullptr);
 // *frame_dev += k (the device frame counter of replayed graphs).
 hipError_t launch_frame_advance(uint32_t* frame_dev, uint32_t k, hipStream_t st);

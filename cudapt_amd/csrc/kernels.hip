@@ -1122,6 +1122,13 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v) { *p = v; }
 __global__ void k_fill_n_u32(uint32_t* p, uint32_t n, uint32_t v) {
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) p[i] = v;
 }
+__global__ void k_queues_clear(uint32_t* queue) {
+  queue[threadIdx.x * kDealStride] = 0u;
+}
+hipError_t launch_queues_clear(uint32_t* queue, hipStream_t st) {
+  k_queues_clear<<<1, kQueues * kDealers, 0, st>>>(queue);
+  return hipGetLastError();
+}
 __global__ void k_frame_begin(FrameCounters* fc, uint32_t n_paths) {
   uint32_t i = threadIdx.x;
   if (i < 16) { fc->active[i] = i == 0 ? n_paths : 0u; fc->shadow[i] = 0u; }
@@ -1591,19 +1598,100 @@ hipError_t launch_extend_persist(const DevScene& sc, PathBuf pb, const FrameCoun
   return hipGetLastError();
 }
 
+// The rays [0, count) of a launch dealt to the waves of a persistent grid.
+// Workgroups go to the chip's eight dies (each with its own L2) in turn, so the
+// rays are cut into kDealers contiguous shares, one a die: neighbouring rays, which meet
+// the same nodes, stay within one L2.  Of its die's share each wave first
+// takes a quarter of an even part with no atomic; further chunks come from the
+// share's counter, half an even part of what the wave knows to be left, so
+// that they shrink towards the end (64 rays at the least).  A wave whose share is
+// dealt out goes on with the next, whose counter it reads before adding to it (atomics on one
+// address are served one after the other).  Launches of up to 64 rays a wave
+// are dealt once, evenly over the waves (kDealLow rays at the least: fewer rays
+// a wave end sooner, 16 / 64 take 25.3 / 25.8 ms in the learned frames).
+// queue: kDealers counters, kDealStride words apart, zero when the launch starts.
+// One share instead of eight takes 28.1 ms in the learned frames against 26.0 and the
+// same elsewhere; one counter with chunks of 256 and no first chunk, as before, 30.5
+// there and 20.2 against 19.2 ms for a still of 64 1280 x 720 frames.
+struct Deal {
+  uint32_t share, len, start, fixed, waves;   // of the share being drawn from (all uniform across the wave)
+  uint32_t left;                              // shares left to visit, this one included
+  uint32_t known;                             // rays of the share known to be dealt
+};
+__device__ __forceinline__ uint32_t deal_clamp(uint32_t v) {
+  v &= ~63u;
+  return v < 64u ? 64u : v > kDealMax ? kDealMax : v;
+}
+__device__ __forceinline__ void deal_share(Deal& D, uint32_t share, uint32_t count) {
+  const uint32_t part = ((count - 1u) / kDealers / 64u + 1u) * 64u;      // count > 0
+  D.share = share;
+  D.start = min((uint64_t)share * part, (uint64_t)count);
+  D.len = min(part, count - D.start);
+  D.waves = gridDim.x > share ? (gridDim.x - share + kDealers - 1u) / kDealers * (kBlock / 64) : 0u;
+  D.fixed = deal_clamp(D.len / (4u * max(D.waves, 1u)));
+}
+__device__ __forceinline__ void deal_first(Deal& D, uint32_t count, uint32_t wave, uint32_t& at, uint32_t& end) {
+  D.left = count ? kDealers : 0u;
+  at = end = 0u;
+  if (!count) return;
+  const uint32_t waves = gridDim.x * (kBlock / 64), k = blockIdx.x * (kBlock / 64) + wave;
+  if (count <= waves * 64u) {
+    D.left = 0u;
+    const uint32_t per = min(64u, max(kDealLow, (count + waves - 1u) / waves));
+    if (k * per < count) {
+      at = k * per;
+      end = min(at + per, count);
+    }
+    return;
+  }
+  deal_share(D, blockIdx.x % kDealers, count);
+  const uint64_t off = (uint64_t)(blockIdx.x / kDealers * (kBlock / 64) + wave) * D.fixed;
+  D.known = D.waves * D.fixed;
+  if (off < D.len) {
+    at = D.start + (uint32_t)off;
+    end = D.start + min((uint32_t)off + D.fixed, D.len);
+  }
+}
+// The wave's next chunk; false when none is left.
+__device__ __forceinline__ bool deal_next(Deal& D, uint32_t count, uint32_t* __restrict__ queue, int lane, uint32_t& at,
+                                          uint32_t& end) {
+  while (D.left) {
+    const uint32_t given = D.waves * D.fixed;
+    uint32_t* ctr = queue + D.share * kDealStride;
+    if (given < D.len && D.known < D.len) {
+      const uint32_t step = deal_clamp((D.len - D.known) / (2u * max(D.waves, 1u)));
+      uint32_t q = 0;
+      if (lane == 0) q = atomicAdd(ctr, step);
+      q = __builtin_amdgcn_readfirstlane(q);
+      D.known = given + q;
+      if (D.known < D.len) {
+        at = D.start + D.known;
+        end = D.start + min(D.known + step, D.len);
+        return true;
+      }
+    }
+    if (--D.left == 0) break;
+    deal_share(D, (D.share + 1u) % kDealers, count);
+    const uint32_t g = D.waves * D.fixed;
+    uint32_t q = 0;
+    if (g < D.len) {
+      if (lane == 0) q = __hip_atomic_load(queue + D.share * kDealStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      q = __builtin_amdgcn_readfirstlane(q);
+    }
+    D.known = g + q;
+  }
+  return false;
+}
+
 // Dynamic refill: a persistent grid whose lanes each trace one ray at a time
-// and take the next as soon as theirs is finished.  A wave hands out ray
-// indices from a chunk it took from the global counter `queue` (one atomic per
-// chunk): kDynChunk rays when the launch has enough for every wave to take
-// several, else 64, so that a small batch still spreads over every wave; lanes
-// refill once at least `refill` (1..64) are idle.
+// and take the next as soon as theirs is finished; lanes refill once at least
+// `refill` (1..64) are idle, from a chunk of rays that the wave holds (Deal).
 // A finished lane writes its result at the wave's next refill point, together
 // with the other finished lanes, not in the traversal loop: the shadow
 // epilogue's read-modify-write would otherwise stall the whole wave on its load
 // every time one lane finishes.
 // OUT 1: closest hit (t, leaf, u, v) into out[ray]; OUT 3: the connection's
 // visibility (k_shadow's epilogue).
-constexpr uint32_t kDynChunk = 256;
 // EYE (closest hit, quantized nodes): ray i is the eye ray of path slot i of
 // the batch fa describes, computed in place of reading ro / rd.  A separate
 // instantiation, so that the plain kernels' code is not touched by it.
@@ -1624,20 +1712,18 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint64_t below = (1ull << lane) - 1ull;
+  // Queries of the trace entry points have no counters (calls on several streams
+  // would share them): wave w takes chunks of 64 w, w + waves, ...
   const uint32_t waves = gridDim.x * (kBlock / 64);
-  const uint32_t chunk = (uint64_t)count >= (uint64_t)kDynChunk * waves ? kDynChunk : 64u;
-  // When one chunk per wave covers the launch, wave w takes chunk w and no
-  // atomic is issued (every wave's atomic on the one counter would cost more
-  // than a small launch's traversal); otherwise every chunk comes from the
-  // counter, in the order waves ask.
-  // Queries of the trace entry points have no counter (calls on several streams
-  // would share it): wave w takes chunks w, w + waves, ...
-  const bool fixed = !API && (uint64_t)count <= (uint64_t)waves * chunk;
-  const uint32_t wave = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  const uint64_t first = fixed || API ? (uint64_t)wave * chunk : (uint64_t)count;
-  uint32_t cnext = (uint32_t)min<uint64_t>(first, count);   // the wave's chunk (uniform across the wave)
-  uint32_t cend = (uint32_t)min<uint64_t>(first + chunk, count);
-  uint32_t base = cnext;                   // where the chunk began (uniform)
+  uint32_t cnext, cend;                    // the wave's chunk (uniform across the wave)
+  uint32_t base = 0;                       // where it began (API)
+  Deal deal;
+  if constexpr (API) {
+    cnext = base = min((blockIdx.x * (kBlock / 64) + wid) * 64u, count);
+    cend = min(cnext + 64u, count);
+  } else {
+    deal_first(deal, count, wid, cnext, cend);
+  }
   bool exhausted = false;                  // uniform
   bool active = false;
   bool pending = false;                    // finished, result not yet written
@@ -1687,18 +1773,15 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
       uint32_t given = 0;
       while (given < n_idle) {
         if (cnext >= cend) {
-          if (fixed) { exhausted = true; break; }
-          uint64_t b;
-          if (API) {
-            b = (uint64_t)base + (uint64_t)waves * chunk;
-          } else {
-            uint32_t q = 0;
-            if (lane == 0) q = atomicAdd(queue, chunk);
-            b = __shfl(q, 0, 64);
+          if constexpr (API) {
+            const uint64_t b = (uint64_t)base + (uint64_t)waves * 64u;
+            if (b >= count) { exhausted = true; break; }
+            base = cnext = (uint32_t)b;
+            cend = (uint32_t)min<uint64_t>(b + 64u, count);
+          } else if (!deal_next(deal, count, queue, lane, cnext, cend)) {
+            exhausted = true;
+            break;
           }
-          if (b >= count) { exhausted = true; break; }
-          base = cnext = (uint32_t)b;
-          cend = (uint32_t)min<uint64_t>(b + chunk, count);
         }
         const uint32_t take = min(n_idle - given, cend - cnext);
         if (!active && rank >= given && rank < given + take) {
@@ -1747,18 +1830,33 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
     }
   }
 }
+// Workgroups of a kernel that a compute unit holds at once.  A persistent grid
+// is no larger: workgroups past it start only when others have ended, and would keep the
+// chunks they begin with until then (8 a compute unit asked for, 6 resident, 8 / 6
+// launched: 26.7 / 26.1 ms for the learned frames, 19.6 / 19.2 the 64-frame still).
+uint32_t resident_groups(const void* kernel) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kBlock, 0) != hipSuccess || n < 1) return 32;
+  return (uint32_t)n;
+}
 hipError_t launch_trace_dyn(const DevScene& sc, const float4* ro, const float4* rd, const uint32_t* count,
                             float4* out, const float4* contrib, PathBuf nxt, DevStats* stats, int lds_stack,
-                            int quant, int shadow, uint32_t grid, uint32_t refill, uint32_t* queue,
+                            int quant, int shadow, uint32_t groups, uint32_t cus, uint32_t refill, uint32_t* queue,
                             hipStream_t st, const FrameArgs* eye) {
-  if (!ro || !rd || !count || !queue || grid == 0 || refill < 1 || refill > 64 || !sc.tris ||
+  if (!ro || !rd || !count || !queue || groups == 0 || cus == 0 || refill < 1 || refill > 64 || !sc.tris ||
       !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
   if (shadow ? (!contrib || !pathbuf_ok(nxt) || eye) : !out) return hipErrorInvalidValue;
   const FrameArgs fa = eye ? *eye : FrameArgs{};
-  k_fill_u32<<<1, 1, 0, st>>>(queue, 0u);
-#define CPT_DYN(O, S, W, Qb) k_trace_dyn<O, S, W, Qb><<<grid, kBlock, 0, st>>>(sc, ro, rd, count, queue, out, contrib, nxt, stats, refill, fa)
-#define CPT_DYN_1E(S, W) k_trace_dyn<1, S, W, true, true><<<grid, kBlock, 0, st>>>(sc, ro, rd, count, queue, out, contrib, nxt, stats, refill, fa)
+#define CPT_DYN_E(O, S, W, Qb, Eb)                                                                              \
+  {                                                                                                             \
+    static const uint32_t resident = resident_groups((const void*)k_trace_dyn<O, S, W, Qb, Eb>);                \
+    const uint32_t grid = (groups < resident ? groups : resident) * cus;                                        \
+    k_trace_dyn<O, S, W, Qb, Eb><<<grid, kBlock, 0, st>>>(sc, ro, rd, count, queue, out, contrib, nxt, stats,   \
+                                                          refill, fa);                                          \
+  }
+#define CPT_DYN(O, S, W, Qb) CPT_DYN_E(O, S, W, Qb, false)
+#define CPT_DYN_1E(S, W) CPT_DYN_E(1, S, W, true, true)
 #define CPT_DYN_3Q(S, W) CPT_DYN(3, S, W, true)
 #define CPT_DYN_3F(S, W) CPT_DYN(3, S, W, false)
 #define CPT_DYN_1Q(S, W) CPT_DYN(1, S, W, true)
@@ -1777,6 +1875,7 @@ hipError_t launch_trace_dyn(const DevScene& sc, const float4* ro, const float4* 
 #undef CPT_DYN_1F
 #undef CPT_DYN_1E
 #undef CPT_DYN
+#undef CPT_DYN_E
   return hipGetLastError();
 }
 
