@@ -748,7 +748,8 @@ const char* const kRefillShadow = "Shadow Refill";
 const char* const kRefillGroups = "Refill Workgroups";
 // path capacity below which rays go one thread per ray whatever the refill
 // settings: a grid that can hold the whole launch gains nothing from refilling
-// (one frame of 800 x 600 per call: shadow 10 % faster one thread per ray)
+// (one frame of 800 x 600 per call: shadow 10 % faster one thread per ray), and
+// below which (twice it for plain frames) one thread carries each path through every bounce
 const char* const kRefillMinPaths = "Refill Min Paths";
 // allocation signal from the learned model's output y (log per-sample
 // variance): 0 = nd / (nd + N) * exp(y) / N, the filter-residual estimate's
@@ -1020,6 +1021,25 @@ int update_gauss(cpt_renderer* r, float sigma, u32 radius) {
   return CPT_OK;
 }
 
+// A launch too small to fill the chip bounce by bounce: each thread carries its
+// path through every bounce (k_mega, k_tail).  Phase times exist only where the
+// phases are launches of their own, so a profiled renderer keeps them.  The line
+// lies where both take the same time: at twice "Refill Min Paths" (2 M paths by
+// default) for plain frames - whole / by bounce, us: 800 x 600 on the sphere grid
+// 936 / 1228, 1280 x 720 1590 / 1831, 1920 x 1080 3229 / 3318, 8 frames of 800 x 600
+// 3377 / 3023 - and at once that for adaptive ones, whose paths crowd on the noisy
+// pixels: 10 bisected frames of 1280 x 720 there 15.0 / 16.2 ms, of 1920 x 1080
+// 28.6 / 26.7.
+bool whole_paths(const cpt_renderer* r, u32 n, double scale = 1.0) {
+  return !r->profiling && (double)n < scale * r->attr(kRefillMinPaths);
+}
+hipError_t trace_whole(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, const Accum& ac) {
+  r->parts = 1;
+  r->extend_launches++;
+  return launch_mega(sc, fa, r->fc.p, r->lv.p, ac, (int)r->attr(kLdsStack), use_nodes8(r, sc),
+                     r->cus > 0 ? (uint32_t)r->cus : 256u, r->stats.p, r->stream);
+}
+
 // gen_eye: the batch starts from fresh eye paths in r->A.  With refilling
 // waves at bounce 0, quantized nodes and one view nothing writes them: the first extension and
 // shading compute each slot's eye path where k_gen_eye would have stored it
@@ -1057,17 +1077,14 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
   const uint32_t groups = (uint32_t)std::min(32.0, std::max(1.0, r->attr(kRefillGroups)));
   if (big) HIP_TRY(launch_queues_clear(r->queue.p, r->stream));
   bool shadow_pending = false;
-  // "Tail Bounce" t > 0: bounces t.. run as one k_tail launch (plain BDPT's
-  // frames and the adaptive frames after the warm-up, whose accumulation goes
-  // through the sample records; the first-hit G-buffer is written at bounce 0,
-  // before any tail)
+  // "Tail Bounce" t > 0: bounces t.. run as one k_tail launch (BDPT's frames),
+  // and those before it too where the whole batch is a small launch
   const double tail_attr = r->attr(kTailBounce);
-  const u32 tail = tail_attr >= 1.0 && tail_attr < (double)fa.eye_depth && ac.apply == 2 &&
-                           !(ac.variant & (kVariantPT | kVariantDisney))
-                       ? (u32)tail_attr
-                       : 0u;
+  const bool tail = tail_attr >= 1.0 && tail_attr < (double)fa.eye_depth &&
+                    !(ac.variant & (kVariantPT | kVariantDisney));
+  const u32 tail0 = tail ? (u32)tail_attr : 0u, tail_from = whole_paths(r, max_n) ? 0u : tail0;
   for (u32 b = 0; b < fa.eye_depth; b++) {
-    if (tail && b == tail) {
+    if (tail && b == tail_from) {
       if (shadow_pending) {                      // the tail shades: bounce b - 1's occlusion results first
         HIP_TRY(hipStreamWaitEvent(r->stream, r->ev_shadow, 0));
         shadow_pending = false;
@@ -1078,7 +1095,7 @@ int bounce_loop(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, u32 ma
       }
       HIP_TRY(timed_begin(r, 10, &ev));
       r->parts = 1;
-      HIP_TRY(launch_tail(sc, fa, cur->view(), r->fc.p, b, groups * cus, r->lv.p, ac, (int)r->attr(kLdsStack),
+      HIP_TRY(launch_tail(sc, fa, cur->view(), r->fc.p, b, tail0, groups, cus, r->lv.p, ac, (int)r->attr(kLdsStack),
                           use_nodes8(r, sc), r->stats.p, r->stream));
       HIP_TRY(timed_end(r, 10, ev));
       break;
@@ -1299,9 +1316,13 @@ int render_adaptive_frame(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa, co
   if (fa.frame0 < warmup_frames(r)) {              // plain 1 spp frames with G-buffer (:1372-1406)
     ac.apply = 1;
     HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
-    HIP_TRY(launch_gen_eye_rec(fa, r->A.view(), ac.rec, r->stream));
-    int rc = bounce_loop(r, sc, fa, n, ac);
-    if (rc) return rc;
+    if (whole_paths(r, n)) {
+      HIP_TRY(trace_whole(r, sc, fa, ac));
+    } else {
+      HIP_TRY(launch_gen_eye_rec(fa, r->A.view(), ac.rec, r->stream));
+      int rc = bounce_loop(r, sc, fa, n, ac);
+      if (rc) return rc;
+    }
     HIP_TRY(launch_add_paths(r->paths.p, nullptr, n, fa.frame0 == 0, r->stream));
   } else {
     int rc = CPT_OK;
@@ -1418,7 +1439,8 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
   std::memset(&jobs, 0, sizeof jobs);
   // the path tracers have no light pass (the Disney mode samples the emitters directly)
   if (!pt && !disney) jobs = light_jobs(r, fa.frame0, fa.nframes);
-  const bool mega = !pt && r->attr(kMegakernel) != 0;
+  const bool mega = !pt && !disney &&
+                    (r->attr(kMegakernel) != 0 || (whole_paths(r, n, 2.0) && r->attr(kTailBounce) < 1.0));
   if (jobs.n) {
     // The first extension reads no light vertex: with the side stream the
     // pass runs there, after everything queued so far (earlier shading reads
@@ -1454,11 +1476,8 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
     ac.tend = r->tend.p;
   }
   if (mega) {
-    r->parts = 1;
-    r->extend_launches++;
     HIP_TRY(timed_begin(r, 0, &ev));
-    HIP_TRY(launch_mega(sc, fa, r->fc.p, r->lv.p, ac, (int)r->attr(kLdsStack), r->attr(kNodeFormat) != 0,
-                        r->stats.p, r->stream));
+    HIP_TRY(trace_whole(r, sc, fa, ac));
     HIP_TRY(timed_end(r, 0, ev));
   } else {
     int rc = bounce_loop(r, sc, fa, n, ac, true);
@@ -2161,8 +2180,12 @@ int batch_enqueue(cpt_batch* b, cpt_scene* s, u32 k) {
   ac.sample_n = r->sample_n.p;
   ac.rec.acc = r->rec_acc.p;
   ac.apply = 2;
-  int rc = bounce_loop(r, sc, fa, n, ac, true);
-  if (rc) return rc;
+  if (!r->persist_chunk && whole_paths(r, n, 2.0)) {
+    HIP_TRY(trace_whole(r, sc, fa, ac));
+  } else {
+    int rc = bounce_loop(r, sc, fa, n, ac, true);
+    if (rc) return rc;
+  }
   HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, 0, r->stream));
   HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, k, fa.eye_depth, r->parts, r->stream));
   HIP_TRY(launch_frame_advance(b->frame_dev.p, k, r->stream));

@@ -225,12 +225,14 @@ hipError_t launch_regen_light(const DevScene& sc, const FrameArgs& fa, LightVert
 hipError_t launch_regen_eye(const DevScene& sc, const FrameArgs& fa, const LightVert* lv, float* result,
                             uint32_t* sample_n, int lds_stack, int quant, DevStats* stats, hipStream_t st);
 // The bounces from bounce0 on, one thread per live slot of cur, as k_mega
-// carries them (grid: workgroups of the persistent launch).
+// carries them (groups: workgroups on each of `cus` compute units); bounces
+// before tail0 count as extension and shadow work.
 hipError_t launch_tail(const DevScene& sc, const FrameArgs& fa, PathBuf cur, FrameCounters* fc, uint32_t bounce0,
-                       uint32_t grid, const LightVert* lv, const Accum& ac, int lds_stack, int quant,
-                       DevStats* stats, hipStream_t st);
+                       uint32_t tail0, uint32_t groups, uint32_t cus, const LightVert* lv, const Accum& ac,
+                       int lds_stack, int quant, DevStats* stats, hipStream_t st);
+// Every path of the batch, from the camera on.
 hipError_t launch_mega(const DevScene& sc, const FrameArgs& fa, FrameCounters* fc, const LightVert* lv,
-                       const Accum& ac, int lds_stack, int quant, DevStats* stats, hipStream_t st);
+                       const Accum& ac, int lds_stack, int quant, uint32_t cus, DevStats* stats, hipStream_t st);
 // Path regeneration's second wavefront: T per frame from ac.term_bounce, the
 // counters of fc reset, and the restarted paths appended to pb.
 hipError_t launch_regen(const FrameArgs& fa, PathBuf pb, const Accum& ac, FrameCounters* fc, hipStream_t st);

@@ -2848,7 +2848,9 @@ hipError_t launch_regen_eye(const DevScene& sc, const FrameArgs& fa, const Light
 // are those of the wavefront passes (k_gen_eye, k_trace_dyn, k_shade,
 // k_shadow), so the image is the same bit for bit; only the schedule differs:
 // no path buffers, no compaction, and lanes of a wave idle once their paths
-// end.  The frame counters receive the same per-bounce counts.
+// end.  The frame counters receive the same per-bounce counts.  Bound by the latency of its
+// chain of node visits: four waves a SIMD (128 VGPRs, 14 of them spilled outside
+// the traversal) take 936 us for an 800 x 600 frame on the sphere grid, three (143) 977.
 // One bounce of a path that one thread carries (k_mega, k_tail): the closest
 // hit, shade_path, and the occlusion ray of the connection it sets up, whose
 // contribution is added when nothing occludes it.
@@ -2879,99 +2881,111 @@ __device__ __forceinline__ void carry_bounce(const DevScene& sc, const FrameArgs
   }
 }
 
-// Per-bounce live and shadow counts of a workgroup into the frame counters,
-// and its traversal counters into the statistics (TAIL: the tail's own
-// counters, with nr extension rays).
-template <bool TAIL>
-__device__ __forceinline__ void carry_flush(FrameCounters* fc, DevStats* stats, const uint32_t* n_live,
-                                            const uint32_t* n_shadow, uint32_t depth, uint32_t en, uint32_t et,
-                                            uint32_t sn, uint32_t st, uint32_t nr = 0) {
-  if (threadIdx.x < depth) {
-    const uint32_t b = threadIdx.x;
-    uint32_t* part = fc->part[blockIdx.x % kPartSlots];
-    if (b + 1 < 16 && n_live[b]) atomicAdd(&part[b + 1], n_live[b]);
-    if (n_shadow[b]) atomicAdd(&part[16 + b], n_shadow[b]);
+// A workgroup's counts: live and shadow rays per bounce; nodes and triangles of
+// the extension and the shadow rays, then the tail's nodes, triangles and rays.
+struct CarryCounts {
+  uint32_t live[16], shadow[16], trav[8];
+};
+__device__ __forceinline__ void carry_counts_clear(CarryCounts& C) {
+  static_assert(sizeof(CarryCounts) == 40 * 4, "one word a thread");
+  if (threadIdx.x < 40) ((uint32_t*)&C)[threadIdx.x] = 0u;
+  __syncthreads();
+}
+// Adds one bounce of a wave.  Called by the whole wave.
+__device__ __forceinline__ void carry_count(CarryCounts& C, uint32_t b, bool tail, uint32_t rays, bool survive,
+                                            bool emit, uint32_t en, uint32_t et, uint32_t sn, uint32_t st) {
+  const uint32_t cs = (uint32_t)__popcll(__ballot(survive)), ce = (uint32_t)__popcll(__ballot(emit));
+  const uint32_t a0 = wave_sum(en), a1 = wave_sum(et), a2 = wave_sum(sn), a3 = wave_sum(st);
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd(&C.live[b], cs);
+    atomicAdd(&C.shadow[b], ce);
+    atomicAdd(&C.trav[tail ? 4 : 0], tail ? a0 + a2 : a0);
+    atomicAdd(&C.trav[tail ? 5 : 1], tail ? a1 + a3 : a1);
+    atomicAdd(&C.trav[tail ? 6 : 2], tail ? rays : a2);
+    if (!tail) atomicAdd(&C.trav[3], a3);
   }
-  if (stats) stats = stat_slot(stats);
-  if (stats && TAIL) {
-    const uint32_t a0 = wave_sum(en + sn), a1 = wave_sum(et + st), a2 = wave_sum(nr);
-    if ((threadIdx.x & 63) == 0 && (a0 | a1 | a2)) {
-      atomicAdd(&stats->tail_nodes, (unsigned long long)a0);
-      atomicAdd(&stats->tail_tris, (unsigned long long)a1);
-      atomicAdd(&stats->tail_rays, (unsigned long long)a2);
-    }
-  } else if (stats) {
-    const uint32_t a0 = wave_sum(en), a1 = wave_sum(et), a2 = wave_sum(sn), a3 = wave_sum(st);
-    if ((threadIdx.x & 63) == 0) {
-      if (a0 | a1) {
-        atomicAdd(&stats->ext_nodes, (unsigned long long)a0);
-        atomicAdd(&stats->ext_tris, (unsigned long long)a1);
-      }
-      if (a2 | a3) {
-        atomicAdd(&stats->sh_nodes, (unsigned long long)a2);
-        atomicAdd(&stats->sh_tris, (unsigned long long)a3);
-      }
-    }
+}
+// Into the frame counters and the statistics.
+__device__ __forceinline__ void carry_flush(FrameCounters* fc, DevStats* stats, const CarryCounts& C, uint32_t depth) {
+  __syncthreads();
+  const uint32_t t = threadIdx.x;
+  if (t < depth) {
+    uint32_t* part = fc->part[blockIdx.x % kPartSlots];
+    if (t + 1 < 16 && C.live[t]) atomicAdd(&part[t + 1], C.live[t]);
+    if (C.shadow[t]) atomicAdd(&part[16 + t], C.shadow[t]);
+  }
+  if (stats && t < 7 && C.trav[t]) {
+    stats = stat_slot(stats);
+    unsigned long long* to[7] = {&stats->ext_nodes, &stats->ext_tris, &stats->sh_nodes, &stats->sh_tris,
+                                 &stats->tail_nodes, &stats->tail_tris, &stats->tail_rays};
+    atomicAdd(to[t], (unsigned long long)C.trav[t]);
   }
 }
 
+// Paths a wave carries: 64, but no more than spread a launch over half the waves
+// resident at once (`waves`), down to 16: a step of fewer rays tests its
+// triangles in fewer rounds and waits for fewer paths, while more waves a SIMD
+// wait for each other.  Frames of 128 x 128 and 256 x 256 paths on the sphere grid,
+// us: 64 a wave 303 / 386, over all resident waves (16) 246 / 354, over half of them
+// (16 / 32) 248 / 360; of 256 x 256 on the Cornell box 179 / 203 / 180.
+__host__ __device__ __forceinline__ uint32_t carry_paths(uint32_t n, uint32_t waves) {
+  const uint32_t w2 = waves / 2u, per = n / w2 + (n % w2 ? 1u : 0u);
+  return per < 16u ? 16u : per > 64u ? 64u : per;
+}
+
 template <int STK, bool Q>
-__global__ __launch_bounds__(kBlock) void k_mega(DevScene sc, FrameArgs fa, FrameCounters* __restrict__ fc,
+__global__ __launch_bounds__(kBlock, 4) void k_mega(DevScene sc, FrameArgs fa, FrameCounters* __restrict__ fc,
                                                  const LightVert* __restrict__ lv, Accum ac,
-                                                 DevStats* __restrict__ stats) {
+                                                 DevStats* __restrict__ stats, uint32_t per) {
   __shared__ TravLds<STK, Q> lds;
-  __shared__ uint32_t n_live[16], n_shadow[16];
-  if (threadIdx.x < 16) { n_live[threadIdx.x] = 0u; n_shadow[threadIdx.x] = 0u; }
-  __syncthreads();
-  const uint32_t wh = fa.width * fa.height;
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  __shared__ CarryCounts counts;
+  carry_counts_clear(counts);
   const int lane = threadIdx.x & 63;
-  uint32_t en = 0, et = 0, sn = 0, st = 0;
-  bool live = i < wh * fa.nframes;
+  const uint32_t i = (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * per + lane;
+  bool live = lane < (int)per && i < fa.width * fa.height * fa.nframes;
   PathState p;
   if (live) {                                               // pixel-major, as k_gen_eye
-    const uint32_t K = fa.nframes, pix = i / K, k = i - pix * K;
-    p = eye_path(fa, pix, k * wh + pix, stream_key(fa.seed, frame_base(fa) + k, 1u, 0u));
-    p.fk = k;
+    uint32_t dk;
+    p = eye_slot(fa, i, dk);
+    unpack_dk(p, dk);
+    if (ac.variant & kVariantGbuf) zero_rec(ac.rec, p.sid); // a miss leaves the G-buffer record at zero
   }
   const uint32_t depth = fa.eye_depth < 16u ? fa.eye_depth : 16u;
   for (uint32_t b = 0; b < depth; b++) {
     if (__ballot(live) == 0ull) break;                    // wave-uniform
     bool survive = false, emit = false;
+    uint32_t en = 0, et = 0, sn = 0, st = 0;
     carry_bounce<STK, Q>(sc, fa, fc, lv, ac, p, lds, live, survive, emit, en, et, sn, st);
     live = survive;
-    const uint32_t cs = (uint32_t)__popcll(__ballot(survive)), ce = (uint32_t)__popcll(__ballot(emit));
-    if (lane == 0) {
-      if (cs) atomicAdd(&n_live[b], cs);
-      if (ce) atomicAdd(&n_shadow[b], ce);
-    }
+    carry_count(counts, b, false, 0u, survive, emit, en, et, sn, st);
   }
-  __syncthreads();
-  carry_flush<false>(fc, stats, n_live, n_shadow, depth, en, et, sn, st);
+  carry_flush(fc, stats, counts, depth);
 }
 
 // The last bounces of the wavefront in one launch.  Once few paths are left,
 // a bounce's refilling grid runs partly empty and each of its three launches
 // (extension, shading, occlusion) waits for its slowest ray; from bounce
-// `bounce0` on, each thread instead takes live slots of `cur` (strided over a
+// `bounce0` on, each wave instead takes live slots of `cur` (strided over a
 // persistent grid) and carries each path through the remaining bounces as
 // k_mega does, with the same per-path arithmetic: the image does not change.
+// Traversal of bounces before `tail0` counts as extension and shadow work, of
+// the others as the tail's.  waves: those resident at once (carry_paths).
 template <int STK, bool Q>
-__global__ __launch_bounds__(kBlock) void k_tail(DevScene sc, FrameArgs fa, PathBuf cur,
-                                                 FrameCounters* __restrict__ fc, uint32_t bounce0,
+__global__ __launch_bounds__(kBlock, 4) void k_tail(DevScene sc, FrameArgs fa, PathBuf cur,
+                                                 FrameCounters* __restrict__ fc, uint32_t bounce0, uint32_t tail0,
                                                  const LightVert* __restrict__ lv, Accum ac,
-                                                 DevStats* __restrict__ stats) {
+                                                 DevStats* __restrict__ stats, uint32_t waves) {
   __shared__ TravLds<STK, Q> lds;
-  __shared__ uint32_t n_live[16], n_shadow[16];
-  if (threadIdx.x < 16) { n_live[threadIdx.x] = 0u; n_shadow[threadIdx.x] = 0u; }
-  __syncthreads();
+  __shared__ CarryCounts counts;
+  carry_counts_clear(counts);
   const uint32_t count = fc->active[bounce0];
+  const uint32_t per = carry_paths(count, waves);
   const int lane = threadIdx.x & 63;
   const uint32_t depth = fa.eye_depth < 16u ? fa.eye_depth : 16u;
-  uint32_t en = 0, et = 0, sn = 0, st = 0, nr = 0;
-  for (uint32_t base = blockIdx.x * kBlock; base < count; base += gridDim.x * kBlock) {   // workgroup-uniform
-    const uint32_t i = base + threadIdx.x;
-    bool live = i < count;
+  const uint32_t wave = blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (uint32_t base = wave * per; base < count; base += gridDim.x * (kBlock / 64) * per) {   // wave-uniform
+    const uint32_t i = base + lane;
+    bool live = lane < (int)per && i < count;
     PathState p;
     if (live) {
       p.ro = cur.ray_o[i];
@@ -2994,29 +3008,27 @@ __global__ __launch_bounds__(kBlock) void k_tail(DevScene sc, FrameArgs fa, Path
     for (uint32_t b = bounce0; b < depth; b++) {
       if (__ballot(live) == 0ull) break;                  // wave-uniform
       bool survive = false, emit = false;
-      nr += live;
+      uint32_t en = 0, et = 0, sn = 0, st = 0;
+      const uint32_t rays = (uint32_t)__popcll(__ballot(live));
       carry_bounce<STK, Q>(sc, fa, fc, lv, ac, p, lds, live, survive, emit, en, et, sn, st);
       live = survive;
-      const uint32_t cs = (uint32_t)__popcll(__ballot(survive)), ce = (uint32_t)__popcll(__ballot(emit));
-      if (lane == 0) {
-        if (cs) atomicAdd(&n_live[b], cs);
-        if (ce) atomicAdd(&n_shadow[b], ce);
-      }
+      carry_count(counts, b, b >= tail0, rays, survive, emit, en, et, sn, st);
     }
   }
-  __syncthreads();
-  carry_flush<true>(fc, stats, n_live, n_shadow, depth, en, et, sn, st, nr);
+  carry_flush(fc, stats, counts, depth);
 }
 hipError_t launch_tail(const DevScene& sc, const FrameArgs& fa, PathBuf cur, FrameCounters* fc, uint32_t bounce0,
-                       uint32_t grid, const LightVert* lv, const Accum& ac, int lds_stack, int quant,
-                       DevStats* stats, hipStream_t st) {
-  // bounce0 >= 1: no path of the tail is at its first hit, so a G-buffer
-  // variant (written at depth 0 only) is allowed
-  if (!fc || !lv || !ac.rec.acc || ac.apply != 2 || fa.eye_depth > 16 ||
-      bounce0 == 0 || bounce0 >= fa.eye_depth || grid == 0 || !pathbuf_ok(cur) || !sc.tris ||
-      !nodes_ok(sc, quant))
+                       uint32_t tail0, uint32_t groups, uint32_t cus, const LightVert* lv, const Accum& ac,
+                       int lds_stack, int quant, DevStats* stats, hipStream_t st) {
+  if (!fc || !lv || !ac.rec.acc || fa.eye_depth > 16 ||
+      bounce0 >= fa.eye_depth || groups == 0 || cus == 0 || !pathbuf_ok(cur) || !sc.tris || !nodes_ok(sc, quant))
     return hipErrorInvalidValue;
-#define CPT_TL(S, W, Q) k_tail<S, Q><<<grid, kBlock, 0, st>>>(sc, fa, cur, fc, bounce0, lv, ac, stats)
+#define CPT_TL(S, W, Q)                                                                                           \
+  {                                                                                                               \
+    static const uint32_t resident = resident_groups((const void*)k_tail<S, Q>);                                  \
+    k_tail<S, Q><<<groups * cus, kBlock, 0, st>>>(sc, fa, cur, fc, bounce0, tail0, lv, ac, stats,                 \
+                                                  resident * cus * (kBlock / 64));                                \
+  }
 #define CPT_TL_Q(S, W) CPT_TL(S, W, true)
 #define CPT_TL_F(S, W) CPT_TL(S, W, false)
   if (quant) {
@@ -3030,15 +3042,18 @@ hipError_t launch_tail(const DevScene& sc, const FrameArgs& fa, PathBuf cur, Fra
   return hipGetLastError();
 }
 hipError_t launch_mega(const DevScene& sc, const FrameArgs& fa, FrameCounters* fc, const LightVert* lv,
-                       const Accum& ac, int lds_stack, int quant, DevStats* stats, hipStream_t st) {
+                       const Accum& ac, int lds_stack, int quant, uint32_t cus, DevStats* stats, hipStream_t st) {
   const uint64_t n = (uint64_t)fa.width * fa.height * fa.nframes;
   if (n == 0) return hipSuccess;
-  if (n > 0xFFFFFFFFull - kBlock || !fc || !lv || !ac.rec.acc || ac.apply != 2 || (ac.variant & kVariantGbuf) ||
-      fa.eye_depth > 16 || !sc.tris ||
-      !nodes_ok(sc, quant))
+  if (n > 0xFFFFFFFFull - 4 * kBlock || !fc || !lv || !ac.rec.acc || fa.eye_depth > 16 || cus == 0 || !sc.tris ||
+      !nodes_ok(sc, quant) || ((ac.variant & kVariantGbuf) && !rec_ok(ac.rec)))
     return hipErrorInvalidValue;
-  dim3 grid((uint32_t)((n + kBlock - 1) / kBlock)), block(kBlock);
-#define CPT_MG(S, W, Q) k_mega<S, Q><<<grid, block, 0, st>>>(sc, fa, fc, lv, ac, stats)
+#define CPT_MG(S, W, Q)                                                                                           \
+  {                                                                                                               \
+    static const uint32_t resident = resident_groups((const void*)k_mega<S, Q>);                                  \
+    const uint32_t per = carry_paths((uint32_t)n, resident * cus * (kBlock / 64)), wg = per * (kBlock / 64);      \
+    k_mega<S, Q><<<(uint32_t)((n + wg - 1) / wg), kBlock, 0, st>>>(sc, fa, fc, lv, ac, stats, per);               \
+  }
   if (quant) {
 #define CPT_MG_Q(S, W) CPT_MG(S, W, true)
 #define CPT_MG_F(S, W) CPT_MG(S, W, false)
