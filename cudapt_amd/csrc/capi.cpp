@@ -790,6 +790,55 @@ struct cpt_mlp {
   }
 };
 
+// Device memory to pageable host memory through a ring of pinned chunks owned
+// by a renderer: the runtime's own staging copies a chunk, waits and copies it
+// on, here the next chunks are under way meanwhile.  Images into fresh arrays, ring /
+// runtime, us: 5.8 MB 341 / 409, 24.9 MB 1281 / 1730, 106 MB 8016 / 10045 (chunks of
+// 256 KB 769 / 2060 for the first two, of 4 MB the same as of 1 MB).
+// Memory that the runtime knows (pinned, managed, device) is copied to directly.
+constexpr size_t kReadChunk = 1u << 20, kReadChunks = 4;
+struct Readback {
+  std::mutex lock;                 // one ring, whoever reads
+  char* ring = nullptr;
+  hipEvent_t done[kReadChunks] = {};
+  ~Readback() {
+    for (auto e : done)
+      if (e) (void)hipEventDestroy(e);
+    if (ring) (void)hipHostFree(ring);
+  }
+  hipError_t read(void* out, const void* src, size_t bytes, hipStream_t st) {
+    hipPointerAttribute_t at;
+    const bool known = hipPointerGetAttributes(&at, out) == hipSuccess && at.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    if (known) {
+      const hipError_t e = hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, st);
+      return e != hipSuccess ? e : hipStreamSynchronize(st);
+    }
+    std::lock_guard<std::mutex> g(lock);
+    hipError_t e = hipSuccess;
+    if (!ring) e = hipHostMalloc((void**)&ring, kReadChunk * kReadChunks, hipHostMallocDefault);
+    for (auto& d : done)
+      if (e == hipSuccess && !d) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
+    const size_t n = (bytes + kReadChunk - 1) / kReadChunk;
+    const auto len = [&](size_t k) { return std::min(kReadChunk, bytes - k * kReadChunk); };
+    const auto start = [&](size_t k) {
+      const size_t slot = k % kReadChunks;
+      e = hipMemcpyAsync(ring + slot * kReadChunk, (const char*)src + k * kReadChunk, len(k), hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipEventRecord(done[slot], st);
+    };
+    for (size_t k = 0; k < std::min(n, kReadChunks) && e == hipSuccess; k++) start(k);
+    for (size_t k = 0; k < n && e == hipSuccess; k++) {
+      const size_t slot = k % kReadChunks;
+      e = hipEventSynchronize(done[slot]);
+      if (e != hipSuccess) break;
+      std::memcpy((char*)out + k * kReadChunk, ring + slot * kReadChunk, len(k));
+      if (k + kReadChunks < n) start(k + kReadChunks);
+    }
+    const hipError_t es = hipStreamSynchronize(st);      // also after an error: nothing writes the ring any more
+    return e != hipSuccess ? e : es;
+  }
+};
+
 struct cpt_renderer {
   int mode = 0;
   u32 W = 0, H = 0;
@@ -828,6 +877,7 @@ struct cpt_renderer {
   // extension (which reads no light vertex); the first shading waits for it
   hipEvent_t ev_light = nullptr;
   bool light_pending = false;
+  Readback readback;
   ~cpt_renderer() {
     for (auto& e : events) { pool.push_back(e.a); pool.push_back(e.b); }
     for (auto e : pool) (void)hipEventDestroy(e);
@@ -1510,9 +1560,9 @@ int copy_result(cpt_renderer* r, float* result) {
   const size_t n = (size_t)r->W * r->H;
   const u32 debug = is_adaptive(r->mode) ? (u32)r->attr(kDebugMode) : 0u;
   if (debug == 0) {
-    HIP_TRY(hipMemcpyAsync(result, r->result.p, n * 12, hipMemcpyDeviceToHost, r->stream));
+    HIP_TRY(r->readback.read(result, r->result.p, n * 12, r->stream));
   } else if (debug == 4) {
-    HIP_TRY(hipMemcpyAsync(result, r->filtered.p, n * 12, hipMemcpyDeviceToHost, r->stream));
+    HIP_TRY(r->readback.read(result, r->filtered.p, n * 12, r->stream));
   } else {
     std::vector<float> grey(n);
     HIP_TRY(hipMemcpyAsync(grey.data(), debug == 1 ? (const void*)r->counts.p : (const void*)r->err.p, n * 4,
@@ -1524,7 +1574,6 @@ int copy_result(cpt_renderer* r, float* result) {
       result[i * 3] = result[i * 3 + 1] = result[i * 3 + 2] = v;
     }
   }
-  HIP_TRY(hipStreamSynchronize(r->stream));
   return CPT_OK;
 }
 
@@ -1653,8 +1702,7 @@ int read_pixels(cpt_renderer* r, int which, size_t off, size_t n, void* out, con
     default:
       return fail(CPT_E_ARG, "%s: buffer %d not produced by this mode", fn, which);
   }
-  HIP_TRY(hipMemcpyAsync(out, src, n * per, hipMemcpyDeviceToHost, r->stream));
-  HIP_TRY(hipStreamSynchronize(r->stream));
+  HIP_TRY(r->readback.read(out, src, n * per, r->stream));
   return CPT_OK;
 }
 
@@ -2429,9 +2477,8 @@ int cpt_batch_read_result(cpt_batch* b, uint32_t view, float* out) {
   if (view >= b->vd.size()) return fail(CPT_E_ARG, "cpt_batch_read_result: view %u out of range", view);
   if (!b->r->allocated) return fail(CPT_E_STATE, "cpt_batch_read_result: nothing rendered yet");
   const ViewDesc& d = b->vd[view];
-  HIP_TRY(hipMemcpyAsync(out, b->r->result.p + (size_t)d.offset * 3, (size_t)d.width * d.height * 12,
-                         hipMemcpyDeviceToHost, b->r->stream));
-  HIP_TRY(hipStreamSynchronize(b->r->stream));
+  HIP_TRY(b->r->readback.read(out, b->r->result.p + (size_t)d.offset * 3, (size_t)d.width * d.height * 12,
+                              b->r->stream));
   return CPT_OK;
 }
 
@@ -2440,9 +2487,7 @@ int cpt_batch_sample_counts(cpt_batch* b, uint32_t view, uint32_t* out) {
   if (view >= b->vd.size()) return fail(CPT_E_ARG, "cpt_batch_sample_counts: view %u out of range", view);
   if (!b->r->allocated) return fail(CPT_E_STATE, "cpt_batch_sample_counts: nothing rendered yet");
   const ViewDesc& d = b->vd[view];
-  HIP_TRY(hipMemcpyAsync(out, b->r->sample_n.p + d.offset, (size_t)d.width * d.height * 4, hipMemcpyDeviceToHost,
-                         b->r->stream));
-  HIP_TRY(hipStreamSynchronize(b->r->stream));
+  HIP_TRY(b->r->readback.read(out, b->r->sample_n.p + d.offset, (size_t)d.width * d.height * 4, b->r->stream));
   return CPT_OK;
 }
 
