@@ -632,8 +632,7 @@ def filter_cross_bilateral(color, pos, norm, diff, sample_n, sigma_color, sigma_
                            nd=5, noalloc=False):
     """Device cross-bilateral + weighted squared residual on host images (copies in and out).
 
-    noalloc: call cpt_filter_cross_bilateral_device_noalloc, which stages its
-    table in the library's static device scratch instead of allocating."""
+    noalloc: call cpt_filter_cross_bilateral_device_noalloc, which allocates nothing."""
     H, W = color.shape[:2]
     bufs = [DeviceBuffer.from_array(np.ascontiguousarray(a, np.float32)) for a in (color, pos, norm)]
     db = DeviceBuffer.from_array(np.ascontiguousarray(diff, np.float32)) if diff is not None else None

@@ -200,19 +200,12 @@ int upload_materials(cpt_scene* s) {
   return CPT_OK;
 }
 
-// cudaBilateralFilter::updateGaussian (src/cudaBilateralFilter.cu:5-24): the
-// spatial table of 2 * radius + 1 taps, sigma = the colour sigma as the
-// reference's callers pass it, zero beyond.
+// The filter's arguments.  Spatial table: cudaBilateralFilter::updateGaussian
+// (src/cudaBilateralFilter.cu:5-24), 2 * radius + 1 taps of ss (the colour
+// sigma as the reference's callers pass it, or one of its own), zero beyond.
+// It travels with the launch: no device copy, so none to share or to wait for.
 constexpr int kFilterTable = 2 * kMaxFilterRadius + 2;
-void filter_table(float sigma_color, u32 radius, float g[kFilterTable]) {
-  for (int i = 0; i < kFilterTable; i++) g[i] = 0.f;
-  for (u32 i = 0; i < 2 * radius + 1; i++) {
-    int x = (int)i - (int)radius;
-    g[i] = std::exp(-(float)(x * x) / (2 * sigma_color * sigma_color));
-  }
-}
-
-FilterArgs filter_args(u32 width, u32 height, float sc, float sp, float sn, float sd, u32 radius, u32 nd,
+FilterArgs filter_args(u32 width, u32 height, float ss, float sc, float sp, float sn, float sd, u32 radius, u32 nd,
                        bool use_diff) {
   FilterArgs f;
   f.width = width; f.height = height; f.radius = radius; f.nd = nd;
@@ -221,34 +214,11 @@ FilterArgs filter_args(u32 width, u32 height, float sc, float sp, float sn, floa
   f.use_diff = use_diff;
   f.kz = 0.f;
   f.cam[0] = f.cam[1] = f.cam[2] = 0.f;
-  return f;
-}
-
-// Staging of cpt_filter_cross_bilateral_device_noalloc: the spatial table the
-// filter kernel reads, kept in a file-scope device array instead of a
-// per-call allocation.  Every device the library runs on holds its own copy
-// (256 bytes) until the process ends.  In host code `scratch` names a host-side
-// stand-in, never the device copy: kernels and copies take the address that
-// hipGetSymbolAddress returns for the current device, cached per device.
-__device__ __align__(256) float scratch[kFilterTable];
-constexpr int kScratchDevices = 64;
-std::mutex g_scratch_mu;
-float* g_scratch_ptr[kScratchDevices] = {};
-
-int filter_scratch(float** out) {
-  int dev = 0;
-  HIP_TRY(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kScratchDevices)
-    return fail(CPT_E_LIMIT, "filter scratch: device %d beyond the %d the library tracks", dev, kScratchDevices);
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (!g_scratch_ptr[dev]) {
-    void* p = nullptr;
-    HIP_TRY(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-    if (!p) return fail(CPT_E_HIP, "filter scratch: hipGetSymbolAddress returned no address on device %d", dev);
-    g_scratch_ptr[dev] = (float*)p;
+  for (int i = 0; i < kFilterTable; i++) {
+    const int x = i - (int)radius;
+    f.gauss[i] = i < 2 * (int)radius + 1 ? std::exp(-(float)(x * x) / (2 * ss * ss)) : 0.f;
   }
-  *out = g_scratch_ptr[dev];
-  return CPT_OK;
+  return f;
 }
 
 }  // namespace
@@ -611,18 +581,10 @@ int cpt_filter_cross_bilateral_device(const float* d_color, const float* d_pos, 
   if (width == 0 || height == 0) return fail(CPT_E_ARG, "cpt_filter_cross_bilateral_device: empty image");
   if (radius > (u32)kMaxFilterRadius) return fail(CPT_E_LIMIT, "cpt_filter_cross_bilateral_device: radius %u > 31", radius);
   hipStream_t st = (hipStream_t)stream;
-  float g[kFilterTable];
-  filter_table(sigma_color, radius, g);
-  float* d_g = nullptr;
-  HIP_TRY(hipMalloc((void**)&d_g, sizeof g));
-  HIP_TRY(hipMemcpyAsync(d_g, g, sizeof g, hipMemcpyHostToDevice, st));
-  const FilterArgs f = filter_args(width, height, sigma_color, sigma_pos, sigma_norm, sigma_diff, radius, nd,
-                                   d_diff != nullptr);
-  hipError_t e = launch_filter_error(f, d_color, d_pos, d_norm, d_diff, d_g, d_sample_n, d_filtered, d_err, st);
-  hipError_t e2 = hipStreamSynchronize(st);
-  (void)hipFree(d_g);
-  HIP_TRY(e);
-  HIP_TRY(e2);
+  const FilterArgs f = filter_args(width, height, sigma_color, sigma_color, sigma_pos, sigma_norm, sigma_diff, radius,
+                                   nd, d_diff != nullptr);
+  HIP_TRY(launch_filter_error(f, d_color, d_pos, d_norm, d_diff, d_sample_n, d_filtered, d_err, st));
+  HIP_TRY(hipStreamSynchronize(st));
   return CPT_OK;
 }
 
@@ -637,20 +599,11 @@ int cpt_filter_cross_bilateral_device_noalloc(const float* d_color, const float*
   if (radius > (u32)kMaxFilterRadius)
     return fail(CPT_E_LIMIT, "cpt_filter_cross_bilateral_device_noalloc: radius %u > %d: the %d-entry scratch table "
                 "holds 2 * radius + 1 taps", radius, kMaxFilterRadius, kFilterTable);
-  float* d_g = nullptr;
-  int rc = filter_scratch(&d_g);
-  if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
-  float g[kFilterTable];
-  filter_table(sigma_color, radius, g);
-  // every entry is rewritten, so nothing of an earlier call's table survives
-  HIP_TRY(hipMemcpyAsync(d_g, g, sizeof g, hipMemcpyHostToDevice, st));
-  const FilterArgs f = filter_args(width, height, sigma_color, sigma_pos, sigma_norm, sigma_diff, radius, nd,
-                                   d_diff != nullptr);
-  hipError_t e = launch_filter_error(f, d_color, d_pos, d_norm, d_diff, d_g, d_sample_n, d_filtered, d_err, st);
-  hipError_t e2 = hipStreamSynchronize(st);       // g is on this stack frame until the copy has run
-  HIP_TRY(e);
-  HIP_TRY(e2);
+  const FilterArgs f = filter_args(width, height, sigma_color, sigma_color, sigma_pos, sigma_norm, sigma_diff, radius,
+                                   nd, d_diff != nullptr);
+  HIP_TRY(launch_filter_error(f, d_color, d_pos, d_norm, d_diff, d_sample_n, d_filtered, d_err, st));
+  HIP_TRY(hipStreamSynchronize(st));
   return CPT_OK;
 }
 
@@ -901,7 +854,7 @@ struct cpt_renderer {
       if (std::strcmp(a.name, name) == 0) a.value = v;
   }
   // adaptive mode
-  DevArray<float> gpos, gnrm, gdif, filtered, err, gauss, err_sum;
+  DevArray<float> gpos, gnrm, gdif, filtered, err, err_sum;
   DevArray<u32> counts, offsets, block_tot, total, big_list, big_n;
   DevArray<u32> paths;                  // eye paths traced per pixel since the last restart
   DevArray<float> sq, maxe;                  // second moment (W*H*3), max of the error map
@@ -912,8 +865,6 @@ struct cpt_renderer {
   DevArray<float4> rec_acc, rec_pos, rec_nrm, rec_dif;
   DevArray<u32> term_bounce, tend;           // path regeneration: where each path ended, per-frame last bounce
   DevArray<uint64_t> term_rng;               // and the RNG state it ended in
-  float gauss_sigma = -1.f;
-  u32 gauss_radius = 0;
   u32 persist_chunk = 0, persist_grid = 0;   // persistent extend grid (0: one thread per ray)
   int cus = 0;                               // compute units of the device
   DevArray<u32> queue;                       // work counters of the refilling launches, then k_extend_persist's
@@ -960,7 +911,6 @@ int renderer_alloc(cpt_renderer* r) {
     HIP_TRY(r->gdif.alloc(n * 3));
     HIP_TRY(r->filtered.alloc(n * 3));
     HIP_TRY(r->err.alloc(n));
-    HIP_TRY(r->gauss.alloc(64));
     HIP_TRY(r->err_sum.alloc(1));
     HIP_TRY(r->counts.alloc(n));
     HIP_TRY(r->paths.alloc(n));
@@ -1053,22 +1003,6 @@ void camera_basis(const float* d, const float* up, float* right, float* up2) {
   float ux = right[1] * d[2] - right[2] * d[1], uy = right[2] * d[0] - right[0] * d[2], uz = right[0] * d[1] - right[1] * d[0];
   float ul = std::sqrt(ux * ux + uy * uy + uz * uz);
   up2[0] = ux / ul; up2[1] = uy / ul; up2[2] = uz / ul;
-}
-
-// Gaussian table of cudaBilateralFilter::updateGaussian (cudaBilateralFilter.cu:5-24),
-// spatial sigma = colour sigma as the reference passes it (AdapBilatAtomic.cu:1327).
-int update_gauss(cpt_renderer* r, float sigma, u32 radius) {
-  if (sigma == r->gauss_sigma && radius == r->gauss_radius) return CPT_OK;
-  float g[64] = {0};
-  for (u32 i = 0; i < 2 * radius + 1; i++) {
-    int x = (int)i - (int)radius;
-    g[i] = std::exp(-(float)(x * x) / (2 * sigma * sigma));
-  }
-  HIP_TRY(hipMemcpyAsync(r->gauss.p, g, sizeof g, hipMemcpyHostToDevice, r->stream));
-  HIP_TRY(hipStreamSynchronize(r->stream));
-  r->gauss_sigma = sigma;
-  r->gauss_radius = radius;
-  return CPT_OK;
 }
 
 // A launch too small to fill the chip bounce by bounce: each thread carries its
@@ -1247,9 +1181,7 @@ int run_filter_at(cpt_renderer* r, size_t off, u32 W, u32 H, const float* cam, c
   // the spatial table takes the colour sigma as the reference's callers pass it
   // (AdapBilatAtomic.cu:1327) unless a spatial sigma of its own is set
   const float ss = (float)r->attr(kFilterSpatial);
-  int rc = update_gauss(r, ss > 0.f ? ss : sc_, radius);
-  if (rc) return rc;
-  FilterArgs f = filter_args(W, H, sc_, sp_, sn_, sd_, radius, (u32)r->attr("Desired Max Sampling"),
+  FilterArgs f = filter_args(W, H, ss > 0.f ? ss : sc_, sc_, sp_, sn_, sd_, radius, (u32)r->attr("Desired Max Sampling"),
                              r->attr("Filter Diffuse Flag") != 0);
   const float sz = (float)r->attr(kFilterDepth);
   if (sz > 0.f) {
@@ -1257,7 +1189,7 @@ int run_filter_at(cpt_renderer* r, size_t off, u32 W, u32 H, const float* cam, c
     f.cam[0] = cam[0]; f.cam[1] = cam[1]; f.cam[2] = cam[2];
   }
   const size_t o3 = 3 * off;
-  HIP_TRY(launch_filter_error(f, src + o3, r->gpos.p + o3, r->gnrm.p + o3, r->gdif.p + o3, r->gauss.p,
+  HIP_TRY(launch_filter_error(f, src + o3, r->gpos.p + o3, r->gnrm.p + o3, r->gdif.p + o3,
                               r->sample_n.p + off, dst + o3, err + off, r->stream));
   return CPT_OK;
 }

@@ -3068,13 +3068,12 @@ hipError_t launch_mega(const DevScene& sc, const FrameArgs& fa, FrameCounters* f
 }
 
 // ---------------------------------------------------------------- adaptive sampling
-// e^x: Cody-Waite reduction + degree-7 Taylor polynomial, 2^k by ldexp
-// (Cody & Waite 1980).  The host oracle evaluates the identical fma sequence.
-__device__ __forceinline__ float cpt_expf(float x) {
-  if (x < -103.0f) return 0.f;
-  if (x > 88.0f) return __builtin_huge_valf();
-  float k = rintf(x * 1.44269504f);
-  float r = fmaf(k, -0.693145751953125f, x);
+// e^-a for a that is 0 or more, or NaN (0 past 103): Cody-Waite reduction +
+// degree-7 Taylor polynomial, 2^k by ldexp (Cody & Waite 1980).  The host oracle
+// evaluates the identical fma sequence.
+__device__ __forceinline__ float cpt_exp_neg(float a) {
+  const float k = rintf(-a * 1.44269504f);
+  float r = fmaf(k, -0.693145751953125f, -a);
   r = fmaf(k, -1.42860676533018e-06f, r);
   float p = 1.f / 5040.f;
   p = fmaf(p, r, 1.f / 720.f);
@@ -3084,7 +3083,8 @@ __device__ __forceinline__ float cpt_expf(float x) {
   p = fmaf(p, r, 0.5f);
   p = fmaf(p, r, 1.f);
   p = fmaf(p, r, 1.f);
-  return ldexpf(p, (int)k);
+  const float e = ldexpf(p, (int)k);
+  return a > 103.f ? 0.f : e;
 }
 __device__ __forceinline__ float sqdist3(const float* a, const float* b) {
   float dx = a[0] - b[0], dy = a[1] - b[1], dz = a[2] - b[2];
@@ -3105,124 +3105,214 @@ constexpr int kTile = 16;
 constexpr int kLdsRadius = 9;     // LDS tile path up to this radius, global reads beyond
 
 // Cross-bilateral over colour/position/normal(/albedo) + the weighted squared
-// residual of pt_calculateSquareError_kernel, one 16x16 tile per workgroup.
-// The (16+2r)^2 input halo is staged in LDS once; every tap then reads LDS.
-// One exponential per tap: the range terms' exponents are summed, each scaled
-// by its 1 / 2 sigma^2 (correctly rounded once per thread) and accumulated
-// with fmas, so a tap takes no division.
-template <bool DIFF, bool LDS>
-__global__ __launch_bounds__(kTile * kTile) void k_filter_error(FilterArgs fa, const float* __restrict__ color,
-                                                                const float* __restrict__ gpos,
-                                                                const float* __restrict__ gnrm,
-                                                                const float* __restrict__ gdif,
-                                                                const float* __restrict__ gauss,
-                                                                const uint32_t* __restrict__ sample_n,
-                                                                float* __restrict__ filtered, float* __restrict__ err) {
-  extern __shared__ float sm[];
-  const int R = (int)fa.radius, TW = kTile + 2 * R, TA = TW * TW;
-  const uint32_t W = fa.width, H = fa.height;
-  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * kTile + tx;
-  const int bx = blockIdx.x * kTile, by = blockIdx.y * kTile;
-  float* sg = sm;                                  // 2R+1 spatial weights
-  float* sc = sg + 2 * kMaxFilterRadius + 2;       // 3 floats per halo pixel, per plane
-  float* sp = sc + 3 * (LDS ? TA : 0);
-  float* sn = sp + 3 * (LDS ? TA : 0);
-  float* sd = sn + 3 * (LDS ? TA : 0);
-  float* sz = sd + 3 * (LDS && DIFF ? TA : 0);     // depth per halo pixel (depth term on)
-  const bool depth = fa.kz > 0.f;
-  const float cam[3] = {fa.cam[0], fa.cam[1], fa.cam[2]};
-  for (int k = tid; k < 2 * R + 1; k += kTile * kTile) sg[k] = gauss[k];
-  if (LDS) {
-    for (int k = tid; k < TA; k += kTile * kTile) {
-      int hx = k % TW, hy = k / TW;
-      size_t g = ((size_t)ref_clamp_i(by + hy - R, H) * W + ref_clamp_i(bx + hx - R, W)) * 3;
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        sc[k * 3 + c] = color[g + c];
-        sp[k * 3 + c] = gpos[g + c];
-        sn[k * 3 + c] = gnrm[g + c];
-        if (DIFF) sd[k * 3 + c] = gdif[g + c];
-      }
-      if (depth) sz[k] = sqrtf(sqdist3(gpos + g, cam));
-    }
+// residual of pt_calculateSquareError_kernel.  One exponential per tap: the
+// range terms' exponents are summed, each scaled by its 1 / 2 sigma^2 (correctly rounded
+// once per thread) and accumulated with fmas, so a tap takes no division.
+// A pixel: its own guides and the sums so far, taps added in raster order.
+template <bool DIFF, bool DEPTH>
+struct FilterPixel {
+  float c[3], p[3], n[3], d[3], z, iz;
+  float sum, t0, t1, t2;
+};
+struct FilterScale {
+  float c, p, n, d, z;
+};
+struct FilterTap {
+  float c[3], p[3], n[3], d[3], z;
+};
+// The tap's negated exponent: 0 or more, or NaN (every scale is the reciprocal of a square).
+template <bool DIFF, bool DEPTH>
+__device__ __forceinline__ float filter_exponent(const FilterPixel<DIFF, DEPTH>& P, const FilterTap& q,
+                                                 const FilterScale& k) {
+  float a = sqd_fma(q.c, P.c) * k.c;
+  a = __builtin_fmaf(sqd_fma(q.p, P.p), k.p, a);
+  a = __builtin_fmaf(sqd_fma(q.n, P.n), k.n, a);
+  if (DIFF) a = __builtin_fmaf(sqd_fma(q.d, P.d), k.d, a);
+  if (DEPTH) {
+    const float dz = (q.z - P.z) * P.iz;
+    a = __builtin_fmaf(dz * dz, k.z, a);
   }
-  __syncthreads();
-  const uint32_t x = bx + tx, y = by + ty;
-  if (x >= W || y >= H) return;
-  const size_t ind = (size_t)y * W + x;
-  float cc[3], cp[3], cn[3], cd[3];
-#pragma unroll
-  for (int c = 0; c < 3; c++) {
-    cc[c] = color[ind * 3 + c];
-    cp[c] = gpos[ind * 3 + c];
-    cn[c] = gnrm[ind * 3 + c];
-    cd[c] = DIFF ? gdif[ind * 3 + c] : 0.f;
-  }
-  const float zc = depth ? sqrtf(sqdist3(cp, cam)) : 0.f;
-  const float izc = zc > 0.f ? 1.f / zc : 0.f;
-  const float ikc = 1.f / fa.kc, ikp = 1.f / fa.kp, ikn = 1.f / fa.kn, ikd = 1.f / fa.kd;
-  const float ikz = depth ? 1.f / fa.kz : 0.f;
-  float sum = 0.f, t0 = 0.f, t1 = 0.f, t2 = 0.f;
-  for (int i = -R; i <= R; i++) {
-    for (int j = -R; j <= R; j++) {
-      const float *qc, *qp, *qn, *qd = nullptr;
-      float zq = 0.f;
-      if (LDS) {
-        int k = (ty + R + i) * TW + (tx + R + j);
-        qc = sc + k * 3; qp = sp + k * 3; qn = sn + k * 3;
-        if (DIFF) qd = sd + k * 3;
-        if (depth) zq = sz[k];
-      } else {
-        size_t g = ((size_t)ref_clamp_i((int)y + i, H) * W + ref_clamp_i((int)x + j, W)) * 3;
-        qc = color + g; qp = gpos + g; qn = gnrm + g;
-        if (DIFF) qd = gdif + g;
-        if (depth) zq = sqrtf(sqdist3(qp, cam));
-      }
-      float a = sqd_fma(qc, cc) * ikc;
-      a = __builtin_fmaf(sqd_fma(qp, cp), ikp, a);
-      a = __builtin_fmaf(sqd_fma(qn, cn), ikn, a);
-      if (DIFF) a = __builtin_fmaf(sqd_fma(qd, cd), ikd, a);
-      if (depth) {
-        const float dz = (zq - zc) * izc;
-        a = __builtin_fmaf(dz * dz, ikz, a);
-      }
-      float f = (sg[i + R] * sg[j + R]) * cpt_expf(-a);
-      t0 = __builtin_fmaf(f, qc[0], t0);
-      t1 = __builtin_fmaf(f, qc[1], t1);
-      t2 = __builtin_fmaf(f, qc[2], t2);
-      sum = sum + f;
-    }
-  }
-  float o0 = t0 / sum, o1 = t1 / sum, o2 = t2 / sum;
+  return a;
+}
+template <bool DIFF, bool DEPTH>
+__device__ __forceinline__ void filter_add(FilterPixel<DIFF, DEPTH>& P, const FilterTap& q, float a, float w) {
+  const float f = w * cpt_exp_neg(a);
+  P.t0 = __builtin_fmaf(f, q.c[0], P.t0);
+  P.t1 = __builtin_fmaf(f, q.c[1], P.t1);
+  P.t2 = __builtin_fmaf(f, q.c[2], P.t2);
+  P.sum = P.sum + f;
+}
+// A tap of exponent past 103 weighs exactly 0 and adds nothing to finite sums;
+// infinite exponents (infinite guides) are left to the arithmetic.
+__device__ __forceinline__ bool filter_zero(float a) { return a > 103.f && a < __builtin_huge_valf(); }
+template <bool DIFF, bool DEPTH>
+__device__ __forceinline__ void filter_store(const FilterArgs& fa, const FilterPixel<DIFF, DEPTH>& P, uint32_t x,
+                                             uint32_t y, const uint32_t* __restrict__ sample_n,
+                                             float* __restrict__ filtered, float* __restrict__ err) {
+  const size_t ind = (size_t)y * fa.width + x;
+  const float o0 = P.t0 / P.sum, o1 = P.t1 / P.sum, o2 = P.t2 / P.sum;
   filtered[ind * 3] = o0;
   filtered[ind * 3 + 1] = o1;
   filtered[ind * 3 + 2] = o2;
   // pt_calculateSquareError_kernel (AdapBilatAtomic.cu:1143-1156)
-  uint32_t sn_ = sample_n[ind];
-  float red = (float)fa.nd / (float)(fa.nd + sn_);
-  if (fa.nd + sn_ < sn_) red = 0.f;
-  float d0 = o0 - cc[0], d1 = o1 - cc[1], d2 = o2 - cc[2];
+  const uint32_t sn = sample_n[ind];
+  float red = (float)fa.nd / (float)(fa.nd + sn);
+  if (fa.nd + sn < sn) red = 0.f;
+  const float d0 = o0 - P.c[0], d1 = o1 - P.c[1], d2 = o2 - P.c[2];
   err[ind] = red * ((d0 * d0 + d1 * d1) + d2 * d2) / 3.f;
+}
+template <bool DIFF, bool DEPTH>
+__device__ __forceinline__ void filter_start(FilterPixel<DIFF, DEPTH>& P, const FilterTap& q) {
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    P.c[c] = q.c[c]; P.p[c] = q.p[c]; P.n[c] = q.n[c];
+    P.d[c] = DIFF ? q.d[c] : 0.f;
+  }
+  P.z = DEPTH ? q.z : 0.f;
+  P.iz = P.z > 0.f ? 1.f / P.z : 0.f;
+  P.sum = P.t0 = P.t1 = P.t2 = 0.f;
+}
+__device__ __forceinline__ FilterScale filter_scale(const FilterArgs& fa, bool depth) {
+  return {1.f / fa.kc, 1.f / fa.kp, 1.f / fa.kn, 1.f / fa.kd, depth ? 1.f / fa.kz : 0.f};
+}
+
+// A 16 x 16 tile a workgroup.  Bound by the arithmetic of the taps (48 instructions each with
+// the albedo guide; the SIMDs' every cycle is taken), so what is not arithmetic is
+// kept small: the halo of (16 + 2R)^2 pixels lies in LDS as records
+// of 12 words, read as 128-bit words that no two lanes of a 16-lane group
+// share a bank for; the products of the spatial weights are tabled; the depth term is
+// its own instance; a tap that weighs 0 in the whole wave ends early.  1920 x 1080,
+// radius 5, with / without the albedo guide: 280 / 244 us; planes of single words,
+// weights multiplied per tap and a depth branch took 381 / 305 (71 instructions a tap),
+// at radius 7 735 / 558 against 524 / 467.  Two pixels of a column a thread, which share each
+// record, 279 / 242 and 572 / 517: twice the LDS leaves half the waves.
+template <bool DIFF, bool DEPTH>
+__global__ __launch_bounds__(kTile * kTile) void k_filter_lds(FilterArgs fa, const float* __restrict__ color,
+                                                              const float* __restrict__ gpos,
+                                                              const float* __restrict__ gnrm,
+                                                              const float* __restrict__ gdif,
+                                                              const uint32_t* __restrict__ sample_n,
+                                                              float* __restrict__ filtered, float* __restrict__ err) {
+  extern __shared__ float4 sm[];
+  const int R = (int)fa.radius, D = 2 * R + 1, TW = kTile + 2 * R, TA = TW * TW;
+  const uint32_t W = fa.width, H = fa.height;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * kTile + tx;
+  const int bx = blockIdx.x * kTile, by = blockIdx.y * kTile;
+  float* rec = (float*)sm;                         // c, p, n, then d or (z, -, -)
+  float* wt = rec + 12 * (size_t)TA;               // spatial weight of tap (i, j)
+  float* sz = wt + (size_t)D * D;                  // depth per halo pixel (DIFF && DEPTH)
+  const float cam[3] = {fa.cam[0], fa.cam[1], fa.cam[2]};
+  for (int k = tid; k < D * D; k += kTile * kTile) {
+    const int i = k / D, j = k - i * D;
+    wt[k] = fa.gauss[i] * fa.gauss[j];
+  }
+  for (int k = tid; k < TA; k += kTile * kTile) {
+    const int hy = k / TW, hx = k - hy * TW;
+    const size_t g = ((size_t)ref_clamp_i(by + hy - R, H) * W + ref_clamp_i(bx + hx - R, W)) * 3;
+    float* r = rec + 12 * k;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      r[c] = color[g + c];
+      r[3 + c] = gpos[g + c];
+      r[6 + c] = gnrm[g + c];
+      if (DIFF) r[9 + c] = gdif[g + c];
+    }
+    if (DEPTH) {
+      const float z = sqrtf(sqdist3(gpos + g, cam));
+      if (DIFF) sz[k] = z; else r[9] = z;
+    }
+  }
+  __syncthreads();
+  const auto load = [&](int k) {
+    FilterTap q;
+    const float4* r = (const float4*)(rec + 12 * k);
+    const float4 a = r[0], b = r[1], c = r[2];
+    q.c[0] = a.x; q.c[1] = a.y; q.c[2] = a.z;
+    q.p[0] = a.w; q.p[1] = b.x; q.p[2] = b.y;
+    q.n[0] = b.z; q.n[1] = b.w; q.n[2] = c.x;
+    q.d[0] = c.y; q.d[1] = c.z; q.d[2] = c.w;
+    q.z = DEPTH ? (DIFF ? sz[k] : c.y) : 0.f;
+    return q;
+  };
+  const FilterScale ks = filter_scale(fa, DEPTH);
+  const uint32_t x = bx + tx, y = by + ty;
+  FilterPixel<DIFF, DEPTH> P;
+  filter_start(P, load((ty + R) * TW + tx + R));
+  for (int i = 0; i < D; i++) {
+    const int row = (ty + i) * TW + tx;
+    for (int j = 0; j < D; j++) {
+      const FilterTap q = load(row + j);
+      const float a = filter_exponent(P, q, ks);
+      if (__ballot(!filter_zero(a)) == 0ull) continue;
+      filter_add(P, q, a, wt[i * D + j]);
+    }
+  }
+  if (x < W && y < H) filter_store(fa, P, x, y, sample_n, filtered, err);
+}
+
+// Radii whose halo does not fit: every tap read from memory.
+template <bool DIFF, bool DEPTH>
+__global__ __launch_bounds__(kTile * kTile) void k_filter_mem(FilterArgs fa, const float* __restrict__ color,
+                                                              const float* __restrict__ gpos,
+                                                              const float* __restrict__ gnrm,
+                                                              const float* __restrict__ gdif,
+                                                              const uint32_t* __restrict__ sample_n,
+                                                              float* __restrict__ filtered, float* __restrict__ err) {
+  __shared__ float sg[2 * kMaxFilterRadius + 2];
+  const int R = (int)fa.radius;
+  const uint32_t W = fa.width, H = fa.height;
+  const int tid = threadIdx.y * kTile + threadIdx.x;
+  const uint32_t x = blockIdx.x * kTile + threadIdx.x, y = blockIdx.y * kTile + threadIdx.y;
+  const float cam[3] = {fa.cam[0], fa.cam[1], fa.cam[2]};
+  if (tid < 2 * R + 1) sg[tid] = fa.gauss[tid];
+  __syncthreads();
+  if (x >= W || y >= H) return;
+  const auto load = [&](int yy, int xx) {
+    const size_t g = ((size_t)ref_clamp_i(yy, H) * W + ref_clamp_i(xx, W)) * 3;
+    FilterTap q;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      q.c[c] = color[g + c]; q.p[c] = gpos[g + c]; q.n[c] = gnrm[g + c];
+      q.d[c] = DIFF ? gdif[g + c] : 0.f;
+    }
+    q.z = DEPTH ? sqrtf(sqdist3(gpos + g, cam)) : 0.f;
+    return q;
+  };
+  const FilterScale ks = filter_scale(fa, DEPTH);
+  FilterPixel<DIFF, DEPTH> P;
+  filter_start(P, load((int)y, (int)x));
+  for (int i = -R; i <= R; i++)
+    for (int j = -R; j <= R; j++) {
+      const FilterTap q = load((int)y + i, (int)x + j);
+      filter_add(P, q, filter_exponent(P, q, ks), sg[i + R] * sg[j + R]);
+    }
+  filter_store(fa, P, x, y, sample_n, filtered, err);
 }
 
 hipError_t launch_filter_error(const FilterArgs& fa, const float* color, const float* gpos, const float* gnrm,
-                               const float* gdif, const float* gauss, const uint32_t* sample_n, float* filtered,
-                               float* err, hipStream_t st) {
-  if (!color || !gpos || !gnrm || !gauss || !sample_n || !filtered || !err || (fa.use_diff && !gdif) ||
+                               const float* gdif, const uint32_t* sample_n, float* filtered, float* err,
+                               hipStream_t st) {
+  if (!color || !gpos || !gnrm || !sample_n || !filtered || !err || (fa.use_diff && !gdif) ||
       (int)fa.radius > kMaxFilterRadius || fa.width == 0 || fa.height == 0)
     return hipErrorInvalidValue;
-  dim3 block(kTile, kTile), grid((fa.width + kTile - 1) / kTile, (fa.height + kTile - 1) / kTile);
-  const bool lds = (int)fa.radius <= kLdsRadius;
-  const int TW = kTile + 2 * (int)fa.radius;
-  size_t bytes = sizeof(float) * (2 * kMaxFilterRadius + 2);
-  if (lds) bytes += sizeof(float) * TW * TW * (3 * (fa.use_diff ? 4 : 3) + (fa.kz > 0.f ? 1 : 0));
-  if (fa.use_diff) {
-    if (lds) k_filter_error<true, true><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, gauss, sample_n, filtered, err);
-    else k_filter_error<true, false><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, gauss, sample_n, filtered, err);
-  } else {
-    if (lds) k_filter_error<false, true><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, gauss, sample_n, filtered, err);
-    else k_filter_error<false, false><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, gauss, sample_n, filtered, err);
+  const int R = (int)fa.radius, D = 2 * R + 1;
+  const bool depth = fa.kz > 0.f, diff = fa.use_diff != 0;
+  const dim3 block(kTile, kTile), grid((fa.width + kTile - 1) / kTile, (fa.height + kTile - 1) / kTile);
+  const int TA = (kTile + 2 * R) * (kTile + 2 * R);
+  const size_t bytes = sizeof(float) * (12 * (size_t)TA + (size_t)D * D + (diff && depth ? TA : 0));
+#define CPT_FILTER(DI, DE)                                                                                      \
+  {                                                                                                             \
+    if (R > kLdsRadius)                                                                                         \
+      k_filter_mem<DI, DE><<<grid, block, 0, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered, err);       \
+    else                                                                                                        \
+      k_filter_lds<DI, DE><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered, err);   \
   }
+  if (diff) {
+    if (depth) CPT_FILTER(true, true) else CPT_FILTER(true, false)
+  } else {
+    if (depth) CPT_FILTER(false, true) else CPT_FILTER(false, false)
+  }
+#undef CPT_FILTER
   return hipGetLastError();
 }
 
