@@ -5,7 +5,7 @@
 // filter-residual error of the adaptive renderer
 // (src/cudaRTBDPTStreamAdapBilatAtomic.cu:1143-1156) as the allocation signal.
 //
-// Training: a workgroup of four waves; each wave takes 64 pixels at a time
+// Training: a workgroup of eight waves; each wave takes 32 pixels at a time
 // and keeps the layer activations in registers between layers (the k-permuted
 // operand scheme below), accumulating its weight gradients over its chunks in
 // MFMA accumulators:
@@ -26,11 +26,19 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// float -> bf16 with round-to-nearest-even (finite inputs).
-__device__ __forceinline__ uint16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+// float -> bf16, round-to-nearest-even (v_cvt_pk_bf16_f32).
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+// Four values, as half of an MFMA operand: a conversion of two takes one instruction.
+__device__ __forceinline__ s16x4 f2bf4(float a, float b, float c, float d) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const uint2 u = {__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2)),
+                   __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{c, d}, bf16x2))};
+  return __builtin_bit_cast(s16x4, u);
+}
+__device__ __forceinline__ bf16x8 join8(s16x4 lo, s16x4 hi) {
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
@@ -88,7 +96,7 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-constexpr int kTrainWaves = 4;                  // waves per training workgroup
+constexpr int kTrainWaves = 8;                  // waves per training workgroup: two a SIMD
 // Training takes 32 pixels per wave at a time (two pixel blocks): the
 // activations of a chunk then fit the register file next to the
 // weight-gradient accumulators; the weight gradients contract over the
@@ -104,7 +112,6 @@ struct MlpWaveLds {
   alignas(16) uint16_t xt[16 * kPlaneStride];    // X^T  [feature][pixel] (features 9..15 zero)
   alignas(16) uint16_t h1t[64 * kPlaneStride];   // H1^T [hidden][pixel], then dZ1^T
   alignas(16) uint16_t dz2t[64 * kPlaneStride];  // dZ2^T [out][pixel]
-  float vec[3][64];                             // dW3, db2, db1 summed over the wave's chunks
 };
 // Weight operands and vectors, shared by the workgroup's waves.
 struct MlpWeightLds {
@@ -113,13 +120,19 @@ struct MlpWeightLds {
   alignas(16) uint16_t w2f[kMlpW2Frag];
   float b1[64], b2[64], w3[64];
 };
-struct MlpTrainLds {
-  MlpWeightLds w;
-  union {
+constexpr int kRedStride = (kMlpParams + 1 + 63) / 64 * 64;      // the loss after the parameters
+union MlpTrainLds {
+  struct {
+    MlpWeightLds w;
     MlpWaveLds wave[kTrainWaves];
-    float red[kMlpParams + 3];                  // the workgroup's gradient, summed wave by wave
-  } u;
+  } f;
+  float red[kTrainWaves][kRedStride];           // the waves' gradients
 };
+static_assert(sizeof(MlpTrainLds) <= 160 * 1024, "a compute unit's LDS");
+// Word of parameter p in red: rows of 64 rotated by 16 words every four rows, so
+// that the four lane groups' stores of one MFMA result (rows 4 apart) fall in
+// different banks.
+__device__ __forceinline__ int red_word(int p) { return (p & ~63) | ((p + ((p >> 8) & 3) * 16) & 63); }
 
 template <bool TRAIN>
 __device__ __forceinline__ void stage_weights(MlpWeightLds& s, const MlpDevWeights& w, int tid, int nthreads) {
@@ -140,12 +153,13 @@ __device__ __forceinline__ void load_x(s16x4 xb[PB], const float* __restrict__ x
 #pragma unroll
   for (int pb = 0; pb < PB; pb++) {
     const uint32_t px = base + pb * 16 + c;
+    float v[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const int f = g * 4 + j;
-      const float v = (f < kMlpIn && px < n) ? x[(size_t)px * kMlpIn + f] : 0.f;
-      xb[pb][j] = (short)f2bf(v);
+      v[j] = (f < kMlpIn && px < n) ? x[(size_t)px * kMlpIn + f] : 0.f;
     }
+    xb[pb] = f2bf4(v[0], v[1], v[2], v[3]);
   }
 }
 
@@ -168,38 +182,57 @@ typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
 // Keeps the scheduler from hoisting the next tile's loads and MFMAs above the
 // current tile's element work: with every tile in flight at once the live
 // set exceeds the register file.
-__device__ __forceinline__ void tile_fence() { __builtin_amdgcn_sched_barrier(0); }
-// Sums v over the 16 pixel lanes of each lane group and adds it to acc[unit]
-// (lane c == 0 of each group writes its four units).
-__device__ __forceinline__ void add_unit_sums(float* acc, float v[4][4], int g, int c, bool first) {
+// No operand is kept in a register over it to be used again either.
+__device__ __forceinline__ void tile_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+// Computes v here: without this the compiler moves the arithmetic past the next
+// branch to v's use and keeps its unpacked inputs in registers instead.
+__device__ __forceinline__ void settle(h16x2& v) {
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  asm volatile("" : "+v"(u));
+  v = __builtin_bit_cast(h16x2, u);
+}
+// Adds to acc, of lane (g, c), the sum over the 16 pixel lanes of its group of unit
+// 16 (c / 4) + 4 g + c % 4, if that is one of block b's (v: the lane's four
+// units of the block).  Within the registers: as ds_bpermute the 192 exchanges of a
+// chunk took a third of its LDS instructions.
+__device__ __forceinline__ void add_unit_sums(float& acc, const float v[4], int b, int c) {
 #pragma unroll
-  for (int b = 0; b < 4; b++)
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      float t = v[b][e];
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) t += __shfl_xor(t, o, 64);
-      if (c == 0) {
-        const int u = b * 16 + g * 4 + e;
-        acc[u] = first ? t : acc[u] + t;
-      }
-    }
+  for (int e = 0; e < 4; e++) {
+    float t = v[e];
+    t += dpp_f<0xB1>(t);                                // lane ^ 1
+    t += dpp_f<0x4E>(t);                                // lane ^ 2
+    t += dpp_f<0x141>(t);                               // lane ^ 7: the other quad, whose lanes are equal
+    t += dpp_f<0x140>(t);                               // lane ^ 15: the other eight
+    acc += c == 4 * b + e ? t : 0.f;
+  }
 }
 
-__global__ __launch_bounds__(64 * kTrainWaves, 1) void k_mlp_train(MlpDevWeights w, const float* __restrict__ x,
+// Bound by latency: a wave's chain of MFMA, exponential, LDS round trip through
+// five layers' products, 2,000 VALU instructions a chunk.  So two waves a SIMD (209
+// VGPRs; one wave with 344 left it idle 65 % of the time), unit sums within the
+// registers, and a workgroup's gradients summed by all its threads at once instead
+// of wave after wave.  65,536 pixels: 20.9 us, 41.8 before; a batch of 500 with its Adam
+// step 16.5 us, 30.3 before.
+__global__ __launch_bounds__(64 * kTrainWaves, 2) void k_mlp_train(MlpDevWeights w, const float* __restrict__ x,
                                                                    const float* __restrict__ target, uint32_t n,
                                                                    float inv_batch, float* __restrict__ part,
                                                                    float* __restrict__ loss_part) {
   __shared__ MlpTrainLds s;
   const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, g = l >> 4, c = l & 15;
-  stage_weights<true>(s.w, w, tid, 64 * kTrainWaves);
-  for (int i = l; i < 3 * 64; i += 64) s.u.wave[wave].vec[i / 64][i % 64] = 0.f;
+  stage_weights<true>(s.f.w, w, tid, 64 * kTrainWaves);
   __syncthreads();
   const float b3 = w.b3[0];
-  MlpWaveLds& L = s.u.wave[wave];
+  MlpWaveLds& L = s.f.wave[wave];
   // weight-gradient accumulators over the wave's chunks (MFMA accumulators)
   f32x4 aw2[4][4], aw1[4];
-  float ab3 = 0.f, aloss = 0.f;
+  float ab3 = 0.f, aloss = 0.f, vw3 = 0.f, vb2 = 0.f, vb1 = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     aw1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -208,7 +241,9 @@ __global__ __launch_bounds__(64 * kTrainWaves, 1) void k_mlp_train(MlpDevWeights
   }
   constexpr int PB = kTrainPB, C = kTrainChunk, S = kPlaneStride;
   const uint32_t nchunks = (n + C - 1) / C;
-  for (uint32_t ch = blockIdx.x * kTrainWaves + wave; ch < nchunks; ch += gridDim.x * kTrainWaves) {
+  // chunk by chunk over the workgroups first: a small batch takes one wave of many
+  for (uint32_t ch = blockIdx.x + gridDim.x * wave; ch < nchunks; ch += gridDim.x * kTrainWaves) {
+    asm volatile("" ::: "memory");                         // the weights are read again, not kept in registers
     const uint32_t base = ch * C;
     s16x4 xb[PB];
     load_x<PB>(xb, x, base, n, g, c);
@@ -220,42 +255,50 @@ __global__ __launch_bounds__(64 * kTrainWaves, 1) void k_mlp_train(MlpDevWeights
     bf16x8 hk[2][PB];                                      // H1^T as layer-2 B operands
     h16x2 dg1[4][PB][2];
 #pragma unroll
-    for (int hb = 0; hb < 4; hb++)
+    for (int hb = 0; hb < 4; hb++) {
 #pragma unroll
       for (int pb = 0; pb < PB; pb++) {
-        const f32x4 z = layer1_tile(s.w.w1f, hb, xb[pb], l);
+        const f32x4 z = layer1_tile(s.f.w.w1f, hb, xb[pb], l);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const int u = hb * 16 + g * 4 + e;
           float gv, dg;
-          gelu_fwd(z[e] + s.w.b1[u], gv, dg);
+          gelu_fwd(z[e] + s.f.w.b1[u], gv, dg);
           dg1[hb][pb][e >> 1][e & 1] = (_Float16)dg;
           const uint16_t hbits = f2bf(gv);
           hk[hb >> 1][pb][(hb & 1) * 4 + e] = as_bf(hbits);
           L.h1t[u * S + pb * 16 + c] = hbits;
         }
-        tile_fence();
+        settle(dg1[hb][pb][0]);
+        settle(dg1[hb][pb][1]);
       }
+      tile_fence();
+    }
     h16x2 h2[4][PB][2], dg2[4][PB][2];
     float ys[PB];
 #pragma unroll
     for (int pb = 0; pb < PB; pb++) ys[pb] = 0.f;
 #pragma unroll
-    for (int ob = 0; ob < 4; ob++)
+    for (int ob = 0; ob < 4; ob++) {
 #pragma unroll
       for (int pb = 0; pb < PB; pb++) {
-        const f32x4 z = layer64_tile<PB>(s.w.w2tf, ob, pb, hk, l);  // Z2^T
+        const f32x4 z = layer64_tile<PB>(s.f.w.w2tf, ob, pb, hk, l);  // Z2^T
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const int u = ob * 16 + g * 4 + e;
           float gv, dg;
-          gelu_fwd(z[e] + s.w.b2[u], gv, dg);
+          gelu_fwd(z[e] + s.f.w.b2[u], gv, dg);
           h2[ob][pb][e >> 1][e & 1] = (_Float16)gv;
           dg2[ob][pb][e >> 1][e & 1] = (_Float16)dg;
-          ys[pb] = fmaf(gv, s.w.w3[u], ys[pb]);
+          ys[pb] = fmaf(gv, s.f.w.w3[u], ys[pb]);
         }
-        tile_fence();
+        for (int q = 0; q < 2; q++) {
+          settle(h2[ob][pb][q]);
+          settle(dg2[ob][pb][q]);
+        }
       }
+      tile_fence();
+    }
     float dy[PB];
 #pragma unroll
     for (int pb = 0; pb < PB; pb++) {
@@ -271,27 +314,28 @@ __global__ __launch_bounds__(64 * kTrainWaves, 1) void k_mlp_train(MlpDevWeights
     }
     // ---- backward
     bf16x8 dk[2][PB];                                      // dZ2^T as B operands
-    float v3[4][4], v2[4][4];
 #pragma unroll
-    for (int ob = 0; ob < 4; ob++)
+    for (int ob = 0; ob < 4; ob++) {
+      float v3[4], v2[4];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int u = ob * 16 + g * 4 + e;
-        const float w3u = s.w.w3[u];
-        v3[ob][e] = v2[ob][e] = 0.f;
+        const float w3u = s.f.w.w3[u];
+        v3[e] = v2[e] = 0.f;
 #pragma unroll
         for (int pb = 0; pb < PB; pb++) {
-          v3[ob][e] = fmaf((float)h2[ob][pb][e >> 1][e & 1], dy[pb], v3[ob][e]);
+          v3[e] = fmaf((float)h2[ob][pb][e >> 1][e & 1], dy[pb], v3[e]);
           const float dz = dy[pb] * w3u * (float)dg2[ob][pb][e >> 1][e & 1];
-          v2[ob][e] += dz;
+          v2[e] += dz;
           const uint16_t bits = f2bf(dz);
           dk[ob >> 1][pb][(ob & 1) * 4 + e] = as_bf(bits);
           L.dz2t[u * S + pb * 16 + c] = bits;
         }
-        tile_fence();
       }
-    add_unit_sums(L.vec[0], v3, g, c, false);
-    add_unit_sums(L.vec[1], v2, g, c, false);
+      add_unit_sums(vw3, v3, ob, c);
+      add_unit_sums(vb2, v2, ob, c);
+      tile_fence();
+    }
     wave_lds_sync();
     // dW2[in][out] += H1^T . dZ2 over the chunk's pixels
 #pragma unroll
@@ -308,25 +352,23 @@ __global__ __launch_bounds__(64 * kTrainWaves, 1) void k_mlp_train(MlpDevWeights
     }
     wave_lds_sync();                                       // H1^T reads done: dZ1^T takes its place
     // dH1^T = W2 . dZ2^T; dZ1 = dH1 * gelu'(Z1)
-    float v1[4][4];
 #pragma unroll
     for (int ib = 0; ib < 4; ib++) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) v1[ib][e] = 0.f;
+      float v1[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int pb = 0; pb < PB; pb++) {
-        const f32x4 dh = layer64_tile<PB>(s.w.w2f, ib, pb, dk, l);
+        const f32x4 dh = layer64_tile<PB>(s.f.w.w2f, ib, pb, dk, l);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const int u = ib * 16 + g * 4 + e;
           const float dz = dh[e] * (float)dg1[ib][pb][e >> 1][e & 1];
-          v1[ib][e] += dz;
+          v1[e] += dz;
           L.h1t[u * S + pb * 16 + c] = f2bf(dz);
         }
-        tile_fence();
       }
+      add_unit_sums(vb1, v1, ib, c);
+      tile_fence();
     }
-    add_unit_sums(L.vec[2], v1, g, c, false);
     wave_lds_sync();
     // dW1[feature][hidden] += X^T . dZ1 over the chunk's pixels
 #pragma unroll
@@ -342,54 +384,61 @@ __global__ __launch_bounds__(64 * kTrainWaves, 1) void k_mlp_train(MlpDevWeights
     ab3 += __shfl_xor(ab3, o, 64);
     aloss += __shfl_xor(aloss, o, 64);
   }
-  // per-unit vectors of the wave into registers before the planes are reused
-  const float vw3 = L.vec[0][l], vb2 = L.vec[1][l], vb1 = L.vec[2][l];
-  __syncthreads();                                         // every wave's planes are dead: red takes them
-  // the workgroup's gradient: waves add theirs in order
-  for (int wv = 0; wv < kTrainWaves; wv++) {
-    if (wave == wv) {
-      auto put = [&](int p, float v) { s.u.red[p] = wv == 0 ? v : s.u.red[p] + v; };
+  // waves that had a chunk: at least the first
+  const int waves = (int)min((nchunks - blockIdx.x + gridDim.x - 1) / gridDim.x, (uint32_t)kTrainWaves);
+  __syncthreads();                                         // weights and planes are dead: red takes their place
+  if (wave < waves) {
+    float* red = s.red[wave];
+    auto put = [&](int p, float v) { red[red_word(p)] = v; };
 #pragma unroll
-      for (int ib = 0; ib < 4; ib++)
+    for (int ib = 0; ib < 4; ib++)
 #pragma unroll
-        for (int ob = 0; ob < 4; ob++)
+      for (int ob = 0; ob < 4; ob++)
 #pragma unroll
-          for (int e = 0; e < 4; e++) put(kMlpOffW2 + (ib * 16 + g * 4 + e) * 64 + ob * 16 + c, aw2[ib][ob][e]);
+        for (int e = 0; e < 4; e++) put(kMlpOffW2 + (ib * 16 + g * 4 + e) * 64 + ob * 16 + c, aw2[ib][ob][e]);
 #pragma unroll
-      for (int hb = 0; hb < 4; hb++)
+    for (int hb = 0; hb < 4; hb++)
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          if (g * 4 + e < kMlpIn) put(kMlpOffW1 + (g * 4 + e) * 64 + hb * 16 + c, aw1[hb][e]);
-      put(kMlpOffW3 + l, vw3);
-      put(kMlpOffB2 + l, vb2);
-      put(kMlpOffB1 + l, vb1);
-      if (l == 0) {
-        put(kMlpOffB3, ab3);
-        put(kMlpParams, aloss);
-      }
+      for (int e = 0; e < 4; e++)
+        if (g * 4 + e < kMlpIn) put(kMlpOffW1 + (g * 4 + e) * 64 + hb * 16 + c, aw1[hb][e]);
+    const int u = (c >> 2) * 16 + g * 4 + (c & 3);
+    put(kMlpOffW3 + u, vw3);
+    put(kMlpOffB2 + u, vb2);
+    put(kMlpOffB1 + u, vb1);
+    if (l == 0) {
+      put(kMlpOffB3, ab3);
+      put(kMlpParams, aloss);
     }
-    __syncthreads();
   }
+  __syncthreads();
+  // the workgroup's gradient: waves added in order
   float* P = part + (size_t)blockIdx.x * kMlpParams;
-  for (int p = tid; p < kMlpParams; p += 64 * kTrainWaves) P[p] = s.u.red[p];
-  if (tid == 0) loss_part[blockIdx.x] = s.u.red[kMlpParams];
+  for (int p = tid; p <= kMlpParams; p += 64 * kTrainWaves) {
+    const int q = red_word(p);
+    float v = s.red[0][q];
+    for (int wv = 1; wv < waves; wv++) v += s.red[wv][q];
+    if (p < kMlpParams) P[p] = v;
+    else loss_part[blockIdx.x] = v;
+  }
 }
 
 // Inference: a wave takes chunks of 16 * kInferBlocks pixels; kInferMinWaves
-// waves per SIMD bound its registers (115 of 128, no spills).
-constexpr int kInferBlocks = 4, kInferMinWaves = 4;
+// waves per SIMD bound its registers (115 of 128, no spills).  Bound by the VALU: of about
+// 2,040 issue slots a chunk half are the 256 exponentials and reciprocals; with the
+// roundings to BF16 two at a time 2,073,600 pixels take 102 us, by hand 113.7.
+constexpr int kInferBlocks = 4, kInferMinWaves = 4, kInferWaves = 4;
 constexpr uint32_t kInferMaxGroups = 2048;
-__global__ __launch_bounds__(64 * kTrainWaves, kInferMinWaves) void k_mlp_infer(MlpDevWeights w,
+__global__ __launch_bounds__(64 * kInferWaves, kInferMinWaves) void k_mlp_infer(MlpDevWeights w,
                                                                                const float* __restrict__ x,
                                                                                uint32_t n, float* __restrict__ y) {
   constexpr int PB = kInferBlocks;
   __shared__ MlpWeightLds s;
   const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, g = l >> 4, c = l & 15;
-  stage_weights<false>(s, w, tid, 64 * kTrainWaves);
+  stage_weights<false>(s, w, tid, 64 * kInferWaves);
   __syncthreads();
   const float b3 = w.b3[0];
   const uint32_t nchunks = (n + 16 * PB - 1) / (16 * PB);
-  for (uint32_t ch = blockIdx.x * kTrainWaves + wave; ch < nchunks; ch += gridDim.x * kTrainWaves) {
+  for (uint32_t ch = blockIdx.x * kInferWaves + wave; ch < nchunks; ch += gridDim.x * kInferWaves) {
     // the weights are read from LDS again for every chunk: held in registers
     // across chunks they would take about 90 of them and halve the waves
     asm volatile("" ::: "memory");
@@ -398,13 +447,20 @@ __global__ __launch_bounds__(64 * kTrainWaves, kInferMinWaves) void k_mlp_infer(
     load_x<PB>(xb, x, base, n, g, c);
     bf16x8 hk[2][PB];
 #pragma unroll
-    for (int hb = 0; hb < 4; hb++)
+    for (int kb = 0; kb < 2; kb++)
 #pragma unroll
       for (int pb = 0; pb < PB; pb++) {
-        const f32x4 z = layer1_tile(s.w1f, hb, xb[pb], l);
+        s16x4 half[2];
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          hk[hb >> 1][pb][(hb & 1) * 4 + e] = as_bf(f2bf(gelu_val(z[e] + s.b1[hb * 16 + g * 4 + e])));
+        for (int q = 0; q < 2; q++) {
+          const int hb = 2 * kb + q;
+          const f32x4 z = layer1_tile(s.w1f, hb, xb[pb], l);
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[e] = gelu_val(z[e] + s.b1[hb * 16 + g * 4 + e]);
+          half[q] = f2bf4(v[0], v[1], v[2], v[3]);
+        }
+        hk[kb][pb] = join8(half[0], half[1]);
       }
     float ys[PB];
 #pragma unroll
@@ -516,8 +572,7 @@ __global__ __launch_bounds__(kAdamParams * kAdamGroups) void k_mlp_adam(
 
 uint32_t mlp_train_groups(uint32_t n) {
   const uint32_t chunks = (n + kTrainChunk - 1) / kTrainChunk;
-  const uint32_t g = (chunks + kTrainWaves - 1) / kTrainWaves;
-  return g < kMlpMaxTrainGroups ? g : kMlpMaxTrainGroups;
+  return chunks < kMlpMaxTrainGroups ? chunks : kMlpMaxTrainGroups;
 }
 
 hipError_t launch_mlp_train(const MlpState& st, const float* x, const float* t, uint32_t n, float* part,
@@ -539,9 +594,9 @@ hipError_t launch_mlp_infer(const MlpState& st, const float* x, uint32_t n, floa
   if (!x || !y) return hipErrorInvalidValue;
   if (n == 0) return hipSuccess;
   const uint32_t chunks = (n + 16 * kInferBlocks - 1) / (16 * kInferBlocks);
-  uint32_t grid = (chunks + kTrainWaves - 1) / kTrainWaves;
+  uint32_t grid = (chunks + kInferWaves - 1) / kInferWaves;
   if (grid > kInferMaxGroups) grid = kInferMaxGroups;
-  k_mlp_infer<<<grid, 64 * kTrainWaves, 0, s>>>(st.dev, x, n, y);
+  k_mlp_infer<<<grid, 64 * kInferWaves, 0, s>>>(st.dev, x, n, y);
   return hipGetLastError();
 }
 __global__ void k_mlp_pack(MlpState st) {
