@@ -904,9 +904,9 @@ int renderer_alloc(cpt_renderer* r) {
     HIP_TRY(r->sq.alloc(n * 3));
     HIP_TRY(r->flags.alloc(n));
     HIP_TRY(r->rank.alloc(n));
-    HIP_TRY(r->rounds.alloc(1));
+    HIP_TRY(r->rounds.alloc(2));
     HIP_TRY(r->maxe.alloc(1));
-    HIP_TRY(r->kept.alloc(1));
+    HIP_TRY(r->kept.alloc(3 * (size_t)kKeptSlots * kDealStride));
     HIP_TRY(r->gnrm.alloc(n * 3));
     HIP_TRY(r->gdif.alloc(n * 3));
     HIP_TRY(r->filtered.alloc(n * 3));
@@ -1223,30 +1223,39 @@ int model_features(cpt_renderer* r, float* d_x) {
 
 // Round-based sample allocation into r->counts / r->offsets / r->total:
 // window bisection (AdapBilatBinary) or window = max error (AdapEmp).  Rounds
-// run on the device in batches; the host reads the done flag between batches.
+// run on the device in batches, a launch each and one that closes the batch's
+// last; the host reads the done flag between batches.
 // After kMaxRounds rounds the remaining slots are filled as the reference's
 // fill kernel does.
 constexpr u32 kMaxRounds = 1024;
-constexpr u32 kRoundBatch = 8;
+// A frame takes 15 to 60 rounds: batches of 8 / 16 / 32 take 10.3 / 9.8 / 9.4 ms for 12
+// empirical frames of 800 x 600 on the sphere grid, 20.7 / 20.7 / 21.2 for bisected
+// ones of 1920 x 1080 on the heightfield (rounds past the end cost a launch each).
+constexpr u32 kRoundBatch = 16;
+static_assert(kMaxRounds % kRoundBatch == 0, "whole batches");
 int allocate_rounds(cpt_renderer* r, const FrameArgs& fa, const float* err, u32 gen, u32 nd, u32 maxp) {
   const u32 n = r->W * r->H;
   const bool bisect = r->mode == CPT_MODE_BDPT_ADAPTIVE_BINARY;
   const float desired = (float)n / (float)(nd ? nd : 1u);
   const float min_prob = (float)r->attr("Min Trace Probability");
   HIP_TRY(launch_error_max(err, n, r->maxe.p, r->stream));
-  HIP_TRY(launch_round_init(r->rounds.p, r->maxe.p, gen, bisect ? 1u : 0u, desired, min_prob, r->counts.p, n,
-                            r->stream));
+  HIP_TRY(launch_round_init(r->rounds.p, r->kept.p, r->maxe.p, gen, bisect ? 1u : 0u, desired, min_prob, r->counts.p,
+                            n, r->stream));
+  u32 j = 0;
+  const RoundState* last = r->rounds.p;
   for (u32 done_rounds = 0; done_rounds < kMaxRounds; done_rounds += kRoundBatch) {
-    for (u32 j = 0; j < kRoundBatch; j++)
-      HIP_TRY(launch_round(fa, err, n, r->rounds.p, r->flags.p, r->rank.p, r->block_tot.p, r->kept.p, r->counts.p,
-                           r->stream));
+    for (u32 k = 0; k <= kRoundBatch; k++, j++)
+      HIP_TRY(launch_round(fa, err, n, r->rounds.p, r->kept.p, j, r->flags.p, r->counts.p, k < kRoundBatch, r->stream));
+    last = r->rounds.p + (j & 1u);
     RoundState h;
-    HIP_TRY(hipMemcpyAsync(&h, r->rounds.p, sizeof h, hipMemcpyDeviceToHost, r->stream));
+    HIP_TRY(hipMemcpyAsync(&h, last, sizeof h, hipMemcpyDeviceToHost, r->stream));
     HIP_TRY(hipStreamSynchronize(r->stream));
     r->last_rounds = h.rounds;
+    if (h.status == kRoundPartial)
+      HIP_TRY(launch_round_rest(last, r->flags.p, n, r->rank.p, r->block_tot.p, r->total.p, r->counts.p, r->stream));
     if (h.done) break;
   }
-  HIP_TRY(launch_round_fill(r->rounds.p, n, r->counts.p, r->stream));
+  HIP_TRY(launch_round_fill(last, n, r->counts.p, r->stream));
   HIP_TRY(launch_cap_counts(r->counts.p, r->paths.p, maxp, n, r->stream));
   HIP_TRY(launch_scan_counts(r->counts.p, n, r->offsets.p, r->block_tot.p, r->total.p, r->stream));
   return CPT_OK;

@@ -296,13 +296,23 @@ struct RoundState {
   uint32_t bisect;     // 1: AdapBilatBinary window bisection, 0: fixed window = max e
   float desired;       // kept pixels per round the bisection aims at
   float min_prob;
-  uint32_t pad;
+  uint32_t status;     // kRound*
+  uint32_t take;       // slots the last closed round filled
 };
-hipError_t launch_round_init(RoundState* rs, const float* maxe, uint32_t gen, uint32_t bisect, float desired,
-                             float min_prob, uint32_t* counts, uint32_t n, hipStream_t st);
-// One round: keep flags, their exclusive scan, count update, state update.
-hipError_t launch_round(const FrameArgs& fa, const float* err, uint32_t n, RoundState* rs, uint32_t* flags,
-                        uint32_t* rank, uint32_t* block_tot, uint32_t* kept, uint32_t* counts, hipStream_t st);
+// A round's kept pixels: none open, flagged but not counted yet, or more than
+// the slots left (launch_round_rest gives them out).
+constexpr uint32_t kRoundIdle = 0, kRoundPending = 1, kRoundPartial = 2;
+constexpr uint32_t kKeptSlots = 64;      // counters of a round's kept pixels, kDealStride words apart
+// rs: two states; kept: three sets of counters.
+hipError_t launch_round_init(RoundState* rs, uint32_t* kept, const float* maxe, uint32_t gen, uint32_t bisect,
+                             float desired, float min_prob, uint32_t* counts, uint32_t n, hipStream_t st);
+// Launch j (from 0): closes the round of launch j - 1 and, with keep, opens one:
+// reads state j & 1, writes the other.
+hipError_t launch_round(const FrameArgs& fa, const float* err, uint32_t n, RoundState* rs, uint32_t* kept, uint32_t j,
+                        uint32_t* flags, uint32_t* counts, int keep, hipStream_t st);
+// After a kRoundPartial state: the first rs->take kept pixels.
+hipError_t launch_round_rest(const RoundState* rs, const uint32_t* flags, uint32_t n, uint32_t* rank,
+                             uint32_t* block_tot, uint32_t* total, uint32_t* counts, hipStream_t st);
 // Unfilled slots go to pixels 0, 1, ... in order (wrapping past W*H).
 hipError_t launch_round_fill(const RoundState* rs, uint32_t n, uint32_t* counts, hipStream_t st);
 // Exclusive scan of given per-pixel counts into offsets and their total.

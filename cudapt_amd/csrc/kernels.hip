@@ -3701,19 +3701,29 @@ __global__ __launch_bounds__(kBlock) void k_error_max(const float* __restrict__ 
   for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
     m = max(m, __float_as_uint(fmaxf(e[i], 0.f)));
   for (int o = 32; o >= 1; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
-  if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+  // one atomic a workgroup, of few: on one address they take about 12 ns each
+  // (4,096 of them, one a wave of 1,024 workgroups, took 48 us)
+  __shared__ uint32_t wm[kBlock / 64];
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kBlock / 64; w++) m = max(m, wm[w]);
+    atomicMax(out, m);
+  }
 }
 hipError_t launch_error_max(const float* err, uint32_t n, float* max_out, hipStream_t st) {
   if (!err || !max_out) return hipErrorInvalidValue;
   k_fill_u32<<<1, 1, 0, st>>>((uint32_t*)max_out, 0u);
   uint32_t nb = (n + kBlock - 1) / kBlock;
-  if (nb > 1024) nb = 1024;
+  if (nb > 256) nb = 256;
   if (nb) k_error_max<<<nb, kBlock, 0, st>>>(err, n, (uint32_t*)max_out);
   return hipGetLastError();
 }
 
-__global__ void k_round_init(RoundState* rs, const float* maxe, uint32_t gen, uint32_t bisect, float desired,
-                             float min_prob) {
+__global__ void k_round_init(RoundState* rs, uint32_t* kept, const float* maxe, uint32_t gen, uint32_t bisect,
+                             float desired, float min_prob) {
+  for (uint32_t i = threadIdx.x; i < 3 * kKeptSlots; i += blockDim.x) kept[i * kDealStride] = 0u;
+  if (threadIdx.x != 0) return;
   RoundState s;
   s.maxe = *maxe;
   s.left = 0.f;
@@ -3726,50 +3736,28 @@ __global__ void k_round_init(RoundState* rs, const float* maxe, uint32_t gen, ui
   s.bisect = bisect;
   s.desired = desired;
   s.min_prob = min_prob;
-  s.pad = 0;
+  s.status = kRoundIdle;
+  s.take = 0;
   *rs = s;
 }
 __global__ __launch_bounds__(kBlock) void k_zero_u32(uint32_t* __restrict__ p, uint32_t n) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i < n) p[i] = 0u;
 }
-hipError_t launch_round_init(RoundState* rs, const float* maxe, uint32_t gen, uint32_t bisect, float desired,
-                             float min_prob, uint32_t* counts, uint32_t n, hipStream_t st) {
-  if (!rs || !maxe || !counts) return hipErrorInvalidValue;
-  k_round_init<<<1, 1, 0, st>>>(rs, maxe, gen, bisect, desired, min_prob);
+hipError_t launch_round_init(RoundState* rs, uint32_t* kept, const float* maxe, uint32_t gen, uint32_t bisect,
+                             float desired, float min_prob, uint32_t* counts, uint32_t n, hipStream_t st) {
+  if (!rs || !kept || !maxe || !counts) return hipErrorInvalidValue;
+  k_round_init<<<1, 64, 0, st>>>(rs, kept, maxe, gen, bisect, desired, min_prob);
   if (n) k_zero_u32<<<(n + kBlock - 1) / kBlock, kBlock, 0, st>>>(counts, n);
   return hipGetLastError();
 }
 
-// pt_genTempAdapPathQueue_kernel: keep unless u * window > max(e, min_prob),
-// u from the stream of (frame, slots filled so far) at the pixel.
-__global__ __launch_bounds__(kBlock) void k_round_keep(uint64_t seed, uint32_t frame, const float* __restrict__ err,
-                                                       uint32_t n, const RoundState* __restrict__ rs,
-                                                       uint32_t* __restrict__ flags) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n || rs->done) return;
-  uint64_t s = 0;
-  const uint64_t inc = ((uint64_t)i << 1) | 1u;
-  pcg32_seed(s, inc, stream_key(seed, frame, 3u, rs->accum));
-  const float u = uniform01(s, inc);
-  flags[i] = (u * rs->window > fmaxf(err[i], rs->min_prob)) ? 0u : 1u;
-}
-// Kept pixels of rank < remaining slots take one sample each.
-__global__ __launch_bounds__(kBlock) void k_round_apply(const uint32_t* __restrict__ flags,
-                                                        const uint32_t* __restrict__ rank, uint32_t n,
-                                                        const RoundState* __restrict__ rs,
-                                                        const uint32_t* __restrict__ kept,
-                                                        uint32_t* __restrict__ counts) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n || rs->done) return;
-  const uint32_t take = min(*kept, rs->gen - rs->accum);
-  if (flags[i] && rank[i] < take) counts[i] += 1u;
-}
-// remove_if + size bookkeeping + the bisection of AdapBilatBinary.cu:1363-1371.
-__global__ void k_round_update(RoundState* rs, const uint32_t* kept) {
-  RoundState s = *rs;
-  if (s.done) return;
-  const uint32_t take = min(*kept, s.gen - s.accum);
+// remove_if + size bookkeeping + the bisection of AdapBilatBinary.cu:1363-1371,
+// for the round that kept `kept` pixels.
+__device__ __forceinline__ void round_update(RoundState& s, uint32_t kept) {
+  const uint32_t take = min(kept, s.gen - s.accum);
+  s.status = take < kept ? kRoundPartial : kRoundIdle;
+  s.take = take;
   s.accum += take;
   s.rounds++;
   if (take == 0u) {
@@ -3780,7 +3768,68 @@ __global__ void k_round_update(RoundState* rs, const uint32_t* kept) {
     s.window = (s.left + s.right) * 0.5f;
   }
   if (s.accum >= s.gen) s.done = 1u;
-  *rs = s;
+}
+// One launch a round (keep = 0: only closes the last).  It closes the round
+// before: every workgroup computes the state after it from the state it ran in and its
+// kept pixels, one thread writes that for the next launch, and the kept
+// pixels take one sample each, all of them unless more were kept than slots are
+// left: that can only be the last round, whose ranks k_round_apply needs a scan for.
+// Then pt_genTempAdapPathQueue_kernel: keep unless u * window > max(e, min_prob),
+// u from the stream of (frame, slots filled so far) at the pixel; kept pixels are counted
+// in kKeptSlots counters, of three sets in turn: read, added to, cleared.
+// Six launches a round (keep, a scan of three, take, update) took 20 us, this 4.
+__global__ __launch_bounds__(kBlock) void k_round(uint64_t seed, uint32_t frame, const float* __restrict__ err,
+                                                  uint32_t n, const RoundState* __restrict__ from,
+                                                  RoundState* __restrict__ to, const uint32_t* __restrict__ kept,
+                                                  uint32_t* __restrict__ keeping, uint32_t* __restrict__ clear,
+                                                  uint32_t* __restrict__ flags, uint32_t* __restrict__ counts,
+                                                  int keep) {
+  __shared__ uint32_t total, wc[kBlock / 64];
+  RoundState s = *from;
+  const bool pending = s.status == kRoundPending;
+  if (threadIdx.x < 64) {
+    const uint32_t t = wave_sum(pending ? kept[threadIdx.x * kDealStride] : 0u);
+    if (threadIdx.x == 0) total = t;
+    if (blockIdx.x == 0) clear[threadIdx.x * kDealStride] = 0u;
+  }
+  __syncthreads();
+  if (pending) round_update(s, total);
+  const bool all = pending && s.status == kRoundIdle;
+  const bool next = keep && !s.done;
+  const float window = s.window;
+  if (next) s.status = kRoundPending;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *to = s;
+  if (!all && !next) return;
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  bool k = false;
+  if (i < n) {
+    if (all && flags[i]) counts[i] += 1u;
+    if (next) {
+      uint64_t r = 0;
+      const uint64_t inc = ((uint64_t)i << 1) | 1u;
+      pcg32_seed(r, inc, stream_key(seed, frame, 3u, s.accum));
+      const float u = uniform01(r, inc);
+      k = !(u * window > fmaxf(err[i], s.min_prob));
+      flags[i] = k ? 1u : 0u;
+    }
+  }
+  if (!next) return;
+  const uint64_t m = __ballot(k);
+  if ((threadIdx.x & 63) == 0) wc[threadIdx.x >> 6] = (uint32_t)__popcll(m);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t t = 0;
+    for (int w = 0; w < kBlock / 64; w++) t += wc[w];
+    if (t) atomicAdd(&keeping[(blockIdx.x % kKeptSlots) * kDealStride], t);
+  }
+}
+// The last round's kept pixels of rank below its slots take one sample each.
+__global__ __launch_bounds__(kBlock) void k_round_apply(const uint32_t* __restrict__ flags,
+                                                        const uint32_t* __restrict__ rank, uint32_t n,
+                                                        const RoundState* __restrict__ rs,
+                                                        uint32_t* __restrict__ counts) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < n && flags[i] && rank[i] < rs->take) counts[i] += 1u;
 }
 __global__ __launch_bounds__(kBlock) void k_round_fill(const RoundState* __restrict__ rs, uint32_t n,
                                                        uint32_t* __restrict__ counts) {
@@ -3829,15 +3878,20 @@ hipError_t launch_scan_counts(const uint32_t* counts, uint32_t n, uint32_t* offs
   if (n) k_scan_add<<<(n + kBlock - 1) / kBlock, kBlock, 0, st>>>(offsets, block_tot, n);
   return hipGetLastError();
 }
-hipError_t launch_round(const FrameArgs& fa, const float* err, uint32_t n, RoundState* rs, uint32_t* flags,
-                        uint32_t* rank, uint32_t* block_tot, uint32_t* kept, uint32_t* counts, hipStream_t st) {
-  if (!err || !rs || !flags || !rank || !block_tot || !kept || !counts || n == 0) return hipErrorInvalidValue;
-  const uint32_t g = (n + kBlock - 1) / kBlock;
-  k_round_keep<<<g, kBlock, 0, st>>>(fa.seed, fa.frame0, err, n, rs, flags);
-  hipError_t e = launch_scan_counts(flags, n, rank, block_tot, kept, st);
+hipError_t launch_round(const FrameArgs& fa, const float* err, uint32_t n, RoundState* rs, uint32_t* kept, uint32_t j,
+                        uint32_t* flags, uint32_t* counts, int keep, hipStream_t st) {
+  if (!err || !rs || !flags || !kept || !counts || n == 0) return hipErrorInvalidValue;
+  const auto set = [&](uint32_t k) { return kept + (size_t)(k % 3u) * kKeptSlots * kDealStride; };
+  k_round<<<(n + kBlock - 1) / kBlock, kBlock, 0, st>>>(fa.seed, fa.frame0, err, n, rs + (j & 1u), rs + ((j + 1u) & 1u),
+                                                        set(j), set(j + 1u), set(j + 2u), flags, counts, keep);
+  return hipGetLastError();
+}
+hipError_t launch_round_rest(const RoundState* rs, const uint32_t* flags, uint32_t n, uint32_t* rank,
+                             uint32_t* block_tot, uint32_t* total, uint32_t* counts, hipStream_t st) {
+  if (!rs || !flags || !rank || !counts || n == 0) return hipErrorInvalidValue;
+  const hipError_t e = launch_scan_counts(flags, n, rank, block_tot, total, st);
   if (e != hipSuccess) return e;
-  k_round_apply<<<g, kBlock, 0, st>>>(flags, rank, n, rs, kept, counts);
-  k_round_update<<<1, 1, 0, st>>>(rs, kept);
+  k_round_apply<<<(n + kBlock - 1) / kBlock, kBlock, 0, st>>>(flags, rank, n, rs, counts);
   return hipGetLastError();
 }
 hipError_t launch_round_fill(const RoundState* rs, uint32_t n, uint32_t* counts, hipStream_t st) {
