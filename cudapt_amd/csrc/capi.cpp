@@ -1172,8 +1172,9 @@ MlpFeatureArgs feature_args(const cpt_renderer* r, size_t off = 0, const float* 
 // (src/cudaRTBDPTStreamAdapBilatAtomic.cu:1409-1430) into r->filtered / r->err.
 // One W x H image starting at pixel `off` of the renderer's buffers, seen
 // from cam (a view of a multi-view batch; the renderer's own image: 0, W, H).
+// moment: also of the second moment, into r->sq_f / r->sq_e.
 int run_filter_at(cpt_renderer* r, size_t off, u32 W, u32 H, const float* cam, const float* src, float* dst,
-                  float* err) {
+                  float* err, bool moment = false) {
   float sc_ = (float)r->attr("Filter Color EuD"), sp_ = (float)r->attr("Filter Pos EuD");
   float sn_ = (float)r->attr("Filter Norm EuD"), sd_ = (float)r->attr("Filter Diff EuD");
   u32 radius = (u32)r->attr("Filter Radius");
@@ -1190,7 +1191,8 @@ int run_filter_at(cpt_renderer* r, size_t off, u32 W, u32 H, const float* cam, c
   }
   const size_t o3 = 3 * off;
   HIP_TRY(launch_filter_error(f, src + o3, r->gpos.p + o3, r->gnrm.p + o3, r->gdif.p + o3,
-                              r->sample_n.p + off, dst + o3, err + off, r->stream));
+                              r->sample_n.p + off, dst + o3, err + off, r->stream, moment ? r->sq.p + o3 : nullptr,
+                              moment ? r->sq_f.p + o3 : nullptr, moment ? r->sq_e.p + off : nullptr));
   return CPT_OK;
 }
 int run_filter(cpt_renderer* r, const float* src, float* dst, float* err) {
@@ -1319,14 +1321,18 @@ int render_adaptive_frame(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa, co
     int rc = CPT_OK;
     const u32 nd = (u32)r->attr("Desired Max Sampling");
     const float* alloc_err = r->err.p;
+    // the learned model's second moment goes through the filter with the image,
+    // unless a profiled renderer counts it as the model's time
+    const bool moment = r->mlp && r->mode != CPT_MODE_BDPT_ADAPTIVE_EMP && !r->profiling;
     if (r->mode == CPT_MODE_BDPT_ADAPTIVE_EMP) {    // AdapEmp.cu:1209
       HIP_TRY(timed_begin(r, 6, &ev));
       HIP_TRY(launch_emp_error(r->result.p, r->sq.p, r->sample_n.p, n, r->err.p, r->stream));
       HIP_TRY(timed_end(r, 6, ev));
     } else {
       HIP_TRY(timed_begin(r, 5, &ev));
+      if (moment && (rc = model_buffers(r))) return rc;
       for (const ViewSpan& v : views) {
-        rc = run_filter_at(r, v.off, v.W, v.H, v.cam, r->result.p, r->filtered.p, r->err.p);
+        rc = run_filter_at(r, v.off, v.W, v.H, v.cam, r->result.p, r->filtered.p, r->err.p, moment);
         if (rc) return rc;
       }
       HIP_TRY(timed_end(r, 5, ev));
@@ -1336,8 +1342,10 @@ int render_adaptive_frame(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa, co
       rc = model_buffers(r);
       if (rc) return rc;
       for (const ViewSpan& v : views) {            // second moment filtered like the image, then the features
-        rc = run_filter_at(r, v.off, v.W, v.H, v.cam, r->sq.p, r->sq_f.p, r->sq_e.p);
-        if (rc) return rc;
+        if (!moment) {
+          rc = run_filter_at(r, v.off, v.W, v.H, v.cam, r->sq.p, r->sq_f.p, r->sq_e.p);
+          if (rc) return rc;
+        }
         HIP_TRY(launch_mlp_features(feature_args(r, v.off, v.cam), v.W * v.H, r->mlp_x.p + v.off * kMlpIn,
                                     r->stream));
       }

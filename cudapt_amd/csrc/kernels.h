@@ -251,9 +251,11 @@ struct FilterArgs {
   float cam[3];
   float gauss[2 * kMaxFilterRadius + 2];   // spatial table: 2 * radius + 1 weights
 };
+// color2: a second image filtered under the same guides.
 hipError_t launch_filter_error(const FilterArgs& fa, const float* color, const float* gpos, const float* gnrm,
                                const float* gdif, const uint32_t* sample_n, float* filtered, float* err,
-                               hipStream_t st);
+                               hipStream_t st, const float* color2 = nullptr, float* filtered2 = nullptr,
+                               float* err2 = nullptr);
 hipError_t launch_error_sum(const float* err, uint32_t n, double* block_sums, float* sum_out, hipStream_t st);
 // paths / maxp: per-pixel path counts and the cap a pass's count stops at (maxp 0: no cap)
 hipError_t launch_alloc_scan(const float* err, const float* sum, uint32_t n, uint32_t gen, uint32_t* counts,

@@ -3108,49 +3108,60 @@ constexpr int kLdsRadius = 9;     // LDS tile path up to this radius, global rea
 // residual of pt_calculateSquareError_kernel.  One exponential per tap: the
 // range terms' exponents are summed, each scaled by its 1 / 2 sigma^2 (correctly rounded
 // once per thread) and accumulated with fmas, so a tap takes no division.
-// A pixel: its own guides and the sums so far, taps added in raster order.
-template <bool DIFF, bool DEPTH>
+// A pixel's guides, and for an image the pixel's own value and the sums so far,
+// taps added in raster order.
 struct FilterPixel {
-  float c[3], p[3], n[3], d[3], z, iz;
-  float sum, t0, t1, t2;
+  float p[3], n[3], d[3], z, iz;
+};
+struct FilterSums {
+  float c[3], sum, t0, t1, t2;
 };
 struct FilterScale {
   float c, p, n, d, z;
 };
 struct FilterTap {
-  float c[3], p[3], n[3], d[3], z;
+  float c[3], p[3], n[3], d[3], z, c2[3];
 };
+// The squared distances of a tap's guides.
+struct FilterTerms {
+  float p, n, d, z;
+};
+template <bool DIFF, bool DEPTH>
+__device__ __forceinline__ FilterTerms filter_terms(const FilterPixel& P, const FilterTap& q) {
+  FilterTerms t;
+  t.p = sqd_fma(q.p, P.p);
+  t.n = sqd_fma(q.n, P.n);
+  t.d = DIFF ? sqd_fma(q.d, P.d) : 0.f;
+  const float dz = DEPTH ? (q.z - P.z) * P.iz : 0.f;
+  t.z = dz * dz;
+  return t;
+}
 // The tap's negated exponent: 0 or more, or NaN (every scale is the reciprocal of a square).
 template <bool DIFF, bool DEPTH>
-__device__ __forceinline__ float filter_exponent(const FilterPixel<DIFF, DEPTH>& P, const FilterTap& q,
+__device__ __forceinline__ float filter_exponent(const float* c, const float* qc, const FilterTerms& t,
                                                  const FilterScale& k) {
-  float a = sqd_fma(q.c, P.c) * k.c;
-  a = __builtin_fmaf(sqd_fma(q.p, P.p), k.p, a);
-  a = __builtin_fmaf(sqd_fma(q.n, P.n), k.n, a);
-  if (DIFF) a = __builtin_fmaf(sqd_fma(q.d, P.d), k.d, a);
-  if (DEPTH) {
-    const float dz = (q.z - P.z) * P.iz;
-    a = __builtin_fmaf(dz * dz, k.z, a);
-  }
+  float a = sqd_fma(qc, c) * k.c;
+  a = __builtin_fmaf(t.p, k.p, a);
+  a = __builtin_fmaf(t.n, k.n, a);
+  if (DIFF) a = __builtin_fmaf(t.d, k.d, a);
+  if (DEPTH) a = __builtin_fmaf(t.z, k.z, a);
   return a;
 }
-template <bool DIFF, bool DEPTH>
-__device__ __forceinline__ void filter_add(FilterPixel<DIFF, DEPTH>& P, const FilterTap& q, float a, float w) {
+__device__ __forceinline__ void filter_add(FilterSums& S, const float* qc, float a, float w) {
   const float f = w * cpt_exp_neg(a);
-  P.t0 = __builtin_fmaf(f, q.c[0], P.t0);
-  P.t1 = __builtin_fmaf(f, q.c[1], P.t1);
-  P.t2 = __builtin_fmaf(f, q.c[2], P.t2);
-  P.sum = P.sum + f;
+  S.t0 = __builtin_fmaf(f, qc[0], S.t0);
+  S.t1 = __builtin_fmaf(f, qc[1], S.t1);
+  S.t2 = __builtin_fmaf(f, qc[2], S.t2);
+  S.sum = S.sum + f;
 }
 // A tap of exponent past 103 weighs exactly 0 and adds nothing to finite sums;
 // infinite exponents (infinite guides) are left to the arithmetic.
 __device__ __forceinline__ bool filter_zero(float a) { return a > 103.f && a < __builtin_huge_valf(); }
-template <bool DIFF, bool DEPTH>
-__device__ __forceinline__ void filter_store(const FilterArgs& fa, const FilterPixel<DIFF, DEPTH>& P, uint32_t x,
-                                             uint32_t y, const uint32_t* __restrict__ sample_n,
-                                             float* __restrict__ filtered, float* __restrict__ err) {
+__device__ __forceinline__ void filter_store(const FilterArgs& fa, const FilterSums& S, uint32_t x, uint32_t y,
+                                             const uint32_t* __restrict__ sample_n, float* __restrict__ filtered,
+                                             float* __restrict__ err) {
   const size_t ind = (size_t)y * fa.width + x;
-  const float o0 = P.t0 / P.sum, o1 = P.t1 / P.sum, o2 = P.t2 / P.sum;
+  const float o0 = S.t0 / S.sum, o1 = S.t1 / S.sum, o2 = S.t2 / S.sum;
   filtered[ind * 3] = o0;
   filtered[ind * 3 + 1] = o1;
   filtered[ind * 3 + 2] = o2;
@@ -3158,19 +3169,23 @@ __device__ __forceinline__ void filter_store(const FilterArgs& fa, const FilterP
   const uint32_t sn = sample_n[ind];
   float red = (float)fa.nd / (float)(fa.nd + sn);
   if (fa.nd + sn < sn) red = 0.f;
-  const float d0 = o0 - P.c[0], d1 = o1 - P.c[1], d2 = o2 - P.c[2];
+  const float d0 = o0 - S.c[0], d1 = o1 - S.c[1], d2 = o2 - S.c[2];
   err[ind] = red * ((d0 * d0 + d1 * d1) + d2 * d2) / 3.f;
 }
 template <bool DIFF, bool DEPTH>
-__device__ __forceinline__ void filter_start(FilterPixel<DIFF, DEPTH>& P, const FilterTap& q) {
+__device__ __forceinline__ void filter_start(FilterPixel& P, const FilterTap& q) {
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    P.c[c] = q.c[c]; P.p[c] = q.p[c]; P.n[c] = q.n[c];
+    P.p[c] = q.p[c]; P.n[c] = q.n[c];
     P.d[c] = DIFF ? q.d[c] : 0.f;
   }
   P.z = DEPTH ? q.z : 0.f;
   P.iz = P.z > 0.f ? 1.f / P.z : 0.f;
-  P.sum = P.t0 = P.t1 = P.t2 = 0.f;
+}
+__device__ __forceinline__ void filter_start(FilterSums& S, const float* qc) {
+#pragma unroll
+  for (int c = 0; c < 3; c++) S.c[c] = qc[c];
+  S.sum = S.t0 = S.t1 = S.t2 = 0.f;
 }
 __device__ __forceinline__ FilterScale filter_scale(const FilterArgs& fa, bool depth) {
   return {1.f / fa.kc, 1.f / fa.kp, 1.f / fa.kn, 1.f / fa.kd, depth ? 1.f / fa.kz : 0.f};
@@ -3186,21 +3201,29 @@ __device__ __forceinline__ FilterScale filter_scale(const FilterArgs& fa, bool d
 // weights multiplied per tap and a depth branch took 381 / 305 (71 instructions a tap),
 // at radius 7 735 / 558 against 524 / 467.  Two pixels of a column a thread, which share each
 // record, 279 / 242 and 572 / 517: twice the LDS leaves half the waves.
-template <bool DIFF, bool DEPTH>
+// PAIR: a second image (color2) under the same guides in the same pass, whose taps share the
+// records and the guides' distances; its pixels take the words of the record that are free.
+// Image and second moment of the learned frames (1920 x 1080, radius 7, depth): 760 us,
+// two passes 1044.
+template <bool DIFF, bool DEPTH, bool PAIR>
 __global__ __launch_bounds__(kTile * kTile) void k_filter_lds(FilterArgs fa, const float* __restrict__ color,
                                                               const float* __restrict__ gpos,
                                                               const float* __restrict__ gnrm,
                                                               const float* __restrict__ gdif,
                                                               const uint32_t* __restrict__ sample_n,
-                                                              float* __restrict__ filtered, float* __restrict__ err) {
+                                                              float* __restrict__ filtered, float* __restrict__ err,
+                                                              const float* __restrict__ color2,
+                                                              float* __restrict__ filtered2,
+                                                              float* __restrict__ err2) {
+  static_assert(!(DIFF && PAIR), "a pair's record has no room for the albedo");
   extern __shared__ float4 sm[];
   const int R = (int)fa.radius, D = 2 * R + 1, TW = kTile + 2 * R, TA = TW * TW;
   const uint32_t W = fa.width, H = fa.height;
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * kTile + tx;
   const int bx = blockIdx.x * kTile, by = blockIdx.y * kTile;
-  float* rec = (float*)sm;                         // c, p, n, then d or (z, -, -)
+  float* rec = (float*)sm;                         // c, p, n, then d, or z and two words of c2, or c2
   float* wt = rec + 12 * (size_t)TA;               // spatial weight of tap (i, j)
-  float* sz = wt + (size_t)D * D;                  // depth per halo pixel (DIFF && DEPTH)
+  float* sz = wt + (size_t)D * D;                  // DEPTH: z (DIFF) or c2's last (PAIR) per halo pixel
   const float cam[3] = {fa.cam[0], fa.cam[1], fa.cam[2]};
   for (int k = tid; k < D * D; k += kTile * kTile) {
     const int i = k / D, j = k - i * D;
@@ -3221,6 +3244,12 @@ __global__ __launch_bounds__(kTile * kTile) void k_filter_lds(FilterArgs fa, con
       const float z = sqrtf(sqdist3(gpos + g, cam));
       if (DIFF) sz[k] = z; else r[9] = z;
     }
+    if (PAIR) {
+      constexpr int at = DEPTH ? 10 : 9;
+      r[at] = color2[g];
+      r[at + 1] = color2[g + 1];
+      if (DEPTH) sz[k] = color2[g + 2]; else r[11] = color2[g + 2];
+    }
   }
   __syncthreads();
   const auto load = [&](int k) {
@@ -3232,22 +3261,36 @@ __global__ __launch_bounds__(kTile * kTile) void k_filter_lds(FilterArgs fa, con
     q.n[0] = b.z; q.n[1] = b.w; q.n[2] = c.x;
     q.d[0] = c.y; q.d[1] = c.z; q.d[2] = c.w;
     q.z = DEPTH ? (DIFF ? sz[k] : c.y) : 0.f;
+    q.c2[0] = DEPTH ? c.z : c.y; q.c2[1] = DEPTH ? c.w : c.z; q.c2[2] = PAIR && DEPTH ? sz[k] : c.w;
     return q;
   };
   const FilterScale ks = filter_scale(fa, DEPTH);
   const uint32_t x = bx + tx, y = by + ty;
-  FilterPixel<DIFF, DEPTH> P;
-  filter_start(P, load((ty + R) * TW + tx + R));
+  FilterPixel P;
+  FilterSums S, S2;
+  {
+    const FilterTap q = load((ty + R) * TW + tx + R);
+    filter_start<DIFF, DEPTH>(P, q);
+    filter_start(S, q.c);
+    if (PAIR) filter_start(S2, q.c2);
+  }
   for (int i = 0; i < D; i++) {
     const int row = (ty + i) * TW + tx;
     for (int j = 0; j < D; j++) {
       const FilterTap q = load(row + j);
-      const float a = filter_exponent(P, q, ks);
-      if (__ballot(!filter_zero(a)) == 0ull) continue;
-      filter_add(P, q, a, wt[i * D + j]);
+      const FilterTerms t = filter_terms<DIFF, DEPTH>(P, q);
+      const float a = filter_exponent<DIFF, DEPTH>(S.c, q.c, t, ks);
+      const float a2 = PAIR ? filter_exponent<DIFF, DEPTH>(S2.c, q.c2, t, ks) : 0.f;
+      if (__ballot(!(filter_zero(a) && (!PAIR || filter_zero(a2)))) == 0ull) continue;
+      const float w = wt[i * D + j];
+      filter_add(S, q.c, a, w);
+      if (PAIR) filter_add(S2, q.c2, a2, w);
     }
   }
-  if (x < W && y < H) filter_store(fa, P, x, y, sample_n, filtered, err);
+  if (x < W && y < H) {
+    filter_store(fa, S, x, y, sample_n, filtered, err);
+    if (PAIR) filter_store(fa, S2, x, y, sample_n, filtered2, err2);
+  }
 }
 
 // Radii whose halo does not fit: every tap read from memory.
@@ -3279,41 +3322,52 @@ __global__ __launch_bounds__(kTile * kTile) void k_filter_mem(FilterArgs fa, con
     return q;
   };
   const FilterScale ks = filter_scale(fa, DEPTH);
-  FilterPixel<DIFF, DEPTH> P;
-  filter_start(P, load((int)y, (int)x));
+  FilterPixel P;
+  FilterSums S;
+  {
+    const FilterTap q = load((int)y, (int)x);
+    filter_start<DIFF, DEPTH>(P, q);
+    filter_start(S, q.c);
+  }
   for (int i = -R; i <= R; i++)
     for (int j = -R; j <= R; j++) {
       const FilterTap q = load((int)y + i, (int)x + j);
-      filter_add(P, q, filter_exponent(P, q, ks), sg[i + R] * sg[j + R]);
+      const float a = filter_exponent<DIFF, DEPTH>(S.c, q.c, filter_terms<DIFF, DEPTH>(P, q), ks);
+      filter_add(S, q.c, a, sg[i + R] * sg[j + R]);
     }
-  filter_store(fa, P, x, y, sample_n, filtered, err);
+  filter_store(fa, S, x, y, sample_n, filtered, err);
 }
 
 hipError_t launch_filter_error(const FilterArgs& fa, const float* color, const float* gpos, const float* gnrm,
                                const float* gdif, const uint32_t* sample_n, float* filtered, float* err,
-                               hipStream_t st) {
+                               hipStream_t st, const float* color2, float* filtered2, float* err2) {
   if (!color || !gpos || !gnrm || !sample_n || !filtered || !err || (fa.use_diff && !gdif) ||
-      (int)fa.radius > kMaxFilterRadius || fa.width == 0 || fa.height == 0)
+      (color2 && (!filtered2 || !err2)) || (int)fa.radius > kMaxFilterRadius || fa.width == 0 || fa.height == 0)
     return hipErrorInvalidValue;
   const int R = (int)fa.radius, D = 2 * R + 1;
-  const bool depth = fa.kz > 0.f, diff = fa.use_diff != 0;
+  const bool depth = fa.kz > 0.f, diff = fa.use_diff != 0, pair = color2 && !diff && R <= kLdsRadius;
   const dim3 block(kTile, kTile), grid((fa.width + kTile - 1) / kTile, (fa.height + kTile - 1) / kTile);
   const int TA = (kTile + 2 * R) * (kTile + 2 * R);
-  const size_t bytes = sizeof(float) * (12 * (size_t)TA + (size_t)D * D + (diff && depth ? TA : 0));
-#define CPT_FILTER(DI, DE)                                                                                      \
-  {                                                                                                             \
-    if (R > kLdsRadius)                                                                                         \
-      k_filter_mem<DI, DE><<<grid, block, 0, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered, err);       \
-    else                                                                                                        \
-      k_filter_lds<DI, DE><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered, err);   \
+  const size_t bytes = sizeof(float) * (12 * (size_t)TA + (size_t)D * D + ((diff || pair) && depth ? TA : 0));
+#define CPT_FILTER(DI, DE, PA)                                                                                    \
+  {                                                                                                               \
+    if (R > kLdsRadius)                                                                                           \
+      k_filter_mem<DI, DE><<<grid, block, 0, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered, err);         \
+    else                                                                                                          \
+      k_filter_lds<DI, DE, PA><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered, err,  \
+                                                           color2, filtered2, err2);                              \
   }
   if (diff) {
-    if (depth) CPT_FILTER(true, true) else CPT_FILTER(true, false)
+    if (depth) CPT_FILTER(true, true, false) else CPT_FILTER(true, false, false)
+  } else if (pair) {
+    if (depth) CPT_FILTER(false, true, true) else CPT_FILTER(false, false, true)
   } else {
-    if (depth) CPT_FILTER(false, true) else CPT_FILTER(false, false)
+    if (depth) CPT_FILTER(false, true, false) else CPT_FILTER(false, false, false)
   }
 #undef CPT_FILTER
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !color2 || pair) return e;
+  return launch_filter_error(fa, color2, gpos, gnrm, gdif, sample_n, filtered2, err2, st, nullptr, nullptr, nullptr);
 }
 
 // Fixed-order double sum (stands in for thrust::reduce, AdapBilatAtomic.cu:1444):

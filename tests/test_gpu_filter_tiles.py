@@ -54,3 +54,23 @@ def test_depth(cpt, radius, diff):
     ref = oracle.bilateral_ext(col, g[0], g[1], g[2] if diff else None, 0.3, 0.5, 0.25, 0.1, radius, ss=2.5, sz=0.05,
                                cam=sc["camera"]["pos"])
     assert _same(got, ref)
+
+
+@pytest.mark.parametrize("radius,diff,depth", [(3, 0, 0.05), (9, 0, 0.05), (7, 0, 0.0), (4, 1, 0.05), (10, 0, 0.05)])
+def test_pair(cpt, radius, diff, depth):
+    """The learned modes filter the second moment in the image's pass; a profiled renderer filters it on its own."""
+    sc = scenes.cornell()
+    S = cpt.Scene(sc)
+    M = cpt.Mlp(3)
+    got = []
+    for prof in (True, False):
+        R = cpt.Renderer(67, 45, mode=cpt.CPT_MODE_BDPT_ADAPTIVE_PLL, **{
+            "Filter Radius": radius, "Filter Diffuse Flag": diff, "Filter Depth EuD": depth, "Filter Color EuD": 0.3,
+            "Filter Pos EuD": 0.5, "Learned Signal": 3})
+        R.set_profiling(prof)
+        R.set_mlp(M)
+        img = R.render(S, sc["camera"], frames=8)
+        got.append([img] + [R.read(b) for b in (cpt.CPT_BUF_FILTERED, cpt.CPT_BUF_ERROR, cpt.CPT_BUF_ALLOC_ERROR,
+                                                cpt.CPT_BUF_SAMPLE_COUNTS)])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
