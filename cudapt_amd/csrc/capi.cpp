@@ -1269,6 +1269,30 @@ u32 warmup_frames(const cpt_renderer* r) {
   return (u32)std::max(r->attr(kWarmup), r->attr(kMinPaths));
 }
 
+// The light pass.  beside: on the side stream, after everything queued so far
+// (earlier shading reads the cache slots it rebuilds), next to what follows here
+// up to the first shading, which waits for it.  It writes only the cache and
+// FrameCounters::light_n.
+int run_light_pass(cpt_renderer* r, const DevScene& sc, const FrameArgs& fa, const LightJobs& jobs, bool beside) {
+  hipEvent_t ev = nullptr;
+  hipStream_t ls = r->stream;
+  if (r->overlap_shadow && beside) {
+    if (!r->side) HIP_TRY(hipStreamCreateWithFlags(&r->side, hipStreamNonBlocking));
+    if (!r->ev_light) HIP_TRY(hipEventCreateWithFlags(&r->ev_light, hipEventDisableTiming));
+    HIP_TRY(hipEventRecord(r->ev_light, r->stream));
+    HIP_TRY(hipStreamWaitEvent(r->side, r->ev_light, 0));
+    ls = r->side;
+  }
+  HIP_TRY(timed_begin(r, 3, &ev, ls));
+  HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, use_nodes8(r, sc), ls));
+  HIP_TRY(timed_end(r, 3, ev, ls));
+  if (ls != r->stream) {
+    HIP_TRY(hipEventRecord(r->ev_light, ls));
+    r->light_pending = true;
+  }
+  return CPT_OK;
+}
+
 // One view of a multi-view adaptive batch: its first pixel in the
 // concatenated buffers, its size and its camera position.
 struct ViewSpan {
@@ -1292,9 +1316,9 @@ int render_adaptive_frame(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa, co
   hipEvent_t ev = nullptr;
   LightJobs jobs = light_jobs(r, fa.frame0, 1);
   if (jobs.n) {
-    HIP_TRY(timed_begin(r, 3, &ev));
-    HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, use_nodes8(r, sc), r->stream));
-    HIP_TRY(timed_end(r, 3, ev));
+    // beside the filter and the allocation, or the first extension; a frame carried whole reads it at once
+    const int rc = run_light_pass(r, sc, fa, jobs, fa.frame0 >= warmup_frames(r) || !whole_paths(r, n));
+    if (rc) return rc;
   }
   Accum ac;
   std::memset(&ac, 0, sizeof ac);
@@ -1441,25 +1465,9 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
   const bool mega = !pt && !disney &&
                     (r->attr(kMegakernel) != 0 || (whole_paths(r, n, 2.0) && r->attr(kTailBounce) < 1.0));
   if (jobs.n) {
-    // The first extension reads no light vertex: with the side stream the
-    // pass runs there, after everything queued so far (earlier shading reads
-    // the cache slots it rebuilds), and the first shading waits for it.
-    // It writes only the cache and FrameCounters::light_n.
-    hipStream_t ls = r->stream;
-    if (r->overlap_shadow && !mega) {
-      if (!r->side) HIP_TRY(hipStreamCreateWithFlags(&r->side, hipStreamNonBlocking));
-      if (!r->ev_light) HIP_TRY(hipEventCreateWithFlags(&r->ev_light, hipEventDisableTiming));
-      HIP_TRY(hipEventRecord(r->ev_light, r->stream));
-      HIP_TRY(hipStreamWaitEvent(r->side, r->ev_light, 0));
-      ls = r->side;
-    }
-    HIP_TRY(timed_begin(r, 3, &ev, ls));
-    HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, use_nodes8(r, sc), ls));
-    HIP_TRY(timed_end(r, 3, ev, ls));
-    if (ls != r->stream) {
-      HIP_TRY(hipEventRecord(r->ev_light, ls));
-      r->light_pending = true;
-    }
+    // the first extension reads no light vertex
+    const int rc = run_light_pass(r, sc, fa, jobs, !mega);
+    if (rc) return rc;
   }
   HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
   Accum ac;
