@@ -293,7 +293,7 @@ class Scene:
     def trace(self, rays: np.ndarray, cull: bool = False) -> np.ndarray:
         """rays: structured RAY_DTYPE or (n, 8) float32. Host arrays in and out."""
         r = np.ascontiguousarray(rays).view(np.float32).reshape(-1, 8)
-        hits = np.zeros(len(r), HIT_DTYPE)
+        hits = np.empty(len(r), HIT_DTYPE)
         _check(lib().cpt_trace_closest(self.h, _ptr(r), len(r), int(cull), _ptr(hits)), "cpt_trace_closest")
         return hits
 
@@ -367,7 +367,8 @@ class Renderer:
         _check(lib().cpt_renderer_set_attrib(self.h, idx, float(value)), "cpt_renderer_set_attrib")
 
     def render(self, scene: Scene, camera: dict, frames: int = 1, result: bool = True):
-        out = np.zeros((self.H, self.W, 3), np.float32) if result else None
+        # not zeroed: the call fills all of it, and clearing 5.8 MB takes as long as copying it
+        out = np.empty((self.H, self.W, 3), np.float32) if result else None
         args = (self.h, scene.h, _f3(camera["pos"]), _f3(camera["dir"]), _f3(camera["up"]),
                 float(camera["fov"]))
         if frames == 1:
@@ -377,7 +378,7 @@ class Renderer:
         return out
 
     def sample_counts(self):
-        out = np.zeros((self.H, self.W), np.uint32)
+        out = np.empty((self.H, self.W), np.uint32)
         _check(lib().cpt_renderer_read_buffer(self.h, CPT_BUF_SAMPLE_N, _ptr(out)), "cpt_renderer_read_buffer")
         return out
 
@@ -387,11 +388,11 @@ class Renderer:
         if which == CPT_BUF_BOUNCE_RAYS:
             out = np.zeros((2, 16), np.uint32)
         elif which in (CPT_BUF_SAMPLE_N, CPT_BUF_SAMPLE_COUNTS, CPT_BUF_PIXEL_PATHS):
-            out = np.zeros((self.H, self.W), np.uint32)
+            out = np.empty((self.H, self.W), np.uint32)
         elif which in (CPT_BUF_ERROR, CPT_BUF_ALLOC_ERROR):
-            out = np.zeros((self.H, self.W), np.float32)
+            out = np.empty((self.H, self.W), np.float32)
         else:
-            out = np.zeros((self.H, self.W, 3), np.float32)
+            out = np.empty((self.H, self.W, 3), np.float32)
         _check(lib().cpt_renderer_read_buffer(self.h, which, _ptr(out)), "cpt_renderer_read_buffer")
         return out
 
@@ -484,13 +485,13 @@ class Batch:
 
     def result(self, view: int) -> np.ndarray:
         w, h = self.views[view]
-        out = np.zeros((h, w, 3), np.float32)
+        out = np.empty((h, w, 3), np.float32)
         _check(lib().cpt_batch_read_result(self.h, view, _ptr(out)), "cpt_batch_read_result")
         return out
 
     def sample_counts(self, view: int) -> np.ndarray:
         w, h = self.views[view]
-        out = np.zeros((h, w), np.uint32)
+        out = np.empty((h, w), np.uint32)
         _check(lib().cpt_batch_sample_counts(self.h, view, _ptr(out)), "cpt_batch_sample_counts")
         return out
 
@@ -498,11 +499,11 @@ class Batch:
         """One view's CPT_BUF_* buffer."""
         w, h = self.views[view]
         if which in (CPT_BUF_SAMPLE_N, CPT_BUF_SAMPLE_COUNTS, CPT_BUF_PIXEL_PATHS):
-            out = np.zeros((h, w), np.uint32)
+            out = np.empty((h, w), np.uint32)
         elif which in (CPT_BUF_ERROR, CPT_BUF_ALLOC_ERROR):
-            out = np.zeros((h, w), np.float32)
+            out = np.empty((h, w), np.float32)
         else:
-            out = np.zeros((h, w, 3), np.float32)
+            out = np.empty((h, w, 3), np.float32)
         _check(lib().cpt_batch_read_buffer(self.h, view, which, _ptr(out)), "cpt_batch_read_buffer")
         return out
 
