@@ -1330,12 +1330,14 @@ int render_adaptive_frame(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa, co
   // empirical files use the plain stream's bounce
   ac.variant = kVariantGbuf | (r->mode == CPT_MODE_BDPT_ADAPTIVE_PLL ? kVariantReflOffset : 0);
   const u32 maxp = (u32)r->attr(kMaxPaths);
+  u32 n_whole = 0;
   if (fa.frame0 < warmup_frames(r)) {              // plain 1 spp frames with G-buffer (:1372-1406)
     ac.apply = 1;
-    HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
     if (whole_paths(r, n)) {
+      n_whole = n;
       HIP_TRY(trace_whole(r, sc, fa, ac));
     } else {
+      HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
       HIP_TRY(launch_gen_eye_rec(fa, r->A.view(), ac.rec, r->stream));
       int rc = bounce_loop(r, sc, fa, n, ac);
       if (rc) return rc;
@@ -1421,7 +1423,7 @@ int render_adaptive_frame(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa, co
                                   r->gnrm.p, r->gdif.p, r->sq.p, r->big_list.p, r->big_n.p, r->stream));
     HIP_TRY(timed_end(r, 8, ev));
   }
-  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, fa.nframes, fa.eye_depth, r->parts, r->stream));
+  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, fa.nframes, fa.eye_depth, r->parts, n_whole, r->stream));
   return CPT_OK;
 }
 
@@ -1469,13 +1471,13 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
     const int rc = run_light_pass(r, sc, fa, jobs, !mega);
     if (rc) return rc;
   }
-  HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
+  if (!mega) HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
   Accum ac;
   std::memset(&ac, 0, sizeof ac);
   ac.result = r->result.p;
   ac.sample_n = r->sample_n.p;
   ac.rec.acc = r->rec_acc.p;
-  ac.apply = 2;
+  ac.apply = mega && fa.nframes == 1 ? 0 : 2;      // one frame carried whole: each path's end applies its pixel
   ac.variant = pt ? kVariantPT | (regen ? kVariantPTRegen : 0) : disney ? kVariantDisney : 0;
   if (regen) {
     ac.term_bounce = r->term_bounce.p;
@@ -1491,7 +1493,7 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
     if (rc) return rc;
   }
   if (regen) {                                     // the restarts, as a second wavefront
-    HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, fa.nframes, fa.eye_depth, r->parts, r->stream));
+    HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, fa.nframes, fa.eye_depth, r->parts, 0, r->stream));
     HIP_TRY(timed_begin(r, 7, &ev));
     HIP_TRY(launch_regen(fa, r->A.view(), ac, r->fc.p, r->stream));
     HIP_TRY(timed_end(r, 7, ev));
@@ -1500,10 +1502,13 @@ int render_batch(cpt_renderer* r, cpt_scene* s, const FrameArgs& fa) {
     int rc = bounce_loop(r, sc, fa, n, ac);
     if (rc) return rc;
   }
-  HIP_TRY(timed_begin(r, 8, &ev));
-  HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, pt ? 1 : 0, r->stream));
-  HIP_TRY(timed_end(r, 8, ev));
-  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, regen ? 0u : fa.nframes, fa.eye_depth, r->parts, r->stream));
+  if (ac.apply == 2) {
+    HIP_TRY(timed_begin(r, 8, &ev));
+    HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, pt ? 1 : 0, r->stream));
+    HIP_TRY(timed_end(r, 8, ev));
+  }
+  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, regen ? 0u : fa.nframes, fa.eye_depth, r->parts, mega ? n : 0u,
+                           r->stream));
   return CPT_OK;
 }
 
@@ -2178,21 +2183,22 @@ int batch_enqueue(cpt_batch* b, cpt_scene* s, u32 k) {
   jobs.dev_groups = (k + 2) / 3 + 1;                 // groups k frames can span
   const u32 n = b->total * k;
   HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, use_nodes8(r, sc), r->stream));
-  HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
+  const bool whole = !r->persist_chunk && whole_paths(r, n, 2.0);
+  if (!whole) HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
   Accum ac;
   std::memset(&ac, 0, sizeof ac);
   ac.result = r->result.p;
   ac.sample_n = r->sample_n.p;
   ac.rec.acc = r->rec_acc.p;
-  ac.apply = 2;
-  if (!r->persist_chunk && whole_paths(r, n, 2.0)) {
+  ac.apply = whole && k == 1 ? 0 : 2;
+  if (whole) {
     HIP_TRY(trace_whole(r, sc, fa, ac));
   } else {
     int rc = bounce_loop(r, sc, fa, n, ac, true);
     if (rc) return rc;
   }
-  HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, 0, r->stream));
-  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, k, fa.eye_depth, r->parts, r->stream));
+  if (ac.apply == 2) HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, 0, r->stream));
+  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, k, fa.eye_depth, r->parts, whole ? n : 0u, r->stream));
   HIP_TRY(launch_frame_advance(b->frame_dev.p, k, r->stream));
   return CPT_OK;
 }

@@ -323,8 +323,9 @@ hipError_t launch_scan_counts(const uint32_t* counts, uint32_t n, uint32_t* offs
 hipError_t launch_shadow(const DevScene& sc, ShadowBuf sb, PathBuf nxt, const FrameCounters* fc, int bounce,
                          uint32_t max_n, int lds_stack, int quant, DevStats* stats, hipStream_t st);
 // parts: add FrameCounters::part in (a tail or a megakernel ran).
+// n_whole: the paths of a frame carried whole without a frame_begin (0: others).
 hipError_t launch_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, int parts,
-                            hipStream_t st);
+                            uint32_t n_whole, hipStream_t st);
 hipError_t launch_queues_clear(uint32_t* queue, hipStream_t st);   // all kQueues launches' counters
 // Closest hit (shadow = 0: hits into out) or connection visibility (shadow = 1:
 // contributions into nxt) of the `*count` rays by a persistent grid whose

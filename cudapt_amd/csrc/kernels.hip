@@ -1155,33 +1155,38 @@ hipError_t launch_frame_begin_dev(FrameCounters* fc, const uint32_t* total, uint
   return hipGetLastError();
 }
 
-__global__ void k_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, int parts) {
-  if (parts) {                                      // 32 counters, two threads each
-    const uint32_t c = threadIdx.x & 31u, half = threadIdx.x >> 5;
-    uint32_t v = 0;
+// n_whole > 0: every one of the frame's n_whole paths was carried whole and no
+// frame_begin ran: the counters are set here, from the parts alone.
+__global__ void k_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, int parts,
+                            uint32_t n_whole) {
+  const uint32_t c = threadIdx.x & 31u, half = threadIdx.x >> 5;   // 32 counters, two threads each
+  uint32_t v = 0;
+  if (parts) {
 #pragma unroll 8
     for (uint32_t s = half; s < kPartSlots; s += 2) {
       v += fc->part[s][c];
       fc->part[s][c] = 0u;
     }
     v += __shfl_xor(v, 32, 64);
-    if (half == 0) {
-      if (c < 16) fc->active[c] += v; else fc->shadow[c - 16] += v;
-    }
-    __syncthreads();
   }
+  uint32_t* at = c < 16 ? &fc->active[c] : &fc->shadow[c - 16];
+  const uint32_t f = v + (n_whole ? (c == 0 ? n_whole : 0u) : *at);
+  if (half == 0) *at = f;
+  const bool counts = half == 0 && (c & 15u) < depth;
+  const auto sum = [](uint32_t x) {                 // 64 bits: the bounces' counts together may pass 32
+    return (unsigned long long)wave_sum(x & 0xFFFFu) + ((unsigned long long)wave_sum(x >> 16) << 16);
+  };
+  const unsigned long long e = sum(counts && c < 16 ? f : 0u), s = sum(counts && c >= 16 ? f : 0u);
   if (threadIdx.x == 0) {
-    unsigned long long e = 0, s = 0;
-    for (uint32_t b = 0; b < depth && b < 16; b++) { e += fc->active[b]; s += fc->shadow[b]; }
     stats->ext_rays += e;
     stats->shadow_rays += s;
-    stats->eye_paths += fc->active[0];
+    stats->eye_paths += f;
     stats->frames += nframes;
   }
 }
 hipError_t launch_frame_end(FrameCounters* fc, DevStats* stats, uint32_t nframes, uint32_t depth, int parts,
-                            hipStream_t st) {
-  k_frame_end<<<1, 64, 0, st>>>(fc, stats, nframes, depth, parts);
+                            uint32_t n_whole, hipStream_t st) {
+  k_frame_end<<<1, 64, 0, st>>>(fc, stats, nframes, depth, parts, n_whole);
   return hipGetLastError();
 }
 __global__ void k_frame_advance(uint32_t* frame_dev, uint32_t k) {
