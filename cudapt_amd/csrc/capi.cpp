@@ -93,7 +93,7 @@ struct cpt_scene {
   hipStream_t stream = nullptr;
   DevArray<Node4> d_nodes4;
   DevArray<Node8> d_nodes8;
-  DevArray<float4> d_tris, d_tris8, d_tris_bin, d_vpos, d_vnrm, d_bnodes, d_tex, d_surf, d_env;
+  DevArray<float4> d_tris, d_tris8, d_tri_box, d_tris_bin, d_vpos, d_vnrm, d_bnodes, d_tex, d_surf, d_env;
   DevArray<uint4> d_tex_desc;
   DevArray<uint4> d_tri_verts;
   DevArray<uint2> d_boff;
@@ -110,6 +110,7 @@ struct cpt_scene {
     s.nodes4 = d_nodes4.p;
     s.nodes8 = bvh.nodes8.empty() ? nullptr : d_nodes8.p;
     s.tris8 = d_tris8.p;
+    s.tri_box = d_tri_box.p;
     s.tris = d_tris.p;
     s.tri_verts = d_tri_verts.p;
     s.vpos = d_vpos.p;
@@ -440,6 +441,18 @@ int cpt_scene_upload(cpt_scene* s) {
     for (int k = 0; k < 3; k++) tris8[(size_t)i * 3 + k] = tris[(size_t)leaf * 3 + k];
     std::memcpy(&tris8[(size_t)i * 3 + 1].w, &leaf, 4);
   }
+  std::vector<float4> tri_box((size_t)nt * 2);
+  for (u32 i = 0; i < nt; i++) {
+    float mn[3], mx[3];
+    for (int k = 0; k < 3; k++) {
+      const u32* v = &s->idx[(size_t)s->bvh.dreorder[i] * 3];
+      const float a = s->pos[(size_t)v[0] * 3 + k], b = s->pos[(size_t)v[1] * 3 + k], c = s->pos[(size_t)v[2] * 3 + k];
+      mn[k] = std::fmin(c, std::fmin(b, a));
+      mx[k] = std::fmax(c, std::fmax(b, a));
+    }
+    tri_box[(size_t)i * 2] = make_float4(mn[0], mn[1], mn[2], 0.f);
+    tri_box[(size_t)i * 2 + 1] = make_float4(mx[0], mx[1], mx[2], 0.f);
+  }
   std::vector<uint4> tv(nt);
   for (u32 i = 0; i < nt; i++) {
     u32 o = s->bvh.dreorder[i];
@@ -461,6 +474,7 @@ int cpt_scene_upload(cpt_scene* s) {
   HIP_TRY(s->d_nodes4.upload(s->bvh.nodes4.data(), s->bvh.nodes4.size(), s->stream));
   HIP_TRY(s->d_nodes8.upload(s->bvh.nodes8.data(), s->bvh.nodes8.size(), s->stream));
   HIP_TRY(s->d_tris8.upload(tris8.data(), tris8.size(), s->stream));
+  HIP_TRY(s->d_tri_box.upload(tri_box.data(), tri_box.size(), s->stream));
   HIP_TRY(s->d_tris.upload(tris.data(), tris.size(), s->stream));
   HIP_TRY(s->d_tris_bin.upload(tris_bin.data(), tris_bin.size(), s->stream));
   HIP_TRY(s->d_tri_verts.upload(tv.data(), tv.size(), s->stream));
@@ -504,7 +518,8 @@ int cpt_trace_closest_device(cpt_scene* s, const cpt_ray* d_rays, uint32_t n, ui
     HIP_TRY(launch_trace(s->dev(), (const float4*)d_rays, n, nullptr, cull, (float4*)d_hits, 1, 0, layout,
                          s->d_stats.p, st));
   else
-    HIP_TRY(launch_trace_rays(s->dev(), (const float4*)d_rays, n, cull, (float4*)d_hits, 0, s->d_stats.p, s->cus, st));
+    HIP_TRY(launch_trace_rays(s->dev(), (const float4*)d_rays, n, cull, (float4*)d_hits, 0, layout == 0, s->d_stats.p,
+                              s->cus, st));
   if (!stream) HIP_TRY(hipStreamSynchronize(st));
   return CPT_OK;
 }
@@ -514,8 +529,8 @@ int cpt_trace_occluded_device(cpt_scene* s, const cpt_ray* d_rays, uint32_t n, u
   if (!s || (n && (!d_rays || !d_occluded))) return fail(CPT_E_ARG, "cpt_trace_occluded_device: null argument");
   if (!s->uploaded) return fail(CPT_E_STATE, "cpt_trace_occluded_device: scene not uploaded");
   hipStream_t st = stream ? (hipStream_t)stream : s->stream;
-  HIP_TRY(launch_trace_rays(s->dev(), (const float4*)d_rays, n, cull, (float4*)d_occluded, 1, s->d_stats.p, s->cus,
-                            st));
+  HIP_TRY(launch_trace_rays(s->dev(), (const float4*)d_rays, n, cull, (float4*)d_occluded, 1, 1, s->d_stats.p,
+                            s->cus, st));
   if (!stream) HIP_TRY(hipStreamSynchronize(st));
   return CPT_OK;
 }
@@ -529,7 +544,7 @@ int cpt_trace_closest(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cu
       HIP_TRY(hipHostMalloc((void**)&s->stage, (sizeof(cpt_ray) + sizeof(cpt_hit)) * kStageRays, hipHostMallocDefault));
     float4* hit = s->stage + 2 * (size_t)kStageRays;
     std::memcpy(s->stage, rays, sizeof(cpt_ray) * n);
-    HIP_TRY(launch_trace_rays(s->dev(), s->stage, n, cull, hit, 0, s->d_stats.p, s->cus, s->stream));
+    HIP_TRY(launch_trace_rays(s->dev(), s->stage, n, cull, hit, 0, 1, s->d_stats.p, s->cus, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     std::memcpy(hits, hit, sizeof(cpt_hit) * n);
     return CPT_OK;
@@ -537,7 +552,7 @@ int cpt_trace_closest(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cu
   HIP_TRY(s->d_rays.alloc((size_t)n * 2));
   HIP_TRY(s->d_hits.alloc(n));
   HIP_TRY(hipMemcpyAsync(s->d_rays.p, rays, sizeof(cpt_ray) * n, hipMemcpyHostToDevice, s->stream));
-  HIP_TRY(launch_trace_rays(s->dev(), s->d_rays.p, n, cull, s->d_hits.p, 0, s->d_stats.p, s->cus, s->stream));
+  HIP_TRY(launch_trace_rays(s->dev(), s->d_rays.p, n, cull, s->d_hits.p, 0, 1, s->d_stats.p, s->cus, s->stream));
   HIP_TRY(hipMemcpyAsync(hits, s->d_hits.p, sizeof(cpt_hit) * n, hipMemcpyDeviceToHost, s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   return CPT_OK;

@@ -21,6 +21,7 @@ struct DevScene {
   const Node4* nodes4;         // 128-byte 4-wide nodes
   const Node8* nodes8;         // 8-wide quantized nodes; null: the scene is too large for them
   const float4* tris8;         // their triangles, 3 per triangle as tris, e0.w = device leaf index bits
+  const float4* tri_box;       // 2 per triangle: its vertices' bounds, in the order of tris
   const float4* tris;          // 3 per triangle: p0 (w = original id bits), e0 = p1-p0, e1 = p2-p0
   const uint4* tri_verts;      // v0, v1, v2, material
   const float4* vpos;          // vertex positions, w = texture u
@@ -159,9 +160,9 @@ constexpr int kBlock = 256;
 hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, const uint32_t* count, uint32_t cull,
                         float4* hits_out, int out_orig, int any_hit, uint32_t layout, DevStats* stats, hipStream_t st, int cost = 0);
 // The trace entry points' rays (cpt_ray records, hits by original triangle id or
-// occlusion flags) over the 8-wide nodes.
+// occlusion flags) over the 8-wide nodes.  fp32: with the answers of the FP32 4-wide ones.
 hipError_t launch_trace_rays(const DevScene& sc, const float4* rays, uint32_t n, uint32_t cull, float4* out, int any,
-                             DevStats* stats, uint32_t cus, hipStream_t st);
+                             int fp32, DevStats* stats, uint32_t cus, hipStream_t st);
 hipError_t launch_frame_begin(FrameCounters* fc, uint32_t n_paths, hipStream_t st);
 hipError_t launch_light_pass(const DevScene& sc, const FrameArgs& fa, const LightJobs& jobs, LightVert* lv,
                              FrameCounters* fc, int quant, hipStream_t st);

@@ -23,9 +23,11 @@
 //
 // Hit semantics: the closest hit is the minimum of (t, original triangle id)
 // over all triangles with 0 <= t < maxDist, each tested with IntersectTri's
-// exact arithmetic (src/cudaRTCommon.cu:42-64).  Box culling is conservative
-// (Ize 2013 slab widening + a slack covering IntersectTri's eps origin shift),
-// so the answer does not depend on the node layout or visiting order.
+// exact arithmetic (src/cudaRTCommon.cu:42-64).  Over the 8-wide nodes culling is
+// conservative, so the answer does not depend on the visiting order.  Over
+// the FP32 4-wide nodes (Ize 2013 slab widening + a slack for IntersectTri's eps
+// origin shift) a ray that touches a triangle's edge within rounding may miss its
+// box: see kQueryFp32 for how often.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -315,17 +317,47 @@ __device__ __forceinline__ bool ray_step(const DevScene& sc, RayState& R, bool c
   return !pop_node<STK>(R, lstk, pstk);
 }
 
-// Closest (ANY: any) hit of one ray, the loop of ray_step.
-template <bool ANY, int STK = CPT_LDS_STACK>
-__device__ bool traverse4(const DevScene& sc, f3 o, f3 d, float maxd, float eps, bool cull, LdsU64* lstk,
-                          TraceHit& h, uint32_t& nn, uint32_t& nt) {
+// Closest (ANY: any) hit of one ray, the loop of ray_step.  pstk:
+// CPT_STACK_TOTAL - STK private entries.
+template <bool ANY, int STK>
+__device__ __forceinline__ bool traverse4(const DevScene& sc, f3 o, f3 d, float maxd, float eps, bool cull,
+                                          LdsU64* lstk, uint64_t* pstk, TraceHit& h, uint32_t& nn, uint32_t& nt) {
   RayState R;
   ray_begin(R, o, d, maxd, eps);
-  uint64_t pstk[CPT_STACK_TOTAL - STK];
   while (!ray_step<ANY, STK>(sc, R, cull, lstk, pstk, nn, nt, nullptr)) {
   }
   h = R.h;
   return h.leaf != kInvalid;
+}
+template <bool ANY, int STK = CPT_LDS_STACK>
+__device__ bool traverse4(const DevScene& sc, f3 o, f3 d, float maxd, float eps, bool cull, LdsU64* lstk,
+                          TraceHit& h, uint32_t& nn, uint32_t& nt) {
+  uint64_t pstk[CPT_STACK_TOTAL - STK];
+  return traverse4<ANY, STK>(sc, o, d, maxd, eps, cull, lstk, pstk, h, nn, nt);
+}
+
+// Whether traverse4 is sure to test the triangle of device leaf index `leaf`,
+// which the ray hits at t: whether the triangle's own box passes child_boxes'
+// test with t as the best hit.  FP32 subtraction, multiplication, minimum and
+// maximum are monotone, so every box round it passes then too.
+// idir: v_rcp's, within 2 u (u = 2^-24) of 1 / d where child_boxes' is within u;
+// the distances here are then within 5 u of the ones there.  Per axis the entry
+// never lies past the exit; across axes the factor 1 + 2^-21 covers
+// both distances' 5 u (child_boxes multiplies the exit by 1 + 6 u).  Exits
+// and reciprocals near the denormals, where no relative bound holds, fail.
+__device__ __forceinline__ bool reached4(const DevScene& sc, uint32_t leaf, f3 o, f3 idir, float t, float eps) {
+  const float4 lo = sc.tri_box[2 * (size_t)leaf], hi = sc.tri_box[2 * (size_t)leaf + 1];
+  const float k = 1.f + 0x1p-21f;
+  const float x0 = (lo.x - o.x) * idir.x, x1 = (hi.x - o.x) * idir.x;
+  const float y0 = (lo.y - o.y) * idir.y, y1 = (hi.y - o.y) * idir.y;
+  const float z0 = (lo.z - o.z) * idir.z, z1 = (hi.z - o.z) * idir.z;
+  const float ex = fminf(x0, x1) * k, fx = fmaxf(x0, x1);
+  const float ey = fminf(y0, y1) * k, fy = fmaxf(y0, y1);
+  const float ez = fminf(z0, z1) * k, fz = fmaxf(z0, z1);
+  return ex <= fminf(fy, fz) && ey <= fminf(fx, fz) && ez <= fminf(fx, fy) &&
+         fmaxf(fmaxf(ex, ey), fmaxf(ez, 0.f)) <= t + cull_slack(t, eps) &&
+         fminf(fx, fminf(fy, fz)) >= 0x1p-100f &&
+         fminf(fabsf(idir.x), fminf(fabsf(idir.y), fabsf(idir.z))) >= 0x1p-100f;
 }
 
 // ---- 8-wide traversal -------------------------------------------------------
@@ -1705,6 +1737,17 @@ __device__ __forceinline__ bool deal_next(Deal& D, uint32_t count, uint32_t* __r
 // every time one lane finishes.
 // OUT 1: closest hit (t, leaf, u, v) into out[ray]; OUT 3: the connection's
 // visibility (k_shadow's epilogue).
+// Query flags: the back-face test; the answers of the FP32 4-wide nodes.  The
+// two layouts' box tests differ where a ray touches a triangle's edge within
+// rounding: the 8-wide one is conservative, so its hit is the (t, id) minimum over
+// all triangles, while child_boxes may cull the box (2 of 126 M rays spread over
+// the sphere grid, a few in 10^5 of those aimed at its edges, one in 10^3 on the
+// Cornell box).  What the 4-wide nodes find the 8-wide ones find too, so a miss
+// stands, and a hit stands if they are sure to test its triangle (reached4); the
+// other rays are traced again by traverse4.  2,097,143 closest hits on the sphere
+// grid 203 -> 217 us, 1,000,003 occlusion rays on the heightfield 131 -> 142 (box
+// gathered from the vertices 229 / 148, with child_boxes' divisions 223 / 145).
+constexpr uint32_t kQueryCull = 1u, kQueryFp32 = 2u;
 // EYE (closest hit, quantized nodes): ray i is the eye ray of path slot i of
 // the batch fa describes, computed in place of reading ro / rd.  A separate
 // instantiation, so that the plain kernels' code is not touched by it.
@@ -1716,11 +1759,12 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
                                                             const float4* __restrict__ contrib, PathBuf nxt,
                                                             DevStats* __restrict__ stats, uint32_t refill,
                                                             FrameArgs fa) {
-  constexpr bool API = OUT == 0 || OUT == 2;        // fa.width rays as cpt_ray records, fa.flags: back-face test
+  constexpr bool API = OUT == 0 || OUT == 2;        // fa.width rays as cpt_ray records, fa.flags: kQuery*
   constexpr bool ANY = OUT == 2 || OUT == 3;
   constexpr int S8 = kStk8<STK>;
   __shared__ TravLds<STK, Q> lds;
-  uint64_t pstk[Q ? kPriv8<S8> : CPT_STACK_TOTAL - STK];
+  static_assert(kPriv8<S8> <= CPT_STACK_TOTAL, "API: the stack of traverse4 too, once the lane's own ray has finished");
+  uint64_t pstk[API ? CPT_STACK_TOTAL : Q ? kPriv8<S8> : CPT_STACK_TOTAL - STK];
   const uint32_t count = API ? fa.width : *countp;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1759,6 +1803,15 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
         h = R.h;
         hit = h.leaf != kInvalid;
       }
+      if constexpr (API) {
+        if (hit && (fa.flags & kQueryFp32)) {
+          const float4 a = ro[2 * (size_t)ray];
+          if (!reached4(sc, h.leaf, ld3(a), R.idir, h.t, R.eps)) {
+            const float4 b4 = ro[2 * (size_t)ray + 1];
+            hit = traverse4<ANY, 0>(sc, ld3(a), ld3(b4), a.w, b4.w, fa.flags & kQueryCull, nullptr, pstk, h, nn, nt);
+          }
+        }
+      }
       if (OUT == 1) {
         float4 r;
         r.x = hit ? h.t : kInfF;
@@ -1767,7 +1820,8 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
         r.w = hit ? h.v : 0.f;
         out[ray] = r;
       } else if (OUT == 0) {
-        out[ray] = make_float4(__uint_as_float(h.orig), h.t, h.u, h.v);
+        out[ray] = hit ? make_float4(__uint_as_float(h.orig), h.t, h.u, h.v)
+                       : make_float4(__uint_as_float(kInvalid), kInfF, 0.f, 0.f);
       } else if (OUT == 2) {
         ((uint32_t*)out)[ray] = hit ? 1u : 0u;
       } else if (!hit) {
@@ -1824,8 +1878,8 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
     if (__ballot(active) == 0ull) break;
     if constexpr (Q) {
       const bool was = active;
-      ray8_step<ANY, S8>(sc, R, active, API && fa.flags, lds.w[wid], (LdsU64*)&lds.w[wid].stk[0][lane], pstk, lane, nn, nt,
-                         spill);
+      ray8_step<ANY, S8>(sc, R, active, API && (fa.flags & kQueryCull), lds.w[wid], (LdsU64*)&lds.w[wid].stk[0][lane],
+                         pstk, lane, nn, nt, spill);
       if (was && !active) pending = true;
     } else if (active && ray_step<ANY, STK>(sc, R, false, lds_column(lds.stk), pstk, nn, nt, spill)) {
       active = false;
@@ -1902,13 +1956,13 @@ hipError_t launch_trace_dyn(const DevScene& sc, const float4* ro, const float4* 
 // and 1,000,003 occlusion rays on the heightfield 255.
 constexpr uint32_t kTraceGroups = 6, kTraceRefill = 16;
 hipError_t launch_trace_rays(const DevScene& sc, const float4* rays, uint32_t n, uint32_t cull, float4* out, int any,
-                             DevStats* stats, uint32_t cus, hipStream_t st) {
+                             int fp32, DevStats* stats, uint32_t cus, hipStream_t st) {
   if (n == 0) return hipSuccess;
   if (!sc.nodes8) return launch_trace(sc, rays, n, nullptr, cull, out, any ? 0 : 1, any, 0, stats, st);
   if (!rays || !out || !sc.tris8 || cus == 0) return hipErrorInvalidValue;
   FrameArgs fa = {};
   fa.width = n;
-  fa.flags = cull ? 1u : 0u;
+  fa.flags = (cull ? kQueryCull : 0u) | (fp32 ? kQueryFp32 : 0u);
   const uint32_t blocks = (n + kBlock - 1) / kBlock;
   const uint32_t grid = blocks < kTraceGroups * cus ? blocks : kTraceGroups * cus;
   if (any)

@@ -146,9 +146,12 @@ int cpt_scene_destroy(cpt_scene* s);
 int cpt_trace_closest(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cull, cpt_hit* hits);
 
 /* Same over device arrays already resident in HBM, launched on `stream`
- * (a hipStream_t, NULL = the scene's stream).  layout 0 and 2 = the device tree
- * (8-wide nodes with quantized boxes, whose culling stays conservative),
- * 1 = the reference's binary CompactBVH layout.  The hits are the same. */
+ * (a hipStream_t, NULL = the scene's stream).  layout 2 = the device tree's
+ * 8-wide nodes, whose culling is conservative: the minimum of (t, triangle id)
+ * over all triangles; 0 = the answers of its FP32 4-wide nodes (as
+ * cpt_trace_closest and cpt_trace_occluded_device give them), which differ where a
+ * ray touches a triangle's edge within rounding and the triangle's box is
+ * missed; 1 = the reference's binary CompactBVH layout, as 0 but for its boxes. */
 int cpt_trace_closest_device(cpt_scene* s, const cpt_ray* d_rays, uint32_t n, uint32_t cull, cpt_hit* d_hits,
                              void* stream, uint32_t layout);
 
