@@ -1761,6 +1761,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
                                                             FrameArgs fa) {
   constexpr bool API = OUT == 0 || OUT == 2;        // fa.width rays as cpt_ray records, fa.flags: kQuery*
   constexpr bool ANY = OUT == 2 || OUT == 3;
+  constexpr bool SH = OUT == 3;                     // counted as shadow rays; queries of either kind are not
   constexpr int S8 = kStk8<STK>;
   __shared__ TravLds<STK, Q> lds;
   static_assert(kPriv8<S8> <= CPT_STACK_TOTAL, "API: the stack of traverse4 too, once the lane's own ray has finished");
@@ -1891,9 +1892,9 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
     uint32_t sn = wave_sum(nn), st = wave_sum(nt);
     const uint32_t ss = *spill;         // the wave's own word, after its last atomic
     if (lane == 0 && (sn | st)) {
-      atomicAdd(OUT == 1 ? &stats->ext_nodes : &stats->sh_nodes, (unsigned long long)sn);
-      atomicAdd(OUT == 1 ? &stats->ext_tris : &stats->sh_tris, (unsigned long long)st);
-      if (ss) atomicAdd(OUT == 1 ? &stats->ext_spill : &stats->sh_spill, (unsigned long long)ss);
+      atomicAdd(SH ? &stats->sh_nodes : &stats->ext_nodes, (unsigned long long)sn);
+      atomicAdd(SH ? &stats->sh_tris : &stats->ext_tris, (unsigned long long)st);
+      if (ss) atomicAdd(SH ? &stats->sh_spill : &stats->ext_spill, (unsigned long long)ss);
     }
   }
 }

@@ -205,7 +205,9 @@ int cpt_trace_cost(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cull,
 #define CPT_DEPTH_NONE 0xFFFFFFFFu
 int cpt_trace_depth(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t spec_depth, uint32_t* out3);
 
-/* Node visits and triangle tests of every traversal since the last reset. */
+/* Node visits and triangle tests of every query's traversal since the last
+ * reset: closest hits, occlusion and costs (layout 0 and 2: visits of 8-wide
+ * nodes, but cpt_trace_cost counts layout 0's own FP32 4-wide ones). */
 int cpt_trace_counters(cpt_scene* s, uint64_t* nodes, uint64_t* tris, uint64_t* rays, int reset);
 
 /* ---- renderer (RTRenderer / <ns>::Render, include/raytracer.h:292-323,
