@@ -429,6 +429,17 @@ __device__ __forceinline__ void ray8_begin(Ray8& R, Wave8<STK>& W, int lane, f3 
   const f3 oi = mk3(-(o.x * R.idir.x), -(o.y * R.idir.y), -(o.z * R.idir.z));
   R.pn = mk3(oi.x - sx, oi.y - sy, oi.z - sz);
   R.pf = mk3(oi.x + sx, oi.y + sy, oi.z + sz);
+  // No triangle is hit from an origin that is infinite or NaN, or along a NaN (the
+  // test's determinant or distance is one): such a ray meets no box, where NaN
+  // distances would pass every box of the tree.
+  constexpr int kNotFinite = 0x207;                  // v_cmp_class: NaN, -inf, +inf
+  if (__builtin_amdgcn_classf(o.x, kNotFinite) || __builtin_amdgcn_classf(o.y, kNotFinite) ||
+      __builtin_amdgcn_classf(o.z, kNotFinite) || __builtin_isunordered(d.x, d.y) ||
+      __builtin_isunordered(d.z, eps)) {
+    R.idir.x = 0.f;
+    R.pn.x = __builtin_huge_valf();
+    R.pf.x = -__builtin_huge_valf();
+  }
   R.eps = eps;
   // no hit lies at t >= 0 below a maximum that is negative or NaN
   R.ht = maxd > 0.f ? maxd : 0.f;
