@@ -1759,6 +1759,7 @@ __device__ __forceinline__ bool deal_next(Deal& D, uint32_t count, uint32_t* __r
 // grid 203 -> 217 us, 1,000,003 occlusion rays on the heightfield 131 -> 142 (box
 // gathered from the vertices 229 / 148, with child_boxes' divisions 223 / 145).
 constexpr uint32_t kQueryCull = 1u, kQueryFp32 = 2u;
+constexpr uint32_t kQueryAgain = 0xFFFFFFFEu;        // written for such a ray until the wave's others are done
 // EYE (closest hit, quantized nodes): ray i is the eye ray of path slot i of
 // the batch fa describes, computed in place of reading ro / rd.  A separate
 // instantiation, so that the plain kernels' code is not touched by it.
@@ -1775,7 +1776,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
   constexpr bool SH = OUT == 3;                     // counted as shadow rays; queries of either kind are not
   constexpr int S8 = kStk8<STK>;
   __shared__ TravLds<STK, Q> lds;
-  static_assert(kPriv8<S8> <= CPT_STACK_TOTAL, "API: the stack of traverse4 too, once the lane's own ray has finished");
+  static_assert(kPriv8<S8> <= CPT_STACK_TOTAL, "API: the stack of traverse4 too, once the wave's rays have finished");
   uint64_t pstk[API ? CPT_STACK_TOTAL : Q ? kPriv8<S8> : CPT_STACK_TOTAL - STK];
   const uint32_t count = API ? fa.width : *countp;
   const int lane = threadIdx.x & 63;
@@ -1796,6 +1797,7 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
   bool exhausted = false;                  // uniform
   bool active = false;
   bool pending = false;                    // finished, result not yet written
+  bool redo = false;                       // API: wrote kQueryAgain
   uint32_t ray = 0;
   std::conditional_t<Q, Ray8, RayState> R = {};   // 8-wide: lanes without a ray visit the root
   uint32_t nn = 0, nt = 0;
@@ -1815,13 +1817,11 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
         h = R.h;
         hit = h.leaf != kInvalid;
       }
+      bool again = false;
       if constexpr (API) {
-        if (hit && (fa.flags & kQueryFp32)) {
-          const float4 a = ro[2 * (size_t)ray];
-          if (!reached4(sc, h.leaf, ld3(a), R.idir, h.t, R.eps)) {
-            const float4 b4 = ro[2 * (size_t)ray + 1];
-            hit = traverse4<ANY, 0>(sc, ld3(a), ld3(b4), a.w, b4.w, fa.flags & kQueryCull, nullptr, pstk, h, nn, nt);
-          }
+        if (fa.flags & kQueryFp32) {
+          if (hit) again = !reached4(sc, h.leaf, ld3(ro[2 * (size_t)ray]), R.idir, h.t, R.eps);
+          redo = redo || again;
         }
       }
       if (OUT == 1) {
@@ -1832,10 +1832,9 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
         r.w = hit ? h.v : 0.f;
         out[ray] = r;
       } else if (OUT == 0) {
-        out[ray] = hit ? make_float4(__uint_as_float(h.orig), h.t, h.u, h.v)
-                       : make_float4(__uint_as_float(kInvalid), kInfF, 0.f, 0.f);
+        out[ray] = make_float4(__uint_as_float(again ? kQueryAgain : h.orig), h.t, h.u, h.v);
       } else if (OUT == 2) {
-        ((uint32_t*)out)[ray] = hit ? 1u : 0u;
+        ((uint32_t*)out)[ray] = again ? kQueryAgain : hit ? 1u : 0u;
       } else if (!hit) {
         const float4 c = contrib[ray];
         const uint32_t bits = __float_as_uint(c.w), slot = bits & ~kShadowNoCount;
@@ -1896,6 +1895,23 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
     } else if (active && ray_step<ANY, STK>(sc, R, false, lds_column(lds.stk), pstk, nn, nt, spill)) {
       active = false;
       pending = true;
+    }
+  }
+  if constexpr (API) {
+    if (__ballot(redo)) {                    // behind the loop, whose registers traverse4 would take
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+      const uint32_t* flag = (const uint32_t*)out;
+      for (uint64_t b = (uint64_t)(blockIdx.x * (kBlock / 64) + wid) * 64u; b < count; b += (uint64_t)waves * 64u) {
+        const uint64_t i = b + lane;
+        if (i >= count || flag[ANY ? i : 4 * i] != kQueryAgain) continue;
+        const float4 a = ro[2 * i], b4 = ro[2 * i + 1];
+        TraceHit h;
+        const bool hit =
+            traverse4<ANY, 0>(sc, ld3(a), ld3(b4), a.w, b4.w, fa.flags & kQueryCull, nullptr, pstk, h, nn, nt);
+        if (ANY) ((uint32_t*)out)[i] = hit ? 1u : 0u;
+        else out[i] = hit ? make_float4(__uint_as_float(h.orig), h.t, h.u, h.v)
+                          : make_float4(__uint_as_float(kInvalid), kInfF, 0.f, 0.f);
+      }
     }
   }
   if (stats) {
