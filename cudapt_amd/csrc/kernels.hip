@@ -1755,7 +1755,9 @@ __device__ __forceinline__ bool deal_next(Deal& D, uint32_t count, uint32_t* __r
 // the sphere grid, a few in 10^5 of those aimed at its edges, one in 10^3 on the
 // Cornell box).  What the 4-wide nodes find the 8-wide ones find too, so a miss
 // stands, and a hit stands if they are sure to test its triangle (reached4); the
-// other rays are traced again by traverse4.  2,097,143 closest hits on the sphere
+// other rays are traced again by traverse4.  So are rays with no hit within
+// 1e20 but a longer reach: IntersectTri's 1e20 for a missed triangle is then a hit
+// of the first one tested.  2,097,143 closest hits on the sphere
 // grid 203 -> 217 us, 1,000,003 occlusion rays on the heightfield 131 -> 142 (box
 // gathered from the vertices 229 / 148, with child_boxes' divisions 223 / 145).
 constexpr uint32_t kQueryCull = 1u, kQueryFp32 = 2u;
@@ -1820,7 +1822,8 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
       bool again = false;
       if constexpr (API) {
         if (fa.flags & kQueryFp32) {
-          if (hit) again = !reached4(sc, h.leaf, ld3(ro[2 * (size_t)ray]), R.idir, h.t, R.eps);
+          again = R.ht > kInfF && !(ANY && hit);
+          if (hit && !again) again = !reached4(sc, h.leaf, ld3(ro[2 * (size_t)ray]), R.idir, h.t, R.eps);
           redo = redo || again;
         }
       }
