@@ -526,6 +526,13 @@ bool collapse_bvh8(BvhHost& b, u32 leaf_max) {
   b.depth8 = 0;
   b.qmag = 1e-30f;
   if (N == 0) return true;
+  for (float lo : bn[0].mn)
+    if (lo == -INFINITY) return false;
+  const auto none = [&] {                                  // traversed in the FP32 layout instead
+    b.nodes8.clear();
+    b.order8.clear();
+    return true;
+  };
   constexpr uint8_t kWhole = 255;
   std::vector<u32> cnt(N, 0), first(N, 0);
   std::vector<std::array<double, kW8 + 1>> F(N);
@@ -607,7 +614,7 @@ bool collapse_bvh8(BvhHost& b, u32 leaf_max) {
     }
     Node8 nd;
     std::memset(&nd, 0, sizeof nd);
-    if (!quantize_slots(nd, box, b.qmag)) return false;
+    if (!quantize_slots(nd, box, b.qmag)) return none();   // an extent past 2^127
     nd.child = (u32)b.nodes8.size();
     nd.tri = (u32)b.order8.size();
     for (int s = 0; s < kW8; s++) {
@@ -625,13 +632,9 @@ bool collapse_bvh8(BvhHost& b, u32 leaf_max) {
       }
     }
     b.nodes8[it.slot] = nd;
-    if (b.nodes8.size() > kMaxNodes8) {                    // traversed in the FP32 layout instead
-      b.nodes8.clear();
-      b.order8.clear();
-      return true;
-    }
+    if (b.nodes8.size() > kMaxNodes8) return none();
   }
-  return b.depth8 <= kMaxDepth8;
+  return b.depth8 <= kMaxDepth8 || none();
 }
 
 }  // namespace cpt

@@ -361,7 +361,7 @@ int cpt_bvh_build_sah(cpt_scene* s, uint32_t max_depth) {
     return fail(CPT_E_STATE, "cpt_bvh_build_sah: build failed");
   collapse_bvh4(s->pos.data(), s->idx.data(), s->bvh, s->leaf_max);
   if (!collapse_bvh8(s->bvh, s->leaf_max))
-    return fail(CPT_E_STATE, "cpt_bvh_build_sah: a node cannot be quantized, or the 8-wide tree is deeper than %u", kMaxDepth8);
+    return fail(CPT_E_STATE, "cpt_bvh_build_sah: a vertex at minus infinity");
   if (s->bvh.depth4 > 31) return fail(CPT_E_LIMIT, "cpt_bvh_build_sah: 4-wide depth %u exceeds 31", s->bvh.depth4);
   s->has_bvh = true;
   s->uploaded = false;
@@ -390,7 +390,7 @@ int cpt_bvh4_set_leaf_size(cpt_scene* s, uint32_t max_tris) {
   if (!s->has_bvh) return CPT_OK;
   collapse_bvh4(s->pos.data(), s->idx.data(), s->bvh, s->leaf_max);
   if (!collapse_bvh8(s->bvh, s->leaf_max))
-    return fail(CPT_E_STATE, "cpt_bvh4_set_leaf_size: a node cannot be quantized, or the 8-wide tree is deeper than %u", kMaxDepth8);
+    return fail(CPT_E_STATE, "cpt_bvh4_set_leaf_size: a vertex at minus infinity");
   if (s->bvh.depth4 > 31) return fail(CPT_E_LIMIT, "cpt_bvh4_set_leaf_size: 4-wide depth %u exceeds 31", s->bvh.depth4);
   s->uploaded = false;
   s->mesh_version++;
@@ -990,7 +990,7 @@ LightJobs light_jobs(cpt_renderer* r, u32 f0, u32 nf) {
   return j;
 }
 
-// "Node Format" 1: the 8-wide quantized nodes (a scene too large for them has none).
+// "Node Format" 1: the 8-wide quantized nodes (not every scene has them: collapse_bvh8).
 bool use_nodes8(const cpt_renderer* r, const DevScene& sc) { return r->attr(kNodeFormat) != 0 && sc.nodes8; }
 
 hipError_t timed_begin(cpt_renderer* r, int kind, hipEvent_t* a, hipStream_t st = nullptr) {

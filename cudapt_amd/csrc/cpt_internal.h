@@ -79,8 +79,9 @@ bool build_bvh_device(const float* pos3, const u32* idx3, u32 nt, BvhHost& out);
 void collapse_bvh4(const float* pos3, const u32* idx3, BvhHost& b, u32 leaf_max);
 // Collapse the device binary tree into 8-wide quantized nodes (SAH-optimal);
 // a leaf child holds at most min(leaf_max, kLeaf8) triangles.  No nodes when
-// they would exceed kMaxNodes8; false when a node cannot be encoded or the tree
-// is deeper than kMaxDepth8.
+// they would exceed kMaxNodes8, an extent cannot be encoded or the tree is deeper than
+// kMaxDepth8 (the FP32 layout serves such a scene); false when a vertex lies at
+// minus infinity.
 bool collapse_bvh8(BvhHost& b, u32 leaf_max);
 
 }  // namespace cpt

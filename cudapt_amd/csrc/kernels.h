@@ -19,7 +19,7 @@ struct DevMaterial {
 // Device-resident scene.  Triangles are in BVH leaf order.
 struct DevScene {
   const Node4* nodes4;         // 128-byte 4-wide nodes
-  const Node8* nodes8;         // 8-wide quantized nodes; null: the scene is too large for them
+  const Node8* nodes8;         // 8-wide quantized nodes; null: the scene has none (collapse_bvh8)
   const float4* tris8;         // their triangles, 3 per triangle as tris, e0.w = device leaf index bits
   const float4* tri_box;       // 2 per triangle: its vertices' bounds, in the order of tris
   const float4* tris;          // 3 per triangle: p0 (w = original id bits), e0 = p1-p0, e1 = p2-p0

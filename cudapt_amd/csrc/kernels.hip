@@ -897,7 +897,7 @@ hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, cons
   dim3 grid((n + kBlock - 1) / kBlock), block(kBlock);
   const float4* ro = rays;
   const float4* rd = rays + 1;
-  if (layout == 2 && !sc.nodes8) layout = 0;       // a scene too large for 8-wide nodes
+  if (layout == 2 && !sc.nodes8) layout = 0;       // not every scene has 8-wide nodes (collapse_bvh8)
   if (layout > 2 || (layout == 2 && !sc.tris8) || (layout == 0 && !sc.nodes4)) return hipErrorInvalidValue;
 #define CPT_TR(L, A, O) k_trace<L, A, O><<<grid, block, 0, st>>>(sc, ro, rd, 2, count, n, cull, hits_out, stats)
   if (cost) {
