@@ -2167,7 +2167,7 @@ void batch_apply_config(cpt_batch* b) {
   r->set_attr(kRefill, b->cfg.refill);
   r->set_attr(kRefillSecondary, b->cfg.refill);
   r->set_attr(kRefillGroups, b->cfg.extend_workgroups);
-  r->set_attr(kRefillMinPaths, 0);               // the batch's schedule applies at every size
+  r->set_attr(kRefillMinPaths, 0);               // the batch's schedule applies at every size (and no whole_paths)
   r->persist_chunk = b->cfg.refill ? 0u : b->cfg.extend_chunk;
   r->persist_grid = r->persist_chunk ? b->cfg.extend_workgroups * (u32)(b->cus > 0 ? b->cus : 256) : 0u;
   b->drop_graph();
@@ -2198,22 +2198,17 @@ int batch_enqueue(cpt_batch* b, cpt_scene* s, u32 k) {
   jobs.dev_groups = (k + 2) / 3 + 1;                 // groups k frames can span
   const u32 n = b->total * k;
   HIP_TRY(launch_light_pass(sc, fa, jobs, r->lv.p, r->fc.p, use_nodes8(r, sc), r->stream));
-  const bool whole = !r->persist_chunk && whole_paths(r, n, 2.0);
-  if (!whole) HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
+  HIP_TRY(launch_frame_begin(r->fc.p, n, r->stream));
   Accum ac;
   std::memset(&ac, 0, sizeof ac);
   ac.result = r->result.p;
   ac.sample_n = r->sample_n.p;
   ac.rec.acc = r->rec_acc.p;
-  ac.apply = whole && k == 1 ? 0 : 2;
-  if (whole) {
-    HIP_TRY(trace_whole(r, sc, fa, ac));
-  } else {
-    int rc = bounce_loop(r, sc, fa, n, ac, true);
-    if (rc) return rc;
-  }
-  if (ac.apply == 2) HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, 0, r->stream));
-  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, k, fa.eye_depth, r->parts, whole ? n : 0u, r->stream));
+  ac.apply = 2;
+  int rc = bounce_loop(r, sc, fa, n, ac, true);
+  if (rc) return rc;
+  HIP_TRY(launch_apply_frames(fa, r->rec_acc.p, r->result.p, r->sample_n.p, 0, r->stream));
+  HIP_TRY(launch_frame_end(r->fc.p, r->stats.p, k, fa.eye_depth, r->parts, 0, r->stream));
   HIP_TRY(launch_frame_advance(b->frame_dev.p, k, r->stream));
   return CPT_OK;
 }
