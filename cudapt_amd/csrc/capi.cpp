@@ -515,8 +515,7 @@ int cpt_trace_closest_device(cpt_scene* s, const cpt_ray* d_rays, uint32_t n, ui
   if (layout > 2) return fail(CPT_E_ARG, "cpt_trace_closest_device: layout %u not 0, 1 or 2", layout);
   hipStream_t st = stream ? (hipStream_t)stream : s->stream;
   if (layout == 1)
-    HIP_TRY(launch_trace(s->dev(), (const float4*)d_rays, n, nullptr, cull, (float4*)d_hits, 1, 0, layout,
-                         s->d_stats.p, st));
+    HIP_TRY(launch_trace(s->dev(), (const float4*)d_rays, n, cull, (float4*)d_hits, 0, layout, 0, s->d_stats.p, st));
   else
     HIP_TRY(launch_trace_rays(s->dev(), (const float4*)d_rays, n, cull, (float4*)d_hits, 0, layout == 0, s->d_stats.p,
                               s->cus, st));
@@ -566,8 +565,7 @@ int cpt_trace_cost(cpt_scene* s, const cpt_ray* rays, uint32_t n, uint32_t cull,
   HIP_TRY(s->d_rays.alloc((size_t)n * 2));
   HIP_TRY(s->d_hits.alloc(n));                  // 16 bytes per ray; the costs take 8
   HIP_TRY(hipMemcpyAsync(s->d_rays.p, rays, sizeof(cpt_ray) * n, hipMemcpyHostToDevice, s->stream));
-  HIP_TRY(launch_trace(s->dev(), s->d_rays.p, n, nullptr, cull, s->d_hits.p, 0, 0, layout, s->d_stats.p, s->stream,
-                       1));
+  HIP_TRY(launch_trace(s->dev(), s->d_rays.p, n, cull, s->d_hits.p, 0, layout, 1, s->d_stats.p, s->stream));
   HIP_TRY(hipMemcpyAsync(cost2, s->d_hits.p, sizeof(uint32_t) * 2 * n, hipMemcpyDeviceToHost, s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   return CPT_OK;

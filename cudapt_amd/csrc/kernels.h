@@ -157,8 +157,11 @@ constexpr int kMaxFilterRadius = 31;   // GAUSSIANCOST_N = 64 entries (include/c
 constexpr int kBlock = 256;
 
 // ---- launches -------------------------------------------------------------
-hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, const uint32_t* count, uint32_t cull,
-                        float4* hits_out, int out_orig, int any_hit, uint32_t layout, DevStats* stats, hipStream_t st, int cost = 0);
+// One thread a ray: closest hits over the FP32 4-wide (layout 0) or binary (1) nodes,
+// occlusion flags over the 4-wide ones; cost: node visits and triangle tests per ray
+// (2: over the 8-wide nodes).
+hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, uint32_t cull, float4* out, int any_hit,
+                        uint32_t layout, int cost, DevStats* stats, hipStream_t st);
 // The trace entry points' rays (cpt_ray records, hits by original triangle id or
 // occlusion flags) over the 8-wide nodes.  fp32: with the answers of the FP32 4-wide ones.
 hipError_t launch_trace_rays(const DevScene& sc, const float4* rays, uint32_t n, uint32_t cull, float4* out, int any,

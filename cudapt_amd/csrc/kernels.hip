@@ -890,24 +890,21 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace(DevScene sc, const float
   }
 }
 
-hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, const uint32_t* count, uint32_t cull,
-                        float4* hits_out, int out_orig, int any_hit, uint32_t layout, DevStats* stats,
-                        hipStream_t st, int cost) {
+hipError_t launch_trace(const DevScene& sc, const float4* rays, uint32_t n, uint32_t cull, float4* out, int any_hit,
+                        uint32_t layout, int cost, DevStats* stats, hipStream_t st) {
   if (n == 0) return hipSuccess;
   dim3 grid((n + kBlock - 1) / kBlock), block(kBlock);
-  const float4* ro = rays;
-  const float4* rd = rays + 1;
   if (layout == 2 && !sc.nodes8) layout = 0;       // not every scene has 8-wide nodes (collapse_bvh8)
   if (layout > 2 || (layout == 2 && !sc.tris8) || (layout == 0 && !sc.nodes4)) return hipErrorInvalidValue;
-#define CPT_TR(L, A, O) k_trace<L, A, O><<<grid, block, 0, st>>>(sc, ro, rd, 2, count, n, cull, hits_out, stats)
+  // hits and flags over the 8-wide nodes are launch_trace_rays', flags over binary ones nobody's
+  if (!cost && (any_hit ? layout != 0 : layout == 2)) return hipErrorInvalidValue;
+#define CPT_TR(L, A, O) k_trace<L, A, O><<<grid, block, 0, st>>>(sc, rays, rays + 1, 2, nullptr, n, cull, out, stats)
   if (cost) {
     if (layout == 0) CPT_TR(0, false, 3); else if (layout == 2) CPT_TR(2, false, 3); else CPT_TR(1, false, 3);
   } else if (any_hit) {
-    if (layout == 0) CPT_TR(0, true, 2); else if (layout == 2) CPT_TR(2, true, 2); else CPT_TR(1, true, 2);
-  } else if (out_orig) {
-    if (layout == 0) CPT_TR(0, false, 0); else if (layout == 2) CPT_TR(2, false, 0); else CPT_TR(1, false, 0);
+    CPT_TR(0, true, 2);
   } else {
-    if (layout == 0) CPT_TR(0, false, 1); else if (layout == 2) CPT_TR(2, false, 1); else CPT_TR(1, false, 1);
+    if (layout == 0) CPT_TR(0, false, 0); else CPT_TR(1, false, 0);
   }
 #undef CPT_TR
   return hipGetLastError();
@@ -1994,7 +1991,7 @@ constexpr uint32_t kTraceGroups = 6, kTraceRefill = 16;
 hipError_t launch_trace_rays(const DevScene& sc, const float4* rays, uint32_t n, uint32_t cull, float4* out, int any,
                              int fp32, DevStats* stats, uint32_t cus, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  if (!sc.nodes8) return launch_trace(sc, rays, n, nullptr, cull, out, any ? 0 : 1, any, 0, stats, st);
+  if (!sc.nodes8) return launch_trace(sc, rays, n, cull, out, any, 0, 0, stats, st);
   if (!rays || !out || !sc.tris8 || cus == 0) return hipErrorInvalidValue;
   FrameArgs fa = {};
   fa.width = n;
