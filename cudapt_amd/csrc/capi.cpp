@@ -758,14 +758,19 @@ struct cpt_mlp {
 
 // Device memory to pageable host memory through a ring of pinned chunks owned
 // by a renderer: the runtime's own staging copies a chunk, waits and copies it
-// on, here the next chunks are under way meanwhile.  Images into fresh arrays, ring /
-// runtime, us: 5.8 MB 341 / 409, 24.9 MB 1281 / 1730, 106 MB 8016 / 10045 (chunks of
-// 256 KB 769 / 2060 for the first two, of 4 MB the same as of 1 MB).
+// on, here the next chunks are under way meanwhile.  Reused / fresh host arrays, ring
+// against runtime, us: 6.3 MB 291 / 298 against 357 / 435, 25 MB 964 / 996 against
+// 1452 / 1848.  Chunks of 1 MB take 5 % less but, for half a second after another
+// renderer's memory was freed, 586 us for the 6.3 MB and 754 for 8.4 MB (runtime 358
+// / 483): each wait then takes 90 us; of 4 MB 307 / 376.  Up to 16 KB one chunk takes
+// 14 us against 23 to 28; in between the runtime is the faster one (64 KB 12 against 20
+// us, 1 MB 60 against 67, 1.5 MB equal) and copies.
 // Memory that the runtime knows (pinned, managed, device) is copied to directly.
-constexpr size_t kReadChunk = 1u << 20, kReadChunks = 4;
+constexpr size_t kReadChunk = 4u << 20, kReadChunks = 3, kReadSmall = 16u << 10, kReadLarge = 3u << 19;
 struct Readback {
   std::mutex lock;                 // one ring, whoever reads
   char* ring = nullptr;
+  size_t cap = 0;                  // no more than the reads so far needed
   hipEvent_t done[kReadChunks] = {};
   ~Readback() {
     for (auto e : done)
@@ -776,20 +781,29 @@ struct Readback {
     hipPointerAttribute_t at;
     const bool known = hipPointerGetAttributes(&at, out) == hipSuccess && at.type != hipMemoryTypeUnregistered;
     (void)hipGetLastError();
-    if (known) {
+    if (known || (bytes > kReadSmall && bytes < kReadLarge)) {
       const hipError_t e = hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, st);
       return e != hipSuccess ? e : hipStreamSynchronize(st);
     }
     std::lock_guard<std::mutex> g(lock);
     hipError_t e = hipSuccess;
-    if (!ring) e = hipHostMalloc((void**)&ring, kReadChunk * kReadChunks, hipHostMallocDefault);
+    const size_t want = std::min(std::max(bytes, kReadSmall), kReadChunk * kReadChunks);
+    if (cap < want) {
+      if (ring) (void)hipHostFree(ring);
+      ring = nullptr;
+      cap = 0;
+      e = hipHostMalloc((void**)&ring, want, hipHostMallocDefault);
+      if (e == hipSuccess) cap = want;
+    }
     for (auto& d : done)
       if (e == hipSuccess && !d) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
-    const size_t n = (bytes + kReadChunk - 1) / kReadChunk;
-    const auto len = [&](size_t k) { return std::min(kReadChunk, bytes - k * kReadChunk); };
+    // a read that fits the ring is cut in as many chunks as it has
+    const size_t third = (bytes / kReadChunks + (1u << 16)) & ~(size_t)0xFFFF;
+    const size_t chunk = std::min(std::max(third, kReadChunk / 4), kReadChunk), n = (bytes + chunk - 1) / chunk;
+    const auto len = [&](size_t k) { return std::min(chunk, bytes - k * chunk); };
     const auto start = [&](size_t k) {
       const size_t slot = k % kReadChunks;
-      e = hipMemcpyAsync(ring + slot * kReadChunk, (const char*)src + k * kReadChunk, len(k), hipMemcpyDeviceToHost, st);
+      e = hipMemcpyAsync(ring + slot * chunk, (const char*)src + k * chunk, len(k), hipMemcpyDeviceToHost, st);
       if (e == hipSuccess) e = hipEventRecord(done[slot], st);
     };
     for (size_t k = 0; k < std::min(n, kReadChunks) && e == hipSuccess; k++) start(k);
@@ -797,7 +811,7 @@ struct Readback {
       const size_t slot = k % kReadChunks;
       e = hipEventSynchronize(done[slot]);
       if (e != hipSuccess) break;
-      std::memcpy((char*)out + k * kReadChunk, ring + slot * kReadChunk, len(k));
+      std::memcpy((char*)out + k * chunk, ring + slot * chunk, len(k));
       if (k + kReadChunks < n) start(k + kReadChunks);
     }
     const hipError_t es = hipStreamSynchronize(st);      // also after an error: nothing writes the ring any more
