@@ -433,26 +433,6 @@ int cpt_scene_upload(cpt_scene* s) {
     return out;
   };
   std::vector<float4> tris = tri_data(s->bvh.dreorder), tris_bin = tri_data(s->bvh.reorder);
-  // the 8-wide tree's triangles: the same records in its own order, each with
-  // its index in the device leaf order
-  std::vector<float4> tris8(s->bvh.order8.size() * 3);
-  for (u32 i = 0; i < (u32)s->bvh.order8.size(); i++) {
-    const u32 leaf = s->bvh.order8[i];
-    for (int k = 0; k < 3; k++) tris8[(size_t)i * 3 + k] = tris[(size_t)leaf * 3 + k];
-    std::memcpy(&tris8[(size_t)i * 3 + 1].w, &leaf, 4);
-  }
-  std::vector<float4> tri_box((size_t)nt * 2);
-  for (u32 i = 0; i < nt; i++) {
-    float mn[3], mx[3];
-    for (int k = 0; k < 3; k++) {
-      const u32* v = &s->idx[(size_t)s->bvh.dreorder[i] * 3];
-      const float a = s->pos[(size_t)v[0] * 3 + k], b = s->pos[(size_t)v[1] * 3 + k], c = s->pos[(size_t)v[2] * 3 + k];
-      mn[k] = std::fmin(c, std::fmin(b, a));
-      mx[k] = std::fmax(c, std::fmax(b, a));
-    }
-    tri_box[(size_t)i * 2] = make_float4(mn[0], mn[1], mn[2], 0.f);
-    tri_box[(size_t)i * 2 + 1] = make_float4(mx[0], mx[1], mx[2], 0.f);
-  }
   std::vector<uint4> tv(nt);
   for (u32 i = 0; i < nt; i++) {
     u32 o = s->bvh.dreorder[i];
@@ -473,12 +453,18 @@ int cpt_scene_upload(cpt_scene* s) {
   }
   HIP_TRY(s->d_nodes4.upload(s->bvh.nodes4.data(), s->bvh.nodes4.size(), s->stream));
   HIP_TRY(s->d_nodes8.upload(s->bvh.nodes8.data(), s->bvh.nodes8.size(), s->stream));
-  HIP_TRY(s->d_tris8.upload(tris8.data(), tris8.size(), s->stream));
-  HIP_TRY(s->d_tri_box.upload(tri_box.data(), tri_box.size(), s->stream));
   HIP_TRY(s->d_tris.upload(tris.data(), tris.size(), s->stream));
   HIP_TRY(s->d_tris_bin.upload(tris_bin.data(), tris_bin.size(), s->stream));
   HIP_TRY(s->d_tri_verts.upload(tv.data(), tv.size(), s->stream));
   HIP_TRY(s->d_vpos.upload(vp.data(), vp.size(), s->stream));
+  // the 8-wide tree's triangles and the triangles' boxes come from what is there by now
+  DevArray<u32> order8;
+  const u32 n8 = (u32)s->bvh.order8.size();
+  HIP_TRY(order8.upload(s->bvh.order8.data(), n8, s->stream));
+  HIP_TRY(s->d_tris8.alloc((size_t)n8 * 3));
+  HIP_TRY(s->d_tri_box.alloc((size_t)nt * 2));
+  HIP_TRY(launch_tri_records(s->d_tris.p, s->d_tri_verts.p, s->d_vpos.p, nt, order8.p, n8, s->d_tris8.p, s->d_tri_box.p,
+                             s->stream));
   HIP_TRY(s->d_vnrm.upload(vn.data(), vn.size(), s->stream));
   HIP_TRY(s->d_bnodes.upload(bnodes.data(), bnodes.size(), s->stream));
   HIP_TRY(s->d_tex.upload(s->tex.data(), s->tex.size(), s->stream));

@@ -157,6 +157,10 @@ constexpr int kMaxFilterRadius = 31;   // GAUSSIANCOST_N = 64 entries (include/c
 constexpr int kBlock = 256;
 
 // ---- launches -------------------------------------------------------------
+// What queries read beside tris: tris8, the n8 triangles of the 8-wide tree's order
+// (device leaf indices), and the bounds of each triangle's vertices (DevScene).
+hipError_t launch_tri_records(const float4* tris, const uint4* tri_verts, const float4* vpos, uint32_t n,
+                              const uint32_t* order8, uint32_t n8, float4* tris8, float4* tri_box, hipStream_t st);
 // One thread a ray: closest hits over the FP32 4-wide (layout 0) or binary (1) nodes,
 // occlusion flags over the 4-wide ones; cost: node visits and triangle tests per ray
 // (2: over the 8-wide nodes).

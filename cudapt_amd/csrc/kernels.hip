@@ -834,6 +834,41 @@ static bool pathbuf_ok(const PathBuf& b) {
 static bool nodes_ok(const DevScene& sc, int quant) { return quant ? sc.nodes8 && sc.tris8 : sc.nodes4 != nullptr; }
 static bool rec_ok(const SampleRec& r) { return r.acc && r.gpos && r.gnrm && r.gdif; }
 
+// ---------------------------------------------------------------- scene records
+// Filled here: the host would gather 48 and 36 bytes a triangle and send 80 over the
+// bus (heightfield of 1,050,976 triangles: upload 129 ms so, 105 here).
+__global__ __launch_bounds__(kBlock) void k_tri_records(const float4* __restrict__ tris,
+                                                        const uint4* __restrict__ tri_verts,
+                                                        const float4* __restrict__ vpos, uint32_t n,
+                                                        const uint32_t* __restrict__ order8, uint32_t n8,
+                                                        float4* __restrict__ tris8, float4* __restrict__ tri_box) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) {
+    const uint4 v = tri_verts[i];
+    const f3 a = ld3(vpos[v.x]), b = ld3(vpos[v.y]), c = ld3(vpos[v.z]);
+    tri_box[2 * (size_t)i] =
+        make_float4(fminf(c.x, fminf(b.x, a.x)), fminf(c.y, fminf(b.y, a.y)), fminf(c.z, fminf(b.z, a.z)), 0.f);
+    tri_box[2 * (size_t)i + 1] =
+        make_float4(fmaxf(c.x, fmaxf(b.x, a.x)), fmaxf(c.y, fmaxf(b.y, a.y)), fmaxf(c.z, fmaxf(b.z, a.z)), 0.f);
+  }
+  if (i < n8) {
+    const uint32_t leaf = order8[i];
+    const float4* T = tris + 3 * (size_t)leaf;
+    float4 e0 = T[1];
+    e0.w = __uint_as_float(leaf);
+    tris8[3 * (size_t)i] = T[0];
+    tris8[3 * (size_t)i + 1] = e0;
+    tris8[3 * (size_t)i + 2] = T[2];
+  }
+}
+hipError_t launch_tri_records(const float4* tris, const uint4* tri_verts, const float4* vpos, uint32_t n,
+                              const uint32_t* order8, uint32_t n8, float4* tris8, float4* tri_box, hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  if (!tris || !tri_verts || !vpos || !tri_box || n8 > n || (n8 && (!order8 || !tris8))) return hipErrorInvalidValue;
+  k_tri_records<<<(n + kBlock - 1) / kBlock, kBlock, 0, st>>>(tris, tri_verts, vpos, n, order8, n8, tris8, tri_box);
+  return hipGetLastError();
+}
+
 // ---------------------------------------------------------------- trace API
 // out mode 0: cpt_hit {orig id, t, u, v}; 1: {t, leaf bits, u, v}; 2: occluded flag.
 // MINW: minimum resident waves per SIMD requested from the register allocator
