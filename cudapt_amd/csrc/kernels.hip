@@ -3332,7 +3332,10 @@ __device__ __forceinline__ FilterScale filter_scale(const FilterArgs& fa, bool d
 // records and the guides' distances; its pixels take the words of the record that are free.
 // Image and second moment of the learned frames (1920 x 1080, radius 7, depth): 760 us,
 // two passes 1044.
-template <bool DIFF, bool DEPTH, bool PAIR>
+// REC: words a record.  At radius 9 records of 12 words leave two workgroups on a compute unit,
+// of 10 three; without albedo and second image 10 hold a pixel (read as 64-bit words,
+// again free of conflicts).  1000 x 700, radius 9: 399 us with 12, 290 with 10.
+template <bool DIFF, bool DEPTH, bool PAIR, int REC>
 __global__ __launch_bounds__(kTile * kTile) void k_filter_lds(FilterArgs fa, const float* __restrict__ color,
                                                               const float* __restrict__ gpos,
                                                               const float* __restrict__ gnrm,
@@ -3343,13 +3346,14 @@ __global__ __launch_bounds__(kTile * kTile) void k_filter_lds(FilterArgs fa, con
                                                               float* __restrict__ filtered2,
                                                               float* __restrict__ err2) {
   static_assert(!(DIFF && PAIR), "a pair's record has no room for the albedo");
+  static_assert(REC == 12 || (REC == 10 && !DIFF && !PAIR), "words of a record");
   extern __shared__ float4 sm[];
   const int R = (int)fa.radius, D = 2 * R + 1, TW = kTile + 2 * R, TA = TW * TW;
   const uint32_t W = fa.width, H = fa.height;
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * kTile + tx;
   const int bx = blockIdx.x * kTile, by = blockIdx.y * kTile;
   float* rec = (float*)sm;                         // c, p, n, then d, or z and two words of c2, or c2
-  float* wt = rec + 12 * (size_t)TA;               // spatial weight of tap (i, j)
+  float* wt = rec + REC * (size_t)TA;              // spatial weight of tap (i, j)
   float* sz = wt + (size_t)D * D;                  // DEPTH: z (DIFF) or c2's last (PAIR) per halo pixel
   const float cam[3] = {fa.cam[0], fa.cam[1], fa.cam[2]};
   for (int k = tid; k < D * D; k += kTile * kTile) {
@@ -3359,7 +3363,7 @@ __global__ __launch_bounds__(kTile * kTile) void k_filter_lds(FilterArgs fa, con
   for (int k = tid; k < TA; k += kTile * kTile) {
     const int hy = k / TW, hx = k - hy * TW;
     const size_t g = ((size_t)ref_clamp_i(by + hy - R, H) * W + ref_clamp_i(bx + hx - R, W)) * 3;
-    float* r = rec + 12 * k;
+    float* r = rec + REC * k;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       r[c] = color[g + c];
@@ -3381,6 +3385,15 @@ __global__ __launch_bounds__(kTile * kTile) void k_filter_lds(FilterArgs fa, con
   __syncthreads();
   const auto load = [&](int k) {
     FilterTap q;
+    if constexpr (REC == 10) {
+      const float2* r = (const float2*)(rec + 10 * k);
+      const float2 a = r[0], b = r[1], c = r[2], d = r[3], e = r[4];
+      q.c[0] = a.x; q.c[1] = a.y; q.c[2] = b.x;
+      q.p[0] = b.y; q.p[1] = c.x; q.p[2] = c.y;
+      q.n[0] = d.x; q.n[1] = d.y; q.n[2] = e.x;
+      q.z = DEPTH ? e.y : 0.f;
+      return q;
+    }
     const float4* r = (const float4*)(rec + 12 * k);
     const float4 a = r[0], b = r[1], c = r[2];
     q.c[0] = a.x; q.c[1] = a.y; q.c[2] = a.z;
@@ -3475,21 +3488,25 @@ hipError_t launch_filter_error(const FilterArgs& fa, const float* color, const f
   const bool depth = fa.kz > 0.f, diff = fa.use_diff != 0, pair = color2 && !diff && R <= kLdsRadius;
   const dim3 block(kTile, kTile), grid((fa.width + kTile - 1) / kTile, (fa.height + kTile - 1) / kTile);
   const int TA = (kTile + 2 * R) * (kTile + 2 * R);
-  const size_t bytes = sizeof(float) * (12 * (size_t)TA + (size_t)D * D + ((diff || pair) && depth ? TA : 0));
-#define CPT_FILTER(DI, DE, PA)                                                                                    \
+  const bool narrow = R == kLdsRadius && !diff && !pair;
+  const size_t bytes =
+      sizeof(float) * ((narrow ? 10 : 12) * (size_t)TA + (size_t)D * D + ((diff || pair) && depth ? TA : 0));
+#define CPT_FILTER(DI, DE, PA, RE)                                                                                \
   {                                                                                                               \
     if (R > kLdsRadius)                                                                                           \
       k_filter_mem<DI, DE><<<grid, block, 0, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered, err);         \
     else                                                                                                          \
-      k_filter_lds<DI, DE, PA><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered, err,  \
-                                                           color2, filtered2, err2);                              \
+      k_filter_lds<DI, DE, PA, RE><<<grid, block, bytes, st>>>(fa, color, gpos, gnrm, gdif, sample_n, filtered,   \
+                                                               err, color2, filtered2, err2);                     \
   }
   if (diff) {
-    if (depth) CPT_FILTER(true, true, false) else CPT_FILTER(true, false, false)
+    if (depth) CPT_FILTER(true, true, false, 12) else CPT_FILTER(true, false, false, 12)
   } else if (pair) {
-    if (depth) CPT_FILTER(false, true, true) else CPT_FILTER(false, false, true)
+    if (depth) CPT_FILTER(false, true, true, 12) else CPT_FILTER(false, false, true, 12)
+  } else if (narrow) {
+    if (depth) CPT_FILTER(false, true, false, 10) else CPT_FILTER(false, false, false, 10)
   } else {
-    if (depth) CPT_FILTER(false, true, false) else CPT_FILTER(false, false, false)
+    if (depth) CPT_FILTER(false, true, false, 12) else CPT_FILTER(false, false, false, 12)
   }
 #undef CPT_FILTER
   const hipError_t e = hipGetLastError();
