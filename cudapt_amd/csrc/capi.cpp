@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -742,45 +743,65 @@ struct cpt_mlp {
   }
 };
 
-// Device memory to pageable host memory through a ring of pinned chunks owned
-// by a renderer: the runtime's own staging copies a chunk, waits and copies it
-// on, here the next chunks are under way meanwhile.  Reused / fresh host arrays, ring
-// against runtime, us: 6.3 MB 291 / 298 against 357 / 435, 25 MB 964 / 996 against
-// 1452 / 1848.  Chunks of 1 MB take 5 % less but, for half a second after another
-// renderer's memory was freed, 586 us for the 6.3 MB and 754 for 8.4 MB (runtime 358
-// / 483): each wait then takes 90 us; of 4 MB 307 / 376.  Up to 16 KB one chunk takes
-// 14 us against 23 to 28; in between the runtime is the faster one (64 KB 12 against 20
-// us, 1 MB 60 against 67, 1.5 MB equal) and copies.
+// Device memory to pageable host memory through a ring of pinned chunks: the
+// runtime's own staging copies a chunk, waits and copies it on, here the next
+// chunks are under way meanwhile.  Reused / fresh host arrays, ring against
+// runtime, us: 6.3 MB 265 / 269 against 357 / 435, 25 MB 972 / 937 against 1452 /
+// 1848.  More than three chunks at a time lose for half a second after another
+// renderer's memory was freed: each one past the third then takes 90 us (chunks of 1
+// MB 586 us for the 6.3 MB and 754 for 8.4 MB, runtime 358 / 483; three chunks 266 /
+// 354).  Up to 16 KB one chunk takes 14 us against 23 to 28; in between the runtime is
+// the faster one (64 KB 12 against 20 us, 1 MB 60 against 67, 1.5 MB equal) and copies.
 // Memory that the runtime knows (pinned, managed, device) is copied to directly.
 constexpr size_t kReadChunk = 4u << 20, kReadChunks = 3, kReadSmall = 16u << 10, kReadLarge = 3u << 19;
+// The pinned memory, one for all renderers of the process (pinning 12 MB takes 5 ms, as
+// much as 50 reads of 6 MB gain) and given back with the last of them; a read that
+// finds it in use, or finds none to be had, is the runtime's.
+struct ReadRing {
+  std::mutex lock;
+  char *small = nullptr, *ring = nullptr;
+  ~ReadRing() {
+    if (small) (void)hipHostFree(small);
+    if (ring) (void)hipHostFree(ring);
+  }
+  char* get(size_t bytes) {        // with the lock held
+    char*& p = bytes <= kReadSmall ? small : ring;
+    if (!p && hipHostMalloc((void**)&p, bytes <= kReadSmall ? kReadSmall : kReadChunk * kReadChunks,
+                            hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+    }
+    return p;
+  }
+  static std::shared_ptr<ReadRing> shared() {
+    static std::mutex m;
+    static std::weak_ptr<ReadRing> w;
+    std::lock_guard<std::mutex> g(m);
+    std::shared_ptr<ReadRing> p = w.lock();
+    if (!p) w = p = std::make_shared<ReadRing>();
+    return p;
+  }
+};
 struct Readback {
-  std::mutex lock;                 // one ring, whoever reads
-  char* ring = nullptr;
-  size_t cap = 0;                  // no more than the reads so far needed
-  hipEvent_t done[kReadChunks] = {};
+  std::shared_ptr<ReadRing> pool = ReadRing::shared();
+  hipEvent_t done[kReadChunks] = {};       // used with the pool's lock held
   ~Readback() {
     for (auto e : done)
       if (e) (void)hipEventDestroy(e);
-    if (ring) (void)hipHostFree(ring);
   }
   hipError_t read(void* out, const void* src, size_t bytes, hipStream_t st) {
     hipPointerAttribute_t at;
     const bool known = hipPointerGetAttributes(&at, out) == hipSuccess && at.type != hipMemoryTypeUnregistered;
     (void)hipGetLastError();
-    if (known || (bytes > kReadSmall && bytes < kReadLarge)) {
+    std::unique_lock<std::mutex> g(pool->lock, std::defer_lock);
+    char* ring = nullptr;
+    if (!known && (bytes <= kReadSmall || bytes >= kReadLarge) && g.try_lock()) ring = pool->get(bytes);
+    if (!ring) {
+      if (g.owns_lock()) g.unlock();
       const hipError_t e = hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, st);
       return e != hipSuccess ? e : hipStreamSynchronize(st);
     }
-    std::lock_guard<std::mutex> g(lock);
     hipError_t e = hipSuccess;
-    const size_t want = std::min(std::max(bytes, kReadSmall), kReadChunk * kReadChunks);
-    if (cap < want) {
-      if (ring) (void)hipHostFree(ring);
-      ring = nullptr;
-      cap = 0;
-      e = hipHostMalloc((void**)&ring, want, hipHostMallocDefault);
-      if (e == hipSuccess) cap = want;
-    }
     for (auto& d : done)
       if (e == hipSuccess && !d) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
     // a read that fits the ring is cut in as many chunks as it has
