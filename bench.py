@@ -8,8 +8,8 @@ before timing; the timed region is K renders of 64 frames each.
 
 metric/value: Mrays/s = (extension + shadow rays traced) / wall time.
 roofline: the closest-hit extension kernel (by default k_trace_dyn: persistent
-  waves that take new rays from a global queue once 64 (first bounce) or 48
-  (later bounces) of their lanes are idle), algorithmic bytes per launch =
+  waves that take new rays, dealt in eight shares of shrinking chunks, one a
+  die, once 64 (first bounce) or 48 (later bounces) of their lanes are idle), algorithmic bytes per launch =
   32 B per ray read from memory (first-bounce eye rays are computed in the
   kernel and read nothing) + 16 B hit out per ray + 128 B per node visited
   (8-wide, or 4-wide in the FP32 layout) + 48 B per triangle tested,
@@ -570,7 +570,7 @@ def main():
     node_bytes = 128                                  # both layouts
     # first-bounce eye rays are computed inside the extension kernel (no 32 B
     # ray read) when the refilling grid runs the first bounce over the
-    # quantized nodes, as the renderer's schedule does above Refill Min Paths
+    # 8-wide nodes, as the renderer's schedule does above Refill Min Paths
     eye_in_kernel = args.refill >= 1 and args.node_format != 0 and WIDTH * HEIGHT * args.in_flight >= (1 << 20)
     ext_rays = st["extension_rays"] - st["tail_rays"]     # the tail kernel's rays are not the extension kernel's
     rays_read = ext_rays - (st["eye_paths"] if eye_in_kernel else 0)

@@ -1042,12 +1042,18 @@ void camera_basis(const float* d, const float* up, float* right, float* up2) {
 // A launch too small to fill the chip bounce by bounce: each thread carries its
 // path through every bounce (k_mega, k_tail).  Phase times exist only where the
 // phases are launches of their own, so a profiled renderer keeps them.  The line
-// lies where both take the same time: at twice "Refill Min Paths" (2 M paths by
-// default) for plain frames - whole / by bounce, us: 800 x 600 on the sphere grid
-// 936 / 1228, 1280 x 720 1590 / 1831, 1920 x 1080 3229 / 3318, 8 frames of 800 x 600
-// 3377 / 3023 - and at once that for adaptive ones, whose paths crowd on the noisy
-// pixels: 10 bisected frames of 1280 x 720 there 15.0 / 16.2 ms, of 1920 x 1080
-// 28.6 / 26.7.
+// lies at twice "Refill Min Paths" (2 M paths by default) for plain frames and at once
+// that for adaptive ones, whose paths crowd on the noisy pixels.  Below it whole paths
+// are the faster form on every scene and depth measured, above it on those whose paths
+// end early.  Whole / by bounce at depth 5, then 15; plain frames without read-back, us:
+//   paths      sphere grid             heightfield             Cornell box
+//   0.48 M      545 /  753, 691 / 1476   400 /  613, 419 /  885   212 /  319, 228 /  640
+//   0.92 M      796 /  906, 1001 / 1695  570 /  760, 587 / 1073   317 /  390, 334 /  710
+//   2.07 M     1457 / 1551, 1791 / 2395 1073 / 1217, 1096 / 1572  554 /  827, 586 / 1170
+//   3.84 M     2506 / 2176, 3066 / 3087 1761 / 1812, 1790 / 2226 1147 / 1538, 1190 / 1819
+// 12 bisected adaptive frames, ms:
+//   0.92 M     14.8 / 15.9, 17.6 / 18.4 11.0 / 12.4, 11.3 / 13.0  7.7 / 10.4, 8.0 / 10.8
+//   2.07 M     28.9 / 26.2, 34.4 / 30.3 20.9 / 20.4, 21.3 / 21.0 14.5 / 18.1, 14.9 / 18.7
 bool whole_paths(const cpt_renderer* r, u32 n, double scale = 1.0) {
   return !r->profiling && (double)n < scale * r->attr(kRefillMinPaths);
 }

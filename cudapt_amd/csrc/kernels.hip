@@ -480,7 +480,7 @@ __device__ __forceinline__ bool ray8_hit(const Wave8<STK>& W, int lane, TraceHit
 // under half the slack, which is subtracted from entries (R.pn) and added to exits
 // (R.pf), so no box that the ray meets in exact arithmetic is culled.
 // Only the loads are masked by `active`: the vector caches serve one line a
-// cycle (80 % of their cycles busy in the secondary rays of the sphere grid), so the
+// cycle (unmasked, 80 % of their cycles busy in the sphere grid's secondary rays), so the
 // lines of idle lanes cost as much as the others', while idle lanes in the arithmetic
 // cost nothing.  Masked / not: still of 64 1280 x 720 frames 18.4 / 19.2 ms, 8 views of
 // the heightfield 11.2 / 12.3 ms, 1,000,003 occlusion rays there 146 / 163 us.
