@@ -1787,13 +1787,13 @@ __device__ __forceinline__ bool deal_next(Deal& D, uint32_t count, uint32_t* __r
 // the sphere grid, a few in 10^5 of those aimed at its edges, one in 10^3 on the
 // Cornell box).  What the 4-wide nodes find the 8-wide ones find too, so a miss
 // stands, and a hit stands if they are sure to test its triangle (reached4); the
-// other rays are traced again by traverse4.  So are rays with no hit within
-// 1e20 but a longer reach: IntersectTri's 1e20 for a missed triangle is then a hit
+// other rays are traced again by traverse4.  So are, with either layout's answers, rays
+// with no hit within 1e20 but a longer reach: IntersectTri's 1e20 for a missed triangle is then a hit
 // of the first one tested.  And rays whose boxes say little of their triangles: of
 // negative eps (culled by distances behind the best hit's), or short (under 1e-2)
 // with a component that escape_zero moves (by 1e-9, far off at their distances): their
 // answer is that of the tree's order and leaves.  2,097,143 closest hits on the sphere
-// grid 203 -> 217 us, 1,000,003 occlusion rays on the heightfield 131 -> 142 (box
+// grid 203 -> 219 us, 1,000,003 occlusion rays on the heightfield 131 -> 142 (box
 // gathered from the vertices 229 / 148, with child_boxes' divisions 223 / 145).
 constexpr uint32_t kQueryCull = 1u, kQueryFp32 = 2u;
 constexpr uint32_t kQueryAgain = 0xFFFFFFFEu;        // written for such a ray until the wave's others are done
@@ -1856,13 +1856,14 @@ __global__ __launch_bounds__(kBlock, MINW) void k_trace_dyn(DevScene sc, const f
       }
       bool again = false;
       if constexpr (API) {
+        again = R.ht > kInfF && !(ANY && hit);
         if (fa.flags & kQueryFp32) {
           const float lo = fminf(fabsf(R.idir.x), fminf(fabsf(R.idir.y), fabsf(R.idir.z)));
           const float hi = fmaxf(fabsf(R.idir.x), fmaxf(fabsf(R.idir.y), fabsf(R.idir.z)));
-          again = (R.ht > kInfF && !(ANY && hit)) || R.eps < 0.f || (lo > 100.f && hi > 4e8f);
+          again = again || R.eps < 0.f || (lo > 100.f && hi > 4e8f);
           if (hit && !again) again = !reached4(sc, h.leaf, ld3(ro[2 * (size_t)ray]), R.idir, h.t, R.eps);
-          redo = redo || again;
         }
+        redo = redo || again;
       }
       if (OUT == 1) {
         float4 r;
